@@ -598,102 +598,131 @@ __global__ void __launch_bounds__(256) k_misfit(const T *d, const float *obs, fl
   if (threadIdx.x == 0) atomicAdd(J, part[0]);
 }
 
-// ---- chain rule (the device form of the host chain in biot_params.cpp) ----
+// ---- chain rule (the gather form of the host chain in biot_params.cpp) ----
 __device__ __forceinline__ double harmonic4(double a, double b, double c, double d)
 {
   if (a == 0 || b == 0 || c == 0 || d == 0) return 0.0;
   return 1.0 / (0.25 * (1 / a + 1 / b + 1 / c + 1 / d));
 }
 
-__global__ void __launch_bounds__(256) k_chain(const ChainArgs c)
+// One thread per window cell p sums what every coefficient that reads p's parameters passes
+// back to it (the cells p and, one step down each axis the coefficient averages over, the cells
+// below), so a cell's six gradients are written once, in a fixed order.  It runs once a gradient
+// and is bound by its FP64 divisions: 0.33 ms at 128^3, where the single grid's chain took about
+// 170 ms on one host thread, after a copy of all 22 FP64 gradient arrays (a 128^3, 100-step
+// gradient: 253 -> 76 ms).  The scatter form (each coefficient adding to the cells it reads, ~30
+// FP64 atomics a cell) summed in an order that changed from run to run.
+struct VelGrad {
+  double gA, gB, gc2;
+};
+// dJ/d(rho, rho_f, rho_f tphi averages) of axis m's velocity coefficients at cell c
+__device__ __forceinline__ VelGrad vel_grad(const ChainArgs &a, int64_t c, int m, const int64_t (&step)[3])
 {
-  const int64_t wsy = c.wx, wsz = (int64_t)c.wx * c.wy;
-  const int64_t nw = wsz * c.wz;
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= nw) return;
-  const int i = (int)(t % c.wx);
-  const int j = (int)((t / c.wx) % c.wy);
-  const int k = (int)(t / wsz);
-  if (i < 1 || i >= c.wx - 1 || j < 1 || j >= c.wy - 1 || k < 1 || k >= c.wz - 1) return;
-  // p: window cell (parameters, coefficient gradients); g: model cell (output)
-  const int64_t p = t;
-  const int64_t g = (int64_t)(c.x0 + i) + (int64_t)(c.y0 + j) * c.msy + (int64_t)(c.z0 + k) * c.msz;
-  auto gK = [&](int kk) { return c.grad[kk][t] * c.kfac[kk]; };
-  const double *mu = c.par[1], *alp = c.par[2], *M = c.par[3];
-  const double *rho = c.par[4], *rhof = c.par[5], *C1 = c.par[6], *tphi = c.par[7];
-  const double k1 = c.Cv * c.dt / c.Cp;   // velocity coefficient scale
-  const double kk = c.dt * c.Cp / c.Cv;   // stress coefficient scale
-  // stress side: K_P1 = C kk/dx, K_P2 = M kk/dx, K_S1 = lambda_c .., K_S2 = H .., K_S3 = C ..
-  const double al = alp[p], Mp = M[p];
-  const double gC = (gK(K_P1) + gK(K_S3)) * kk * c.Hinv;
-  const double glc = gK(K_S1) * kk * c.Hinv;
-  const double gH = gK(K_S2) * kk * c.Hinv;
-  const double gMd = gK(K_P2) * kk * c.Hinv;
-  atomicAdd(&c.out[0][g], glc + gH);
-  double gmu_c = 2 * gH;
-  atomicAdd(&c.out[2][g], gC * Mp + (glc + gH) * 2 * al * Mp);
-  atomicAdd(&c.out[3][g], gMd + gC * al + (glc + gH) * al * al);
-  // shear: 4-cell harmonic means, d mu_bar / d mu_i = mu_bar^2 / (4 mu_i^2)
-  const int64_t wq[3][4] = {{0, 1, wsy, wsy + 1}, {0, 1, wsz, wsz + 1}, {0, wsy, wsz, wsz + wsy}};
-  const int64_t mq[3][4] = {{0, 1, c.msy, c.msy + 1}, {0, 1, c.msz, c.msz + 1},
-                            {0, c.msy, c.msz, c.msz + c.msy}};
-  const int kidx[3] = {K_SXY, K_SXZ, K_SYZ};
-  for (int m = 0; m < 3; ++m) {
-    const double m0 = mu[p + wq[m][0]], m1 = mu[p + wq[m][1]], m2 = mu[p + wq[m][2]], m3 = mu[p + wq[m][3]];
-    const double hm = harmonic4(m0, m1, m2, m3);
-    if (hm == 0) continue;
-    const double gg = gK(kidx[m]) * kk * c.Hinv;
-    for (int e = 0; e < 4; ++e) {
-      const double me = mu[p + wq[m][e]];
-      const double v = gg * hm * hm / (4 * me * me);
-      if (e == 0) gmu_c += v;
-      else atomicAdd(&c.out[1][g + mq[m][e]], v);
-    }
-  }
-  atomicAdd(&c.out[1][g], gmu_c);
-  // velocity side, per staggering direction
-  const int64_t wstep[3] = {1, wsy, wsz}, mstep[3] = {1, c.msy, c.msz};
-  double A[3], B[3], c1[3], D[3];
+  const double *rho = a.par[4], *rhof = a.par[5], *C1 = a.par[6], *tphi = a.par[7];
   bool c1zero = false, azero = false;
-  for (int m = 0; m < 3; ++m) {
-    const int64_t p2 = p + wstep[m];
-    A[m] = 0.5 * (rho[p] + rho[p2]);
-    B[m] = 0.5 * (rhof[p] + rhof[p2]);
-    c1[m] = 0.5 * (C1[p] + C1[p2]);
-    const double c2 = 0.5 * (tphi[p] * rhof[p] + tphi[p2] * rhof[p2]);
-    D[m] = (c2 - B[m] * B[m] / A[m]) + 0.5 * c.dt * c1[m];
-    c1zero |= c1[m] == 0;
-    azero |= A[m] == 0;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    c1zero |= 0.5 * (C1[c] + C1[c + step[d]]) == 0;
+    azero |= 0.5 * (rho[c] + rho[c + step[d]]) == 0;
   }
-  double grho_c = 0, grf_c = 0;
-  for (int m = 0; m < 3; ++m) {
-    double gA = 0, gB = 0, gc2 = 0;
-    if (!c1zero) {
-      const double gW1 = gK(K_W1X + m), gW2 = gK(K_W2X + m);
-      // W3y multiplies the pressure term of both qy and qz, so its gradient holds both;
-      // W3z is never read
-      const double gW3 = m < 2 ? gK(K_W3X + m) : 0.0;
-      const double D2 = D[m] * D[m];
-      const double dW1_dmp = c.dt * c1[m] / D2;
-      const double dW3_dmp = -k1 * c.Hinv / D2;
-      const double dW2_dmp = -k1 * c.Hinv * (B[m] / A[m]) / D2;
-      const double gmp = gW1 * dW1_dmp + gW2 * dW2_dmp + gW3 * dW3_dmp;
-      gA += gmp * B[m] * B[m] / (A[m] * A[m]) - gW2 * k1 * c.Hinv * B[m] / (A[m] * A[m] * D[m]);
-      gB += gmp * (-2 * B[m] / A[m]) + gW2 * k1 * c.Hinv / (A[m] * D[m]);
-      gc2 += gmp;
-    }
-    if (!azero) {
-      const double gU1 = gK(K_U1X + m), gU2 = gK(K_U2X + m);
-      gA += -gU1 * k1 * c.Hinv / (A[m] * A[m]) - gU2 * B[m] / (A[m] * A[m]);
-      gB += gU2 / A[m];
-    }
-    grho_c += 0.5 * gA;
-    atomicAdd(&c.out[4][g + mstep[m]], 0.5 * gA);
-    grf_c += 0.5 * gB + 0.5 * gc2 * tphi[p];
-    atomicAdd(&c.out[5][g + mstep[m]], 0.5 * gB + 0.5 * gc2 * tphi[p + wstep[m]]);
+  const double k1 = a.Cv * a.dt / a.Cp;  // velocity coefficient scale
+  const int64_t c2i = c + step[m];
+  const double A = 0.5 * (rho[c] + rho[c2i]), B = 0.5 * (rhof[c] + rhof[c2i]);
+  const double c1 = 0.5 * (C1[c] + C1[c2i]);
+  const double c2 = 0.5 * (tphi[c] * rhof[c] + tphi[c2i] * rhof[c2i]);
+  const double D = (c2 - B * B / A) + 0.5 * a.dt * c1;
+  auto gK = [&](int kk) { return a.grad[kk][c] * a.kfac[kk]; };
+  VelGrad g{0, 0, 0};
+  if (!c1zero) {
+    const double gW1 = gK(K_W1X + m), gW2 = gK(K_W2X + m);
+    // W3y multiplies the pressure term of both qy and qz, so its gradient holds both;
+    // W3z is never read
+    const double gW3 = m < 2 ? gK(K_W3X + m) : 0.0;
+    const double D2 = D * D;
+    const double dW1_dmp = a.dt * c1 / D2;
+    const double dW3_dmp = -k1 * a.Hinv / D2;
+    const double dW2_dmp = -k1 * a.Hinv * (B / A) / D2;
+    const double gmp = gW1 * dW1_dmp + gW2 * dW2_dmp + gW3 * dW3_dmp;
+    g.gA += gmp * B * B / (A * A) - gW2 * k1 * a.Hinv * B / (A * A * D);
+    g.gB += gmp * (-2 * B / A) + gW2 * k1 * a.Hinv / (A * D);
+    g.gc2 += gmp;
   }
-  atomicAdd(&c.out[4][g], grho_c);
-  atomicAdd(&c.out[5][g], grf_c);
+  if (!azero) {
+    const double gU1 = gK(K_U1X + m), gU2 = gK(K_U2X + m);
+    g.gA += -gU1 * k1 * a.Hinv / (A * A) - gU2 * B / (A * A);
+    g.gB += gU2 / A;
+  }
+  return g;
+}
+
+__global__ void __launch_bounds__(256) k_chain(const ChainArgs a)
+{
+  const int64_t wsy = a.wx, wsz = (int64_t)a.wx * a.wy;
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= wsz * a.wz) return;
+  const int pos[3] = {(int)(p % a.wx), (int)((p / a.wx) % a.wy), (int)(p / wsz)};
+  const int dims[3] = {a.wx, a.wy, a.wz};
+  const int64_t step[3] = {1, wsy, wsz};
+  // whether the cell dx, dy, dz steps below p has coefficients (the cells off the window's outer
+  // planes do)
+  auto holds = [&](int dx, int dy, int dz) {
+    const int d[3] = {dx, dy, dz};
+    bool ok = true;
+#pragma unroll
+    for (int m = 0; m < 3; ++m) ok = ok && pos[m] - d[m] >= 1 && pos[m] - d[m] < dims[m] - 1;
+    return ok;
+  };
+  const double *mu = a.par[1], *alp = a.par[2], *M = a.par[3], *tphi = a.par[7];
+  const double kk = a.dt * a.Cp / a.Cv;  // stress coefficient scale
+  double g[6] = {0, 0, 0, 0, 0, 0};      // lambda mu alpha M rho rho_f
+  if (holds(0, 0, 0)) {
+    // stress side: K_P1 = C kk/dx, K_P2 = M kk/dx, K_S1 = lambda_c .., K_S2 = H .., K_S3 = C ..
+    auto gK = [&](int k) { return a.grad[k][p] * a.kfac[k]; };
+    const double al = alp[p], Mp = M[p];
+    const double gC = (gK(K_P1) + gK(K_S3)) * kk * a.Hinv;
+    const double glc = gK(K_S1) * kk * a.Hinv;
+    const double gH = gK(K_S2) * kk * a.Hinv;
+    const double gMd = gK(K_P2) * kk * a.Hinv;
+    g[0] = glc + gH;
+    g[1] = 2 * gH;
+    g[2] = gC * Mp + (glc + gH) * 2 * al * Mp;
+    g[3] = gMd + gC * al + (glc + gH) * al * al;
+  }
+  // shear: 4-cell harmonic means, d mu_bar / d mu_i = mu_bar^2 / (4 mu_i^2); p is a corner of
+  // four quads in each coordinate plane
+  constexpr int ax[3][2] = {{0, 1}, {0, 2}, {1, 2}};
+  constexpr int kidx[3] = {K_SXY, K_SXZ, K_SYZ};
+  const double mp = mu[p];
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    const int64_t sa = step[ax[m][0]], sb = step[ax[m][1]];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      int d[3] = {0, 0, 0};
+      d[ax[m][0]] = e & 1;
+      d[ax[m][1]] = e >> 1;
+      if (!holds(d[0], d[1], d[2])) continue;
+      const int64_t c = p - (e & 1) * sa - (e >> 1) * sb;
+      const double hm = harmonic4(mu[c], mu[c + sa], mu[c + sb], mu[c + sa + sb]);
+      if (hm == 0) continue;
+      g[1] += a.grad[kidx[m]][c] * a.kfac[kidx[m]] * kk * a.Hinv * hm * hm / (4 * mp * mp);
+    }
+  }
+  // velocity side: p is the lower or the upper cell of each axis's averages
+#pragma unroll
+  for (int m = 0; m < 3; ++m)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      int d[3] = {0, 0, 0};
+      d[m] = e;
+      if (!holds(d[0], d[1], d[2])) continue;
+      const VelGrad v = vel_grad(a, p - e * step[m], m, step);
+      g[4] += 0.5 * v.gA;
+      g[5] += 0.5 * v.gB + 0.5 * v.gc2 * tphi[p];
+    }
+  const int64_t o = (a.x0 + pos[0]) + (a.y0 + pos[1]) * a.msy + (a.z0 + pos[2]) * a.msz;
+#pragma unroll
+  for (int q = 0; q < 6; ++q) a.out[q][o] = a.add ? a.out[q][o] + g[q] : g[q];
 }
 
 // ---- batched state copies ----

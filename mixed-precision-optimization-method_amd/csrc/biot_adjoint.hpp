@@ -78,8 +78,10 @@ hipError_t launch_adjoint_inject_batch(int prec, const InjectArgs *tab, int nsho
                                        int max_ncomp, int it, hipStream_t s);
 
 // Chain rule on the device: storage-unit coefficient gradients of one window (grad[k] times
-// kfac[k] gives dJ/dK) -> dJ/d(lambda, mu, alpha, M, rho, rho_f), added (FP64 atomics) into
-// the model-grid arrays out[6] at the window's position.  Parameters are the window's.
+// kfac[k] gives dJ/dK) -> dJ/d(lambda, mu, alpha, M, rho, rho_f), written to (add: added into)
+// the model-grid arrays out[6] at the window's position.  One thread owns one model cell, so
+// overlapping windows are added by launches that follow one another on a stream.  Parameters
+// are the window's.
 struct ChainArgs {
   const double *grad[NKC];
   double kfac[NKC];
@@ -89,6 +91,7 @@ struct ChainArgs {
   int x0, y0, z0;            // window origin in the model grid
   int64_t msy, msz;          // model strides
   double dt, Cv, Cp, Hinv;
+  int add;
 };
 hipError_t launch_chain(const ChainArgs &c, hipStream_t s);
 

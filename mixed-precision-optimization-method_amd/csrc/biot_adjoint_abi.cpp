@@ -243,25 +243,45 @@ extern "C" int biot_adjoint(biot_handle *h, const float *adj_source, double *con
     AHIP(h, launch_adjoint_flush(h->prec, order, A, h->stream));  // the segment's float partial sums
   }
   AHIP(h, hipEventRecord(h->ev1, h->stream));
+
+  // ---- gradients out.  The parameter gradients: chain rule on the device, six arrays copied
+  // back.  The parameters' upload runs beside the sweep, which is queued by now.
+  if (grad_params) {
+    double *par = nullptr, *out = nullptr;
+    if ((rc = h->chain_buffers(par, out))) return rc;
+    ChainArgs c{};
+    for (int k = 0; k < NKC; ++k) {
+      c.grad[k] = h->d_grad + (size_t)k * n;
+      c.kfac[k] = h->kfac[k];
+    }
+    for (int q = 0; q < 8; ++q) c.par[q] = par + (size_t)q * n;
+    for (int q = 0; q < 6; ++q) c.out[q] = out + (size_t)q * n;
+    c.wx = h->g.nx;
+    c.wy = h->g.ny;
+    c.wz = h->g.nz;
+    c.msy = h->g.nx;
+    c.msz = (int64_t)h->g.nx * h->g.ny;
+    const CoefScales s = coef_scales(h);
+    c.dt = s.dt;
+    c.Cv = s.Cv;
+    c.Cp = s.Cp;
+    c.Hinv = s.Hinv;
+    AHIP(h, launch_chain(c, h->stream));
+    AHIP(h, hipStreamSynchronize(h->stream));
+    for (int q = 0; q < 6; ++q)
+      AHIP(h, hipMemcpy(grad_params[q], out + (size_t)q * n, (size_t)n * sizeof(double), hipMemcpyDeviceToHost));
+  }
   AHIP(h, hipEventSynchronize(h->ev1));
   float ms = 0;
   AHIP(h, hipEventElapsedTime(&ms, h->ev0, h->ev1));
   h->last_ms = ms;
-
-  // ---- gradients out: storage-unit coefficient gradients times the per-array factor
-  std::vector<double> gK((size_t)NKC * n);
-  AHIP(h, hipMemcpy(gK.data(), h->d_grad, gK.size() * sizeof(double), hipMemcpyDeviceToHost));
-  for (int k = 0; k < NKC; ++k)
+  // coefficient gradients: storage units times the per-array factor
+  for (int k = 0; k < NKC && grad_coef; ++k) {
+    double *g = grad_coef[k];
+    if (!g) continue;
+    AHIP(h, hipMemcpy(g, h->d_grad + (size_t)k * n, (size_t)n * sizeof(double), hipMemcpyDeviceToHost));
     if (h->kfac[k] != 1.0)
-      for (int64_t c = 0; c < n; ++c) gK[(size_t)k * n + c] *= h->kfac[k];
-  if (grad_coef)
-    for (int k = 0; k < NKC; ++k)
-      if (grad_coef[k]) std::memcpy(grad_coef[k], gK.data() + (size_t)k * n, (size_t)n * sizeof(double));
-  if (grad_params) {
-    const double *gk[NKC];
-    for (int k = 0; k < NKC; ++k) gk[k] = gK.data() + (size_t)k * n;
-    for (int q = 0; q < 6; ++q) std::memset(grad_params[q], 0, (size_t)n * sizeof(double));
-    chain_params(h->g.nx, h->g.ny, h->g.nz, coef_scales(h), param_view(h), gk, grad_params);
+      for (int64_t c = 0; c < n; ++c) g[c] *= h->kfac[k];
   }
   return BIOT_OK;
 }

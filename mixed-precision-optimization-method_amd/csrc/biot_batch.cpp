@@ -691,6 +691,7 @@ int gradient_group(biot_batch *b, int s0, int s1, int nt, int every, const float
     c.Cv = b->cfg.Cv;
     c.Cp = b->cfg.Cp;
     c.Hinv = (double)(1.0f / b->cfg.dx);
+    c.add = 1;
     BHIP(b, launch_chain(c, b->stream));
   }
   for (int i = s0; i < s1; ++i) b->shots[i].h->it = nt;

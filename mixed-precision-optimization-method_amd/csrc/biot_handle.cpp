@@ -189,6 +189,37 @@ void biot_handle::adj_args(AdjArgs &A) const
   A.nupd = (uint32_t)((int64_t)(g.nx - 2 * hh) * (g.ny - 2 * hh) * (g.nz - 2 * hh));
 }
 
+// The six gradient outputs go over the float partial sums (88 n bytes, flushed by now) or, on
+// FP64 handles, over the adjoint wavefields (200 n bytes, no longer read).  The parameters take
+// 64 n bytes of their own, uploaded on the side stream while the sweep runs; where that does
+// not fit, they go over the adjoint wavefields once the sweep is done.
+int biot_handle::chain_buffers(double *&par_dev, double *&out)
+{
+  double *over_lam = (double *)d_lam;
+  out = prec == BIOT_FP64 ? over_lam + (size_t)8 * n : (double *)d_gpart;
+  par_dev = d_par;
+  if (d_par) return BIOT_OK;  // an earlier sweep of the same checkpointed run
+  hipStream_t s = side;
+  if (!s && hipStreamCreate(&side) == hipSuccess) s = side;
+  if (s && hipMalloc((void **)&d_par, (size_t)8 * n * sizeof(double)) == hipSuccess) {
+    par_dev = d_par;
+  } else {
+    d_par = nullptr;
+    (void)hipGetLastError();
+    par_dev = over_lam;
+    s = stream;
+  }
+  bool ok = true;
+  for (int q = 0; q < 8 && ok; ++q)
+    ok = hipMemcpyAsync(par_dev + (size_t)q * n, par[q].data(), (size_t)n * sizeof(double), hipMemcpyHostToDevice,
+                        s) == hipSuccess;
+  if (hipStreamSynchronize(s) == hipSuccess && ok) return BIOT_OK;
+  if (d_par) (void)hipFree(d_par);
+  d_par = nullptr;
+  err = "parameter upload failed";
+  return BIOT_ERR_HIP;
+}
+
 void biot_handle::inject_args(InjectArgs &I) const
 {
   const size_t asz = prec == BIOT_FP64 ? 8 : 4;
@@ -216,7 +247,7 @@ void biot_handle::free_adjoint()
     (void)hipFree(d_kpack);
     d_kpack = nullptr;
   }
-  for (void **p : {&d_slots, &d_lam, (void **)&d_grad, (void **)&d_gpart, (void **)&d_adjsrc})
+  for (void **p : {&d_slots, &d_lam, (void **)&d_grad, (void **)&d_gpart, (void **)&d_adjsrc, (void **)&d_par})
     if (*p) {
       (void)hipFree(*p);
       *p = nullptr;
@@ -251,6 +282,7 @@ biot_handle::~biot_handle()
   if (d_traces64) (void)hipFree(d_traces64);
   if (ev0) (void)hipEventDestroy(ev0);
   if (ev1) (void)hipEventDestroy(ev1);
+  if (side) (void)hipStreamDestroy(side);
   if (stream) (void)hipStreamDestroy(stream);
 }
 

@@ -109,6 +109,8 @@ struct biot_handle {
   double *d_grad = nullptr;                  // 22 FP64 coefficient gradients
   float *d_gpart = nullptr;                  // 22 float per-segment partial sums (not FP64 handles)
   float *d_adjsrc = nullptr;                 // adjoint source traces
+  double *d_par = nullptr;                   // the 8 parameter arrays of par, for the chain rule
+  hipStream_t side = nullptr;                // uploads beside a running sweep (made on first use)
   size_t state_bytes() const;
   size_t state_off(int piece) const;  // 0 fields, 1..3 carries of x, y, z, 4 total
   size_t state_lo_off() const;        // the residual block (lo_bytes())
@@ -128,6 +130,9 @@ struct biot_handle {
   size_t lam_bytes() const;                  // adjoint wavefields, carries, derivative adjoints
   int alloc_adjoint(int every);              // d_slots (every+1 states; none for 0), d_lam, d_grad, d_adjsrc
   void adj_args(biot::AdjArgs &A) const;     // after alloc_adjoint
+  // the device copy of par and room for the 6 parameter gradients, for work queued on the stream
+  // after the sweep that is queued now
+  int chain_buffers(double *&par_dev, double *&out);
   void inject_args(biot::InjectArgs &I) const;
 };
 
