@@ -297,7 +297,8 @@ int biot_batch_shot_count(biot_batch *b, int32_t *n);
 int biot_batch_set_model(biot_batch *b, const biot_params *model_params);
 /* the per-shot grid (for reading fields or traces through the single-grid calls) */
 int biot_batch_shot_handle(biot_batch *b, int32_t shot, biot_handle **h);
-/* tile shape and persistent grid size (blocks, a multiple of 8) of the batched launches */
+/* tile shape and persistent grid size (blocks, a multiple of 8) of the batched launches; until
+ * they are set or tuned, a shape that fits the shots' sizes and one block per tile */
 int biot_batch_set_launch(biot_batch *b, int32_t bx, int32_t by, int32_t zchunk, int32_t blocks);
 int biot_batch_get_launch(biot_batch *b, int32_t *bx, int32_t *by, int32_t *zchunk, int32_t *blocks);
 /* times tile shapes and grid sizes over trial_steps steps and keeps the fastest; leaves
@@ -322,7 +323,9 @@ int biot_batch_release(biot_batch *b);
 
 /* ---- launch shapes ---- */
 /* Tile shape of the two stencil kernels: bx*by threads per block (bx*by <= 256, bx a
- * multiple of 64), each thread marching zchunk planes of its column. */
+ * multiple of 64), each thread marching zchunk planes of its column.  A block covers bx x by
+ * cells of the x-y plane; with by = 1, bx consecutive cells that run on from row to row.  A new
+ * handle has a shape that fits its grid size. */
 int biot_set_launch_shape(biot_handle *h, int32_t bx, int32_t by, int32_t zchunk);
 int biot_get_launch_shape(biot_handle *h, int32_t *bx, int32_t *by, int32_t *zchunk);
 /* Times every candidate tile shape for trial_steps steps on this grid and keeps the

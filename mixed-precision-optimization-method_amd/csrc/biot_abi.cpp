@@ -246,7 +246,7 @@ extern "C" int biot_create(const biot_grid *g, biot_handle **out)
   if (hipSetDevice(g->device) != hipSuccess || hipStreamCreate(&h->stream) != hipSuccess ||
       hipEventCreate(&h->ev0) != hipSuccess || hipEventCreate(&h->ev1) != hipSuccess)
     return refuse(h, BIOT_ERR_HIP, "device, stream or event set-up failed");
-  h->shape = default_shape(h->prec, g->order);
+  h->shape = default_shape(h->prec, plane_waves(*g));
   rc = h->allocate();
   if (rc) {
     const std::string e = h->err;
@@ -701,7 +701,7 @@ std::string tune_key(const biot_handle *h)
   for (auto &ch : arch)
     if (ch == ' ') ch = '_';
   char buf[256];
-  snprintf(buf, sizeof buf, "v3 %s p%d o%d %dx%dx%d", arch.c_str(), h->prec, h->g.order, h->g.nx,
+  snprintf(buf, sizeof buf, "v4 %s p%d o%d %dx%dx%d", arch.c_str(), h->prec, h->g.order, h->g.nx,
            h->g.ny, h->g.nz);
   return buf;
 }
@@ -753,7 +753,7 @@ extern "C" int biot_autotune(biot_handle *h, int32_t trial_steps)
     return biot_reset(h);
   }
   static const int shapes[][2] = {{64, 4}, {64, 2}, {64, 1}, {128, 2}, {128, 1}, {256, 1}};
-  static const int chunks[] = {1, 2, 4, 8, 16, 32, 64};
+  static const int chunks[] = {1, 2, 3, 4, 8, 16, 32, 64};
   const int nzi = h->g.nz - h->g.order;
   double best_ms = 1e30;
   const LaunchShape keep = h->shape;

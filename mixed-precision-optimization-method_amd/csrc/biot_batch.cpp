@@ -38,8 +38,9 @@ struct biot_batch {
   };
   std::vector<Shot> shots;
 
-  LaunchShape shape{64, 4, 8};
-  int blocks = 2048;               // persistent grid of the batched stencil launches
+  LaunchShape shape{64, 1, 1};
+  int blocks = 8;                  // grid of the batched stencil launches
+  bool launch_set = false;         // shape and blocks are the caller's or the autotuner's
 
   // forward tables
   StepArgs *d_step = nullptr;
@@ -290,6 +291,23 @@ extern "C" int biot_batch_shot_count(biot_batch *b, int32_t *n)
 
 namespace {
 
+// tile shape and grid for shots [s0, s1) where neither the caller nor the autotuner chose them:
+// the shape a single grid of as many waves gets, and one block per tile (a smaller grid that
+// takes its tiles from the work queue is 6 % slower over 16 windows of 96-187 cells)
+void default_launch(biot_batch *b, int s0, int s1)
+{
+  int64_t waves = 0, tiles = 0;
+  for (int i = s0; i < s1; ++i) waves += plane_waves(b->shots[i].h->g);
+  b->shape = default_shape(b->cfg.precision, waves);
+  for (int i = s0; i < s1; ++i) {
+    StepArgs a;
+    b->shots[i].h->fill_args(a);
+    set_tiles(a, b->shape, b->cfg.order / 2);
+    tiles += a.ntiles;
+  }
+  b->blocks = (int)((tiles + 7) / 8 * 8);
+}
+
 // device tables of the forward launches for the current shape, for shots [s0, s1) (all
 // shots when s1 < 0); the tables hold the subset from their first entry
 int build_tables(biot_batch *b, int s0 = 0, int s1 = -1)
@@ -299,6 +317,7 @@ int build_tables(biot_batch *b, int s0 = 0, int s1 = -1)
   if (all) s1 = (int)b->shots.size();
   const int S = s1 - s0;
   if (S <= 0) return bfail(b, BIOT_ERR_STATE, "no shots");
+  if (!b->launch_set) default_launch(b, s0, s1);
   const int Sall = (int)b->shots.size();
   std::vector<StepArgs> st(S);
   std::vector<int> tiles(S + 1, 0);
@@ -311,11 +330,7 @@ int build_tables(biot_batch *b, int s0 = 0, int s1 = -1)
     biot_handle *h = b->shots[s0 + i].h;
     StepArgs &a = st[i];
     h->fill_args(a);
-    a.zchunk = b->shape.zchunk;
-    a.gx = (a.nx + b->shape.bx - 1) / b->shape.bx;
-    a.gy = (a.ny + b->shape.by - 1) / b->shape.by;
-    a.gz = (a.nz - 2 * h2 + a.zchunk - 1) / a.zchunk;
-    a.ntiles = a.gx * a.gy * a.gz;
+    set_tiles(a, b->shape, h2);
     tiles[i + 1] = tiles[i] + a.ntiles;
     h->source_args(src[i]);
     h->record_args(rec[i]);
@@ -427,6 +442,7 @@ extern "C" int biot_batch_set_launch(biot_batch *b, int32_t bx, int32_t by, int3
     return bfail(b, BIOT_ERR_ARG, "launch %dx%d, zchunk %d, %d blocks not allowed", bx, by, zchunk, blocks);
   b->shape = LaunchShape{bx, by, zchunk};
   b->blocks = blocks;
+  b->launch_set = true;
   b->built = false;
   b->drop_graph();
   return BIOT_OK;
@@ -435,6 +451,7 @@ extern "C" int biot_batch_set_launch(biot_batch *b, int32_t bx, int32_t by, int3
 extern "C" int biot_batch_get_launch(biot_batch *b, int32_t *bx, int32_t *by, int32_t *zchunk, int32_t *blocks)
 {
   if (!b || !bx || !by || !zchunk || !blocks) return BIOT_ERR_ARG;
+  if (!b->launch_set && !b->shots.empty()) default_launch(b, 0, (int)b->shots.size());
   *bx = b->shape.bx;
   *by = b->shape.by;
   *zchunk = b->shape.zchunk;
@@ -448,10 +465,12 @@ extern "C" int biot_batch_autotune(biot_batch *b, int32_t trial_steps)
   if (trial_steps < 1 || trial_steps > 1000) return bfail(b, BIOT_ERR_ARG, "trial_steps must be 1..1000");
   if (b->shots.empty()) return bfail(b, BIOT_ERR_STATE, "no shots");
   static const int shapes[][2] = {{64, 4}, {64, 2}, {64, 1}, {128, 2}, {128, 1}, {256, 1}};
-  static const int chunks[] = {2, 4, 8, 16, 32};
+  static const int chunks[] = {2, 3, 4, 8, 16};
   static const int grids[] = {1024, 2048, 4096, 1 << 30};
   const LaunchShape keep = b->shape;
   const int keep_blocks = b->blocks;
+  const bool keep_set = b->launch_set;
+  b->launch_set = true;
   LaunchShape best = keep;
   int best_blocks = keep_blocks;
   double best_ms = 1e30;
@@ -483,6 +502,7 @@ extern "C" int biot_batch_autotune(biot_batch *b, int32_t trial_steps)
       }
   b->shape = rc ? keep : best;
   b->blocks = rc ? keep_blocks : best_blocks;
+  b->launch_set = rc ? keep_set : true;
   b->built = false;
   b->drop_graph();
   if (rc) return rc == BIOT_ERR_HIP ? bfail(b, rc, "autotune timing failed") : rc;

@@ -122,6 +122,8 @@ struct StepArgs {
   int64_t sy, sz;            // strides
   int zchunk;
   int gx, gy, gz, ntiles;    // tile grid (x-y tiles of the block shape, z chunks)
+  int xy0;                   // one-row blocks: the plane cell the first tile starts at
+  uint32_t nx_rcp;           // ceil(2^32 / nx)
 };
 
 inline size_t field_bytes(int prec) { return prec == PREC_FP64 ? 8 : prec == PREC_FP32 ? 4 : 2; }
@@ -133,6 +135,24 @@ inline size_t carry_bytes(int prec) { return prec == PREC_FP64 ? 8 : prec == PRE
 struct LaunchShape {
   int bx, by, zchunk;
 };
+// the tile grid of shape sh over the update box (h cells off every face): rectangles of bx x by
+// cells, or for by = 1 runs of bx consecutive cells of the x-y plane, the first starting on a
+// 64-cell boundary of the plane
+inline void set_tiles(StepArgs &a, LaunchShape sh, int h)
+{
+  a.zchunk = sh.zchunk;
+  a.xy0 = (h * a.nx) & ~63;
+  a.nx_rcp = (uint32_t)((((uint64_t)1 << 32) + (uint64_t)a.nx - 1) / (uint64_t)a.nx);
+  if (sh.by == 1) {
+    a.gx = (int)(((int64_t)(a.ny - h) * a.nx - a.xy0 + sh.bx - 1) / sh.bx);
+    a.gy = 1;
+  } else {
+    a.gx = (a.nx + sh.bx - 1) / sh.bx;
+    a.gy = (a.ny + sh.by - 1) / sh.by;
+  }
+  a.gz = (a.nz - 2 * h + a.zchunk - 1) / a.zchunk;
+  a.ntiles = a.gx * a.gy * a.gz;
+}
 
 hipError_t launch_velocity(int prec, int order, const StepArgs &args, LaunchShape shape,
                            hipStream_t s);

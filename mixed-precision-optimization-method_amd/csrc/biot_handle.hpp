@@ -136,7 +136,9 @@ struct biot_handle {
   void inject_args(biot::InjectArgs &I) const;
 };
 
-biot::LaunchShape default_shape(int prec, int order);
+// the tile shape of a launch over that many waves a z plane (plane_waves: of one grid)
+biot::LaunchShape default_shape(int prec, int64_t plane_waves);
+int64_t plane_waves(const biot_grid &g);
 // reference arrays -> unscaled kernel coefficients on the host (1/dx and 0.01 folded)
 void host_kernel_coefs(double Hinv, const std::vector<float> (&ref)[BIOT_NCOEF],
                        std::vector<double> (&K)[biot::NKC]);

@@ -484,6 +484,27 @@ __device__ __forceinline__ bool tile_of(const StepArgs &a, int &tx, int &ty, int
   return true;
 }
 
+// The thread's column (i, j) of tile (tx, ty); false outside the update box.  A block of one row
+// takes consecutive cells of the x-y plane, running on from row to row, so that its waves are
+// full whatever nx is (a 64-wide tile leaves 36 % of the lanes of a 45-cell row idle, 26 % at 99);
+// a block of several rows takes a rectangle.  i = l mod nx by the host's reciprocal
+// ceil(2^32 / nx), whose quotient is at most one too large.
+template <int h, class AT>
+__device__ __forceinline__ bool cell_xy(const AT &a, int tx, int ty, int &i, int &j)
+{
+  if (blockDim.y == 1) {
+    const u32 l = (u32)a.xy0 + (u32)tx * blockDim.x + threadIdx.x;
+    u32 q = __umulhi(l, a.nx_rcp);
+    if (q * (u32)a.nx > l) --q;
+    j = (int)q;
+    i = (int)(l - q * (u32)a.nx);
+  } else {
+    i = tx * blockDim.x + threadIdx.x;
+    j = ty * blockDim.y + threadIdx.y;
+  }
+  return i >= h && i < a.nx - h && j >= h && j < a.ny - h;
+}
+
 template <typename A>
 __device__ __forceinline__ A prof(const void *p, int i)
 {
@@ -501,9 +522,8 @@ __device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int t
   using A = typename P::A;
   constexpr int h = ORDER / 2;
   constexpr int W = 2 * h;
-  const int i = tx * blockDim.x + threadIdx.x;
-  const int j = ty * blockDim.y + threadIdx.y;
-  if (i < h || i >= a.nx - h || j < h || j >= a.ny - h) return;
+  int i, j;
+  if (!cell_xy<h>(a, tx, ty, i, j)) return;
   const int kb = h + tz * a.zchunk;
   const int ke = min(kb + a.zchunk, a.nz - h);
   if (kb >= ke) return;
@@ -705,9 +725,8 @@ __device__ __forceinline__ void stress_tile(const AT &a, int tx, int ty, int tz)
   using A = typename P::A;
   constexpr int h = ORDER / 2;
   constexpr int W = 2 * h;
-  const int i = tx * blockDim.x + threadIdx.x;
-  const int j = ty * blockDim.y + threadIdx.y;
-  if (i < h || i >= a.nx - h || j < h || j >= a.ny - h) return;
+  int i, j;
+  if (!cell_xy<h>(a, tx, ty, i, j)) return;
   const int kb = h + tz * a.zchunk;
   const int ke = min(kb + a.zchunk, a.nz - h);
   if (kb >= ke) return;
@@ -1114,11 +1133,7 @@ hipError_t launch_step(const StepArgs &in, LaunchShape sh, hipStream_t s)
   const int nzi = a.nz - 2 * h;
   if (nzi <= 0 || a.nx <= 2 * h || a.ny <= 2 * h) return hipSuccess;
   if (sh.zchunk <= 0) return hipErrorInvalidValue;
-  a.zchunk = sh.zchunk;
-  a.gx = (a.nx + sh.bx - 1) / sh.bx;
-  a.gy = (a.ny + sh.by - 1) / sh.by;
-  a.gz = (nzi + a.zchunk - 1) / a.zchunk;
-  a.ntiles = a.gx * a.gy * a.gz;
+  set_tiles(a, sh, h);
   dim3 block(sh.bx, sh.by, 1);
   dim3 grid((unsigned)(((a.ntiles + 7) / 8) * 8));
   if (VEL)
