@@ -531,6 +531,7 @@ extern "C" int biot_set_receivers(biot_handle *h, const int64_t *cells, int64_t 
   for (int f = 0; f < NFIELD; ++f)
     if (mask & (1u << f)) h->comp[h->ncomp++] = f;
   h->nrec = nrec;
+  h->rec_cells.assign(cells, cells + nrec);
   h->rec_mask = mask;
   h->nt_max = nt_max;
   const size_t tr = (size_t)h->ncomp * nt_max * nrec;
@@ -574,6 +575,10 @@ extern "C" int biot_reset(biot_handle *h)
   return BIOT_OK;
 }
 
+// Per step: source, velocity, stress, record.  Inside a run of steps the source and the receivers
+// ride on the two half-step launches (FuseArgs); the run's first source and its last step's
+// stresses and p have launches of their own, and so have all of them where a receiver samples
+// what the source changes.
 int biot_handle::enqueue_steps(int nsteps, hipEvent_t *marks, char *states)
 {
   const size_t sb = states ? state_bytes() : 0;
@@ -581,32 +586,44 @@ int biot_handle::enqueue_steps(int nsteps, hipEvent_t *marks, char *states)
   source_args(sa);
   RecordArgs ra;
   record_args(ra);
+  const bool src_fused = source_in_stress(), rec_fused = !source_recorded();
+  auto failed = [&](hipError_t e, const char *what) {
+    return e == hipSuccess ? BIOT_OK : fail(this, BIOT_ERR_HIP, "%s launch: %s", what, hipGetErrorString(e));
+  };
+  // the arguments that record components first..last-1 of step `step`, or null
+  auto record = [&](int step, int first, int last) -> const RecordArgs * {
+    ra.it = step;
+    ra.c0 = first;
+    ra.c1 = last;
+    return d_traces && step >= 0 && step < nt_max && last > first ? &ra : nullptr;
+  };
+  const int nvel = ra.nvel;
 
   StepArgs args;
   fill_args(args);
 
-  for (int s = 0; s < nsteps; ++s) {
-    if (d_wavelet && src_mask && it < (int)wavelet.size()) {
+  int rc = BIOT_OK;
+  for (int s = 0; s < nsteps && !rc; ++s) {
+    if ((s == 0 || !src_fused) && has_source(it)) {
       sa.it = it;
-      hipError_t e = launch_source(prec, sa, stream);
-      if (e != hipSuccess) return fail(this, BIOT_ERR_HIP, "source launch: %s", hipGetErrorString(e));
+      if ((rc = failed(launch_source(prec, sa, stream), "source"))) break;
     }
     if (states) save_state(states + (size_t)s * sb);
     if (marks) (void)hipEventRecord(marks[3 * s], stream);
-    hipError_t e = launch_velocity(prec, g.order, args, shape, stream);
-    if (e != hipSuccess) return fail(this, BIOT_ERR_HIP, "velocity launch: %s", hipGetErrorString(e));
+    const RecordArgs *before = rec_fused && s > 0 ? record(it - 1, nvel, ncomp) : nullptr;
+    if ((rc = failed(launch_velocity(prec, g.order, args, shape, stream, before), "velocity"))) break;
     if (marks) (void)hipEventRecord(marks[3 * s + 1], stream);
-    e = launch_stress(prec, g.order, args, shape, stream);
-    if (e != hipSuccess) return fail(this, BIOT_ERR_HIP, "stress launch: %s", hipGetErrorString(e));
+    const bool next = src_fused && s + 1 < nsteps && has_source(it + 1);
+    sa.it = it + 1;
+    if ((rc = failed(launch_stress(prec, g.order, args, shape, stream, record(it, 0, nvel), next ? &sa : nullptr),
+                     "stress")))
+      break;
     if (marks) (void)hipEventRecord(marks[3 * s + 2], stream);
-    if (d_traces && it < nt_max) {
-      ra.it = it;
-      e = launch_record(prec, ra, stream);
-      if (e != hipSuccess) return fail(this, BIOT_ERR_HIP, "record launch: %s", hipGetErrorString(e));
-    }
+    if (!rec_fused || s + 1 == nsteps)
+      if (const RecordArgs *r = record(it, nvel, ncomp)) rc = failed(launch_record(prec, *r, stream), "record");
     ++it;
   }
-  return BIOT_OK;
+  return rc;
 }
 
 extern "C" int biot_run(biot_handle *h, int32_t nsteps)

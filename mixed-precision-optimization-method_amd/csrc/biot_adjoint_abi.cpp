@@ -205,6 +205,7 @@ extern "C" int biot_adjoint(biot_handle *h, const float *adj_source, double *con
   h->source_args(sa);
   StepArgs st;
   h->fill_args(st);
+  const bool src_fused = h->source_in_stress();
   const size_t sb = h->state_bytes();
   auto slot = [&](int q) { return (char *)h->d_slots + (size_t)q * sb; };
 
@@ -227,13 +228,15 @@ extern "C" int biot_adjoint(biot_handle *h, const float *adj_source, double *con
     h->load_state(h->ckpt[s]);
     for (int q = 0; q < K; ++q) {
       const int it = n0 + q;
-      if (h->d_wavelet && h->src_mask && it < (int)h->wavelet.size()) {
+      if ((q == 0 || !src_fused) && h->has_source(it)) {
         sa.it = it;
         AHIP(h, launch_source(h->prec, sa, h->stream));
       }
       h->save_state(slot(q));  // state of step it after its source
       AHIP(h, launch_velocity(h->prec, order, st, h->shape, h->stream));
-      AHIP(h, launch_stress(h->prec, order, st, h->shape, h->stream));
+      const bool next = src_fused && q + 1 < K && h->has_source(it + 1);
+      sa.it = it + 1;
+      AHIP(h, launch_stress(h->prec, order, st, h->shape, h->stream, nullptr, next ? &sa : nullptr));
     }
     h->save_state(slot(K));
     for (int it = n0 + K - 1; it >= n0; --it) {

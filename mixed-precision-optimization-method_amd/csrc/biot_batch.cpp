@@ -53,6 +53,7 @@ struct biot_batch {
   int nactive = 0;                 // shots the current tables cover
   int64_t max_nrec = 0;
   int max_ncomp = 0;
+  bool fused = false;              // every shot's source and receivers can ride on the half steps
   bool built = false;
   // captured steps
   hipGraphExec_t gexec = nullptr;
@@ -186,7 +187,7 @@ extern "C" int biot_batch_create(const biot_batch_config *c, biot_batch **out)
   b->cfg = *c;
   if (hipSetDevice(c->device) != hipSuccess || hipStreamCreate(&b->stream) != hipSuccess ||
       hipEventCreate(&b->ev0) != hipSuccess || hipEventCreate(&b->ev1) != hipSuccess ||
-      hipMalloc((void **)&b->d_it, sizeof(int)) != hipSuccess ||
+      hipMalloc((void **)&b->d_it, 3 * sizeof(int)) != hipSuccess ||
       hipMalloc((void **)&b->d_queue, 16 * sizeof(int)) != hipSuccess ||
       hipMemset(b->d_queue, 0, 16 * sizeof(int)) != hipSuccess)
     return refuse(b, BIOT_ERR_HIP, "device, stream, event or counter set-up failed");
@@ -325,6 +326,7 @@ int build_tables(biot_batch *b, int s0 = 0, int s1 = -1)
   std::vector<RecordArgs> rec(S);
   b->max_nrec = 0;
   b->max_ncomp = 0;
+  b->fused = true;
   const int h2 = b->cfg.order / 2;
   for (int i = 0; i < S; ++i) {
     biot_handle *h = b->shots[s0 + i].h;
@@ -336,6 +338,7 @@ int build_tables(biot_batch *b, int s0 = 0, int s1 = -1)
     h->record_args(rec[i]);
     b->max_nrec = std::max(b->max_nrec, h->nrec);
     b->max_ncomp = std::max(b->max_ncomp, h->ncomp);
+    b->fused = b->fused && !h->source_recorded() && (!h->src_mask || h->source_in_stress());
   }
   b->total_tiles = tiles[S];
   b->nactive = S;
@@ -358,26 +361,49 @@ BatchArgs batch_args(const biot_batch *b)
 {
   // a grid smaller than the tile list takes its tiles from the work queue
   int *q = b->blocks < b->total_tiles ? b->d_queue : nullptr;
-  return BatchArgs{b->d_step, b->d_tiles, b->nactive, b->total_tiles, q};
+  BatchArgs a{};
+  a.shots = b->d_step;
+  a.tile_start = b->d_tiles;
+  a.nshots = b->nactive;
+  a.total_tiles = b->total_tiles;
+  a.queue = q;
+  a.src = b->fused ? b->d_src : nullptr;
+  a.rec = b->d_rec;
+  a.it = b->d_it;
+  return a;
 }
 
-// one step of every shot: source, velocity, stress, (record), counter + 1
-int enqueue_step(biot_batch *b, bool record)
+// step `off` after the counter's of every shot: velocity, stress, and the source of the next
+// step and the recorded samples on them (FuseArgs); where a shot's source or receivers cannot
+// ride on the half steps, source and record launches for all.  The first step's source is
+// start_steps' launch, the last step's stresses and p are end_steps'.
+int enqueue_step(biot_batch *b, bool record, int off)
 {
-  const int S = b->nactive;
   const int prec = b->cfg.precision, order = b->cfg.order;
-  const BatchArgs ba = batch_args(b);
-  BHIP(b, launch_source_batch(prec, b->d_src, S, b->d_it, b->stream));
-  BHIP(b, launch_step_batch(prec, order, true, ba, b->shape, b->blocks, b->stream));
-  BHIP(b, launch_step_batch(prec, order, false, ba, b->shape, b->blocks, b->stream));
-  if (record) BHIP(b, launch_record_batch(prec, b->d_rec, S, b->max_nrec, b->max_ncomp, b->d_it, b->stream));
-  BHIP(b, launch_advance(b->d_it, b->stream));
+  BatchArgs ba = batch_args(b);
+  ba.off = off;
+  const int64_t rec = record && b->fused ? b->max_nrec : 0;
+  if (!b->fused) BHIP(b, launch_source_batch(prec, b->d_src, b->nactive, b->d_it, off, b->stream));
+  BHIP(b, launch_step_batch(prec, order, true, ba, b->shape, b->blocks, rec, b->stream));
+  BHIP(b, launch_step_batch(prec, order, false, ba, b->shape, b->blocks, rec, b->stream));
+  if (record && !b->fused)
+    BHIP(b, launch_record_batch(prec, b->d_rec, b->nactive, b->max_nrec, true, b->d_it, off, b->stream));
   return BIOT_OK;
 }
 
-int set_counter(biot_batch *b, int it)
+// the counter at step `it` of a run of n steps, its first source added
+int start_steps(biot_batch *b, int it, int n)
 {
-  BHIP(b, launch_set_counter(b->d_it, it, b->stream));
+  BHIP(b, launch_set_counter(b->d_it, it, it + n, b->stream));
+  if (b->fused)
+    BHIP(b, launch_source_batch(b->cfg.precision, b->d_src, b->nactive, b->d_it, 0, b->stream));
+  return BIOT_OK;
+}
+// the counter is past the run's last step (off: its distance from the counter)
+int end_steps(biot_batch *b, bool record, int off)
+{
+  if (record && b->fused)
+    BHIP(b, launch_record_batch(b->cfg.precision, b->d_rec, b->nactive, b->max_nrec, false, b->d_it, off, b->stream));
   return BIOT_OK;
 }
 
@@ -388,7 +414,8 @@ int ensure_graph(biot_batch *b, int steps, bool record)
   hipGraph_t graph = nullptr;
   BHIP(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
   int rc = BIOT_OK;
-  for (int s = 0; s < steps && !rc; ++s) rc = enqueue_step(b, record);
+  for (int s = 0; s < steps && !rc; ++s) rc = enqueue_step(b, record, s);
+  if (!rc && launch_advance(b->d_it, steps, b->stream) != hipSuccess) rc = BIOT_ERR_HIP;
   hipGraph_t g2 = nullptr;
   const hipError_t e = hipStreamEndCapture(b->stream, &g2);
   graph = g2;
@@ -408,20 +435,20 @@ int ensure_graph(biot_batch *b, int steps, bool record)
   return BIOT_OK;
 }
 
-// nt steps from the counter's current value: whole graphs, then single steps
-int run_steps(biot_batch *b, int nt, int graph_steps, bool record)
+// steps it..it+nt-1: whole graphs, then single steps
+int run_steps(biot_batch *b, int it, int nt, int graph_steps, bool record)
 {
+  int rc = start_steps(b, it, nt);
+  if (rc) return rc;
   int done = 0;
   if (graph_steps > 0 && nt >= graph_steps) {
-    int rc = ensure_graph(b, graph_steps, record);
-    if (rc) return rc;
+    if ((rc = ensure_graph(b, graph_steps, record))) return rc;
     for (; done + graph_steps <= nt; done += graph_steps) BHIP(b, hipGraphLaunch(b->gexec, b->stream));
   }
-  for (; done < nt; ++done) {
-    int rc = enqueue_step(b, record);
-    if (rc) return rc;
-  }
-  return BIOT_OK;
+  int off = 0;
+  for (; done < nt; ++done, ++off)
+    if ((rc = enqueue_step(b, record, off))) return rc;
+  return end_steps(b, record, off - 1);
 }
 
 int reset_all(biot_batch *b)
@@ -486,11 +513,11 @@ extern "C" int biot_batch_autotune(biot_batch *b, int32_t trial_steps)
         const int gb = std::min(gblocks, ((b->total_tiles + 7) / 8) * 8);
         if (gblocks == (1 << 30) || gb == gblocks) b->blocks = gb;
         else continue;  // a grid larger than the tile list is the "one block per tile" case
-        if ((rc = set_counter(b, 0))) break;
-        if ((rc = enqueue_step(b, false))) break;  // warm-up
+        if ((rc = start_steps(b, 0, trial_steps + 1))) break;
+        if ((rc = enqueue_step(b, false, 0))) break;  // warm-up
         float ms = 0;
         if (hipEventRecord(b->ev0, b->stream) != hipSuccess) rc = BIOT_ERR_HIP;
-        for (int s = 0; s < trial_steps && !rc; ++s) rc = enqueue_step(b, false);
+        for (int s = 0; s < trial_steps && !rc; ++s) rc = enqueue_step(b, false, s + 1);
         if (!rc && (hipEventRecord(b->ev1, b->stream) != hipSuccess || hipEventSynchronize(b->ev1) != hipSuccess ||
                     hipEventElapsedTime(&ms, b->ev0, b->ev1) != hipSuccess))
           rc = BIOT_ERR_HIP;
@@ -515,10 +542,9 @@ extern "C" int biot_batch_forward(biot_batch *b, int32_t nt, int32_t graph_steps
   if (nt <= 0 || graph_steps < 0) return bfail(b, BIOT_ERR_ARG, "nt must be positive, graph_steps >= 0");
   int rc = build_tables(b);
   if (!rc) rc = reset_all(b);
-  if (!rc) rc = set_counter(b, 0);
   if (rc) return rc;
   BHIP(b, hipEventRecord(b->ev0, b->stream));
-  rc = run_steps(b, nt, graph_steps, true);
+  rc = run_steps(b, 0, nt, graph_steps, true);
   if (rc) return rc;
   BHIP(b, hipEventRecord(b->ev1, b->stream));
   BHIP(b, hipEventSynchronize(b->ev1));
@@ -649,12 +675,11 @@ int gradient_group(biot_batch *b, int s0, int s1, int nt, int every, const float
     int r = biot_reset(b->shots[i].h);
     if (r) return hfail(b, b->shots[i].h, r, "reset");
   }
-  if ((rc = set_counter(b, 0))) return rc;
 
   // ---- forward with checkpoints
   for (int k = 0; k < nseg; ++k) {
     BHIP(b, save_ckpt(k));
-    if ((rc = run_steps(b, std::min(every, nt - k * every), 0, true))) return rc;
+    if ((rc = run_steps(b, k * every, std::min(every, nt - k * every), 0, true))) return rc;
   }
   // ---- FP64 misfit per shot; the residual is the adjoint source
   for (int i = s0; i < s1; ++i) {
@@ -672,14 +697,14 @@ int gradient_group(biot_batch *b, int s0, int s1, int nt, int every, const float
   for (int k = nseg - 1; k >= 0; --k) {
     const int n0 = k * every, K = std::min(every, nt - n0);
     BHIP(b, load_ckpt(k));
-    BHIP(b, launch_set_counter(b->d_it, n0, b->stream));
-    const BatchArgs ba = batch_args(b);
+    if ((rc = start_steps(b, n0, K))) return rc;
     for (int q = 0; q < K; ++q) {
-      BHIP(b, launch_source_batch(prec, b->d_src, S, b->d_it, b->stream));
+      if (!b->fused) BHIP(b, launch_source_batch(prec, b->d_src, S, b->d_it, q, b->stream));
       BHIP(b, save_slot(q));
-      BHIP(b, launch_step_batch(prec, order, true, ba, b->shape, b->blocks, b->stream));
-      BHIP(b, launch_step_batch(prec, order, false, ba, b->shape, b->blocks, b->stream));
-      BHIP(b, launch_advance(b->d_it, b->stream));
+      BatchArgs ba = batch_args(b);
+      ba.off = q;
+      BHIP(b, launch_step_batch(prec, order, true, ba, b->shape, b->blocks, 0, b->stream));
+      BHIP(b, launch_step_batch(prec, order, false, ba, b->shape, b->blocks, 0, b->stream));
     }
     BHIP(b, save_slot(K));
     for (int it = n0 + K - 1; it >= n0; --it) {

@@ -122,6 +122,7 @@ struct StepArgs {
   int64_t sy, sz;            // strides
   int zchunk;
   int gx, gy, gz, ntiles;    // tile grid (x-y tiles of the block shape, z chunks)
+  int src[3];                // the source cell (no cell's position: no source)
   int xy0;                   // one-row blocks: the plane cell the first tile starts at
   uint32_t nx_rcp;           // ceil(2^32 / nx)
 };
@@ -154,10 +155,6 @@ inline void set_tiles(StepArgs &a, LaunchShape sh, int h)
   a.ntiles = a.gx * a.gy * a.gz;
 }
 
-hipError_t launch_velocity(int prec, int order, const StepArgs &args, LaunchShape shape,
-                           hipStream_t s);
-hipError_t launch_stress(int prec, int order, const StepArgs &args, LaunchShape shape,
-                         hipStream_t s);
 struct SourceArgs {
   void *f[NFIELD];
   int8_t *lo[NFIELD];
@@ -173,8 +170,10 @@ struct RecordArgs {
   const int8_t *lo[NFIELD];
   const int64_t *rec;       // device receiver cells
   int64_t nrec;
-  int comp[NFIELD];
+  int comp[NFIELD];         // recorded fields, ascending
   int ncomp;
+  int c0, c1;               // the components this launch records
+  int nvel;                 // components 0..nvel-1 are velocities, the others stresses and p
   float scale[NFIELD];      // storage scale per recorded component
   float *traces;            // device [comp][nt_max][nrec]
   double *traces64;         // same layout in double (FP64 handles), or null
@@ -182,6 +181,24 @@ struct RecordArgs {
                             // none so far), or null
   int it, nt_max;
 };
+// A half step's launch also does the work around it that touches only fields it leaves alone:
+// the velocity launch records the stresses and p of the step before, the stress launch the
+// velocities of its own step (blocks after the tiles'), and the thread that updates the source
+// cell's stresses then adds the next step's source there.  On their own the two were 4.5 us
+// launches of a few waves (200 steps of 64^3 FP32 with their outputs: 6.4 ms in four launches a
+// step, 5.7 ms in two; 45x38x53 at order 2, 150 steps: 3.8 ms and 3.3 ms).
+struct FuseArgs {
+  int tile_blocks;          // blocks of the tiles (set by the launcher); the others record
+  int record;               // rec holds something to record
+  int source;               // src is to be added (stress launch)
+  RecordArgs rec;
+  SourceArgs src;
+};
+// rec (c0, c1 and it set; may be null), src (it set; stress launch; may be null): see FuseArgs
+hipError_t launch_velocity(int prec, int order, const StepArgs &args, LaunchShape shape, hipStream_t s,
+                           const RecordArgs *rec = nullptr);
+hipError_t launch_stress(int prec, int order, const StepArgs &args, LaunchShape shape, hipStream_t s,
+                         const RecordArgs *rec = nullptr, const SourceArgs *src = nullptr);
 // the byte pattern a cleared non-finite flag holds (every byte 0x7F): larger than any step
 constexpr int NONFINITE_NONE = 0x7F7F7F7F;
 hipError_t launch_source(int prec, const SourceArgs &a, hipStream_t s);
@@ -220,17 +237,28 @@ struct BatchArgs {
   int nshots, total_tiles;
   int *queue;               // device, 16 ints (zero between launches): per XCD group the tile
                             // counter and the count of finished blocks; null: one block per tile
+  // the work around the half step, as FuseArgs per shot: step it[0] + off, the sources of steps
+  // below it[1] added by the stress launch (src null: none), the blocks from tile_blocks on
+  // recording rec_blocks blocks a shot (rec_blocks 0: none; a step before it[2] is not recorded)
+  const SourceArgs *src;
+  const RecordArgs *rec;
+  const int *it;
+  int off, tile_blocks, rec_blocks;
 };
-// blocks: the persistent grid size (a multiple of 8)
+// blocks: the persistent grid size (a multiple of 8); max_nrec: the most receivers a shot has
+// (0: record nothing)
 hipError_t launch_step_batch(int prec, int order, bool vel, const BatchArgs &b, LaunchShape sh,
-                             int blocks, hipStream_t s);
-hipError_t launch_source_batch(int prec, const SourceArgs *tab, int nshots, const int *it,
+                             int blocks, int64_t max_nrec, hipStream_t s);
+// the sources of step it[0] + off; the components of step it[0] + off (vel: the velocities too,
+// else the stresses and p alone)
+hipError_t launch_source_batch(int prec, const SourceArgs *tab, int nshots, const int *it, int off,
                                hipStream_t s);
 hipError_t launch_record_batch(int prec, const RecordArgs *tab, int nshots, int64_t max_nrec,
-                               int max_ncomp, const int *it, hipStream_t s);
-// *it += 1 / *it = v on the device (kernels, so they may sit in a captured graph)
-hipError_t launch_advance(int *it, hipStream_t s);
-hipError_t launch_set_counter(int *it, int v, hipStream_t s);
+                               bool vel, const int *it, int off, hipStream_t s);
+// it[0] += d / it[0] = it[2] = v, it[1] = end on the device (kernels, so they may sit in a
+// captured graph)
+hipError_t launch_advance(int *it, int d, hipStream_t s);
+hipError_t launch_set_counter(int *it, int v, int end, hipStream_t s);
 // multiply a stored array by f (lo: its residuals or null); carries use prec of the carry
 // type, i.e. pass PREC_FP32 for FP16C/FP16T carries and PREC_FP16 for FP16 carries
 hipError_t launch_rescale(int prec, void *p, int8_t *lo, int64_t n, double f, hipStream_t s);

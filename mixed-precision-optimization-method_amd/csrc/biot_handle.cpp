@@ -73,11 +73,27 @@ void biot_handle::record_args(RecordArgs &ra) const
   for (int c = 0; c < ncomp; ++c) {
     ra.comp[c] = comp[c];
     ra.scale[c] = fscale[comp[c]];
+    ra.nvel += comp[c] < 6;
   }
+  ra.c1 = ncomp;
   ra.traces = (float *)d_traces;
   ra.traces64 = d_traces64;
   ra.nonfinite = d_flag;
   ra.nt_max = nt_max;
+}
+
+bool biot_handle::source_recorded() const
+{
+  return (src_mask & rec_mask & ~0x3Fu) &&
+         std::find(rec_cells.begin(), rec_cells.end(), src_cell) != rec_cells.end();
+}
+
+bool biot_handle::source_in_stress() const
+{
+  if (!d_wavelet || !src_mask || (src_mask & 0x3Fu) || source_recorded()) return false;
+  const int h = g.order / 2;
+  const int64_t i = src_cell % g.nx, j = src_cell / g.nx % g.ny, k = src_cell / ((int64_t)g.nx * g.ny);
+  return i >= h && i < g.nx - h && j >= h && j < g.ny - h && k >= h && k < g.nz - h;
 }
 
 int biot_handle::clear_nonfinite()
@@ -330,6 +346,9 @@ void biot_handle::fill_args(StepArgs &a) const
     a.R[ax] = R[ax];
     for (int q = 0; q < 4; ++q) a.prof[ax][q] = d_prof[ax][q];
   }
+  a.src[0] = src_mask ? (int)(src_cell % g.nx) : -1;
+  a.src[1] = (int)(src_cell / g.nx % g.ny);
+  a.src[2] = (int)(src_cell / ((int64_t)g.nx * g.ny));
   a.nx = g.nx;
   a.ny = g.ny;
   a.nz = g.nz;

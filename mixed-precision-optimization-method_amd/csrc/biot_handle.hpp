@@ -55,6 +55,7 @@ struct biot_handle {
   void *d_traces = nullptr;
   double *d_traces64 = nullptr;  // FP64 handles: the traces in double as well
   int64_t nrec = 0;
+  std::vector<int64_t> rec_cells;  // host copy
   uint32_t rec_mask = 0;
   int comp[biot::NFIELD] = {};
   int ncomp = 0;
@@ -124,7 +125,14 @@ struct biot_handle {
 
   // argument blocks shared by the single-grid and batched drivers
   void source_args(biot::SourceArgs &sa) const;
-  void record_args(biot::RecordArgs &ra) const;
+  void record_args(biot::RecordArgs &ra) const;  // every component
+  bool has_source(int step) const { return d_wavelet && src_mask && step < (int)wavelet.size(); }
+  // whether a receiver records a stress or p at the source cell that the source changes: it then
+  // has to be sampled before the next step's source is added
+  bool source_recorded() const;
+  // whether the stress launch can add the next step's source (fields it writes, at a cell it
+  // updates, not sampled after it)
+  bool source_in_stress() const;
   int clear_nonfinite();                     // enqueue a clear of d_flag on the stream
   int check_nonfinite();                     // synchronize; BIOT_ERR_NONFINITE if it was set
   size_t lam_bytes() const;                  // adjoint wavefields, carries, derivative adjoints

@@ -471,7 +471,8 @@ __device__ __forceinline__ int slab_pos(int i, int n, int Lw, int Rw)
 // b % 8 in order; each XCD here gets one contiguous range of tiles, x fastest then y then
 // z, so the y- and z-adjacent tiles whose halos overlap are processed by the same XCD,
 // close in time, and the halo re-reads hit that XCD's L2.
-__device__ __forceinline__ bool tile_of(const StepArgs &a, int &tx, int &ty, int &tz)
+template <class AT>
+__device__ __forceinline__ bool tile_of(const AT &a, int &tx, int &ty, int &tz)
 {
   const int b = blockIdx.x;
   const int per = (a.ntiles + 7) >> 3;
@@ -718,18 +719,20 @@ __device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int t
   }
 }
 
-// one x-y tile of the update box, planes kb..ke-1 of z chunk tz
+// one x-y tile of the update box, planes kb..ke-1 of z chunk tz; true in the thread that updated
+// the source cell
 template <class P, int ORDER, bool NT, class AT>
-__device__ __forceinline__ void stress_tile(const AT &a, int tx, int ty, int tz)
+__device__ __forceinline__ bool stress_tile(const AT &a, int tx, int ty, int tz)
 {
   using A = typename P::A;
   constexpr int h = ORDER / 2;
   constexpr int W = 2 * h;
   int i, j;
-  if (!cell_xy<h>(a, tx, ty, i, j)) return;
+  if (!cell_xy<h>(a, tx, ty, i, j)) return false;
   const int kb = h + tz * a.zchunk;
   const int ke = min(kb + a.zchunk, a.nz - h);
-  if (kb >= ke) return;
+  if (kb >= ke) return false;
+  const bool own = i == a.src[0] && j == a.src[1] && a.src[2] >= kb && a.src[2] < ke;
   const u32 sy = (u32)a.sy, sz = (u32)a.sz;
   const u32 col = (u32)i + (u32)j * sy;
 
@@ -889,120 +892,40 @@ __device__ __forceinline__ void stress_tile(const AT &a, int tx, int ty, int tz)
       wvy[m] = wvy[m + 1];
     }
   }
+  return own;
 }
 
-template <class P, int ORDER>
-__global__ void __launch_bounds__(256) k_velocity(const StepArgs a)
-{
-  int tx, ty, tz;
-  if (!tile_of(a, tx, ty, tz)) return;
-  velocity_tile<P, ORDER, true>(a, tx, ty, tz);
-}
-template <class P, int ORDER>
-__global__ void __launch_bounds__(256) k_stress(const StepArgs a)
-{
-  int tx, ty, tz;
-  if (!tile_of(a, tx, ty, tz)) return;
-  stress_tile<P, ORDER, true>(a, tx, ty, tz);
-}
-
-// Batched forms: one persistent grid walks the tiles of every shot.  The shots' tile
-// lists are concatenated (tile_start[s] = first global tile of shot s); each XCD takes one
-// contiguous range of that list, so a shot's neighbouring tiles share an L2, and a block
-// strides through its XCD's range until it is exhausted (every wave exits).
-// The argument tables are read-only for a launch and indexed uniformly per block: read
-// them through the constant address space, so the compiler keeps them in scalar registers
-// (as it does kernel arguments) instead of a VGPR pair per pointer.
-typedef __attribute__((address_space(4))) const StepArgs CStepArgs;
-typedef __attribute__((address_space(4))) const int CInt;
-__device__ __forceinline__ int shot_of(const BatchArgs &b, int t)
-{
-  CInt *ts = ((CInt *)b.tile_start);
-  int lo = 0, hi = b.nshots - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (ts[mid] <= t) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
-}
-template <class P, int ORDER, bool VEL>
-__global__ void __launch_bounds__(256) k_step_batch(const BatchArgs b)
-{
-  // workgroup b goes to XCD b % 8; XCD group x owns the contiguous tile range [begin, end) of
-  // the concatenated tile lists
-  const int x = blockIdx.x & 7;
-  const int per = (b.total_tiles + 7) >> 3;
-  const int begin = x * per, end = min((x + 1) * per, b.total_tiles);
-  auto tile = [&](int t) {
-    const int s = shot_of(b, t);
-    const CStepArgs &a = ((CStepArgs *)b.shots)[s];
-    const int lt = t - ((CInt *)b.tile_start)[s];
-    const int tx = lt % a.gx, r = lt / a.gx, ty = r % a.gy, tz = r / a.gy;
-    if (VEL) velocity_tile<P, ORDER, false>(a, tx, ty, tz);
-    else stress_tile<P, ORDER, false>(a, tx, ty, tz);
-  };
-  // Both mappings run one loop, so the tile body is inlined once (two inlined copies took the
-  // residual policies' kernels to 248-256 VGPRs).
-  // Fixed mapping (no queue): block l of the group takes tiles l, l + per_x, ...
-  // Work queue: a block takes the group's next tile from the group's counter (one atomic a
-  // tile, the next one claimed while the current one runs), so blocks that drew cheap tiles
-  // take more.  Every block ends on one claim past the range; the last block of the group to
-  // make it sets the group's two counters back to zero for the next launch (no other block
-  // of the group touches them after its own last claim).  The branches on the queue are
-  // uniform over the launch, so the barriers inside them are reached by every thread.
-  __shared__ int s_next;
-  const bool queue = b.queue != nullptr;
-  const bool lead = threadIdx.x == 0 && threadIdx.y == 0;
-  int *ctr = queue ? b.queue + x : nullptr, *done = queue ? b.queue + 8 + x : nullptr;
-  int t = begin + (blockIdx.x >> 3);
-  if (queue) {
-    if (lead) s_next = atomicAdd(ctr, 1);
-    __syncthreads();
-    t = begin + s_next;
-  }
-  while (t < end) {
-    if (queue) {
-      __syncthreads();  // every thread has read s_next
-      if (lead) s_next = atomicAdd(ctr, 1);
-    }
-    tile(t);
-    if (queue) {
-      __syncthreads();  // the next claim is in s_next
-      t = begin + s_next;
-    } else {
-      t += gridDim.x >> 3;
-    }
-  }
-  if (queue && lead && atomicAdd(done, 1) == (int)(gridDim.x >> 3) - 1) {
-    atomicExch(ctr, 0);
-    atomicExch(done, 0);
-  }
-}
-
-// Source injection (kernel.cu:130-142) for one cell: one lane per field.
-template <class P>
-__device__ __forceinline__ void source_cell(const SourceArgs &sa, int it)
+// Source injection (kernel.cu:130-142) of step it into field f of the source cell.
+template <class P, class SA>
+__device__ __forceinline__ void source_field(const SA &sa, int f, int it)
 {
   using A = typename P::A;
-  const int f = threadIdx.x;
-  if (f >= NFIELD || !(sa.mask & (1u << f))) return;
   const u32 c = (u32)sa.cell;
   const bool cf = (P::cmask >> f) & 1u;
   const A amp = (A)sa.wavelet[it] * (A)sa.inv_scale[f];
   store_raw<P>(sa.f[f], sa.lo[f], cf, c, load_raw<P>(sa.f[f], sa.lo[f], cf, c) + amp);
 }
+// one lane per field
 template <class P>
-__global__ void k_source(const SourceArgs sa)
+__device__ __forceinline__ void source_cell(const SourceArgs &sa, int it)
 {
-  source_cell<P>(sa, sa.it);
+  const int f = threadIdx.x;
+  if (f >= NFIELD || !(sa.mask & (1u << f))) return;
+  source_field<P>(sa, f, it);
+}
+// After a tile of the stress half step: the thread that updated the source cell adds step it's
+// source to it.  No other thread of the launch reads or writes that cell's stresses.
+template <class P, class SA>
+__device__ __forceinline__ void source_owner(const SA &sa, int it)
+{
+  for (int f = 0; f < NFIELD; ++f)
+    if (sa.mask & (1u << f)) source_field<P>(sa, f, it);
 }
 
 // Receiver sampling: traces[comp][it][rec] = field value * storage scale.
-template <class P>
-__device__ __forceinline__ void record_one(const RecordArgs &ra, int64_t r, int ci, int it)
+template <class P, class RA>
+__device__ __forceinline__ void record_one(const RA &ra, int64_t r, int ci, int it)
 {
-  if (r >= ra.nrec || ci >= ra.ncomp) return;
   const int f = ra.comp[ci];
   // the product of two floats is exact in double, so (float)v is the rounded float product
   const double v = (double)load_raw<P>(ra.f[f], ra.lo[f], (P::cmask >> f) & 1u, (u32)ra.rec[r]) *
@@ -1015,37 +938,180 @@ __device__ __forceinline__ void record_one(const RecordArgs &ra, int64_t r, int 
   // at which a receiver sees NaN or Inf
   if (ra.nonfinite && !__builtin_isfinite(vf)) atomicMin(ra.nonfinite, it);
 }
+// components c0..c1-1 of the receiver a block-th thread of recording block b stands for
+template <class P, class RA>
+__device__ __forceinline__ void record_block(const RA &ra, int b, int c0, int c1, int it)
+{
+  const int64_t r = (int64_t)b * (blockDim.x * blockDim.y) + threadIdx.y * blockDim.x + threadIdx.x;
+  if (r >= ra.nrec) return;
+  for (int ci = c0; ci < c1; ++ci) record_one<P>(ra, r, ci, it);
+}
+
+// the constant address space: uniform reads through it stay in scalar registers
+typedef __attribute__((address_space(4))) const StepArgs CStepArgs;
+typedef __attribute__((address_space(4))) const FuseArgs CFuseArgs;
+typedef __attribute__((address_space(4))) const BatchArgs CBatchArgs;
+typedef __attribute__((address_space(4))) const int CInt;
+typedef __attribute__((address_space(4))) const SourceArgs CSourceArgs;
+typedef __attribute__((address_space(4))) const RecordArgs CRecordArgs;
+// the kernel's arguments (the first of type T) read from the argument segment here and not before;
+// the stress kernel's FuseArgs follow its StepArgs without padding
+static_assert(sizeof(StepArgs) % alignof(FuseArgs) == 0, "FuseArgs must follow StepArgs directly");
+template <class T>
+__device__ __forceinline__ __attribute__((address_space(4))) const T *late_args()
+{
+  uint64_t p = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return (__attribute__((address_space(4))) const T *)p;
+}
+
+template <class P, int ORDER>
+__global__ void __launch_bounds__(256) k_velocity(const StepArgs a, const FuseArgs u)
+{
+  if ((int)blockIdx.x >= u.tile_blocks) {
+    record_block<P>(u.rec, blockIdx.x - u.tile_blocks, u.rec.c0, u.rec.c1, u.rec.it);
+    return;
+  }
+  int tx, ty, tz;
+  if (!tile_of(a, tx, ty, tz)) return;
+  velocity_tile<P, ORDER, true>(a, tx, ty, tz);
+}
+template <class P, int ORDER>
+__global__ void __launch_bounds__(256) k_stress(const StepArgs a, const FuseArgs u)
+{
+  if ((int)blockIdx.x >= u.tile_blocks) {
+    record_block<P>(u.rec, blockIdx.x - u.tile_blocks, u.rec.c0, u.rec.c1, u.rec.it);
+    return;
+  }
+  int tx, ty, tz;
+  if (!tile_of(a, tx, ty, tz)) return;
+  if (!stress_tile<P, ORDER, true>(a, tx, ty, tz)) return;
+  // the arguments of what follows are read here, so that none of them is kept in scalar registers
+  // over the plane loop (kept, they spilled 16 more of the FP16T kernel's)
+  CFuseArgs &u1 = *(CFuseArgs *)(late_args<StepArgs>() + 1);
+  if (u1.source) source_owner<P>(u1.src, u1.src.it);
+}
+
+// Batched forms: one launch covers the tiles of every shot.  The shots' tile lists are
+// concatenated (tile_start[s] = first global tile of shot s); each XCD takes one contiguous range
+// of that list, so a shot's neighbouring tiles share an L2.  The argument tables are read-only for
+// a launch and indexed uniformly per block: read them through the constant address space, so the
+// compiler keeps them in scalar registers (as it does kernel arguments) instead of a VGPR pair per
+// pointer.
+template <class BA>
+__device__ __forceinline__ int shot_of(const BA &b, int t)
+{
+  CInt *ts = ((CInt *)b.tile_start);
+  int lo = 0, hi = b.nshots - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (ts[mid] <= t) lo = mid;
+    else hi = mid - 1;
+  }
+  return lo;
+}
+// tile t of the concatenated lists
+template <class P, int ORDER, bool VEL>
+__device__ __forceinline__ void batch_tile(const BatchArgs &b, int t)
+{
+  const int s = shot_of(b, t);
+  const CStepArgs &a = ((CStepArgs *)b.shots)[s];
+  const int lt = t - ((CInt *)b.tile_start)[s];
+  const int tx = lt % a.gx, r = lt / a.gx, ty = r % a.gy, tz = r / a.gy;
+  if constexpr (VEL) {
+    velocity_tile<P, ORDER, false>(a, tx, ty, tz);
+  } else if (stress_tile<P, ORDER, false>(a, tx, ty, tz)) {
+    CBatchArgs &b1 = *late_args<BatchArgs>();
+    CSourceArgs &sa = ((CSourceArgs *)b1.src)[shot_of(b1, t)];
+    const int it = ((CInt *)b1.it)[0] + b1.off + 1;
+    if (b1.src && sa.wavelet && it < sa.nt_w && it < ((CInt *)b1.it)[1]) source_owner<P>(sa, it);
+  }
+}
+// QUEUE false: one block per tile, workgroup b on XCD b % 8, XCD group x owning the contiguous tile
+// range [begin, end).  QUEUE: a smaller grid whose blocks take their group's next tile from the
+// group's counter (one atomic a tile, the next one claimed while the current one runs), so blocks
+// that drew cheap tiles take more.  Every block ends on one claim past the range; the last block
+// of the group to make it sets the group's two counters back to zero for the next launch (no
+// other block of the group touches them after its own last claim).  Two kernels, because one loop
+// for both kept the queue's state in scalar registers over the plane loop (6-35 of them spilled
+// at order 4; without the queue 0-5, and FP16's velocity kernel fits 5 waves a SIMD, not 4).
+template <class P, int ORDER, bool VEL, bool QUEUE>
+__global__ void __launch_bounds__(256) k_step_batch(const BatchArgs b)
+{
+  if ((int)blockIdx.x >= b.tile_blocks) {
+    // velocity launch: the stresses and p of the step before; stress launch: the step's velocities
+    const int rb = blockIdx.x - b.tile_blocks, s = rb / b.rec_blocks;
+    const CRecordArgs &ra = ((CRecordArgs *)b.rec)[s];
+    const int it = ((CInt *)b.it)[0] + b.off - (VEL ? 1 : 0);
+    if (!ra.traces || it < ((CInt *)b.it)[2] || it >= ra.nt_max) return;
+    record_block<P>(ra, rb - s * b.rec_blocks, VEL ? ra.nvel : 0, VEL ? ra.ncomp : ra.nvel, it);
+    return;
+  }
+  const int x = blockIdx.x & 7;
+  const int per = (b.total_tiles + 7) >> 3;
+  const int begin = x * per, end = min((x + 1) * per, b.total_tiles);
+  if constexpr (!QUEUE) {
+    const int t = begin + (blockIdx.x >> 3);
+    if (t < end) batch_tile<P, ORDER, VEL>(b, t);
+  } else {
+    // every thread of the block reaches each barrier: the claims are the block's
+    __shared__ int s_next;
+    const bool lead = threadIdx.x == 0 && threadIdx.y == 0;
+    int *ctr = b.queue + x, *done = b.queue + 8 + x;
+    if (lead) s_next = atomicAdd(ctr, 1);
+    __syncthreads();
+    int t = begin + s_next;
+    while (t < end) {
+      __syncthreads();  // every thread has read s_next
+      if (lead) s_next = atomicAdd(ctr, 1);
+      batch_tile<P, ORDER, VEL>(b, t);
+      __syncthreads();  // the next claim is in s_next
+      t = begin + s_next;
+    }
+    if (lead && atomicAdd(done, 1) == (b.tile_blocks >> 3) - 1) {
+      atomicExch(ctr, 0);
+      atomicExch(done, 0);
+    }
+  }
+}
+
+template <class P>
+__global__ void k_source(const SourceArgs sa)
+{
+  source_cell<P>(sa, sa.it);
+}
+
 template <class P>
 __global__ void k_record(const RecordArgs ra)
 {
-  record_one<P>(ra, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, (int)blockIdx.y, ra.it);
+  record_block<P>(ra, blockIdx.x, ra.c0, ra.c1, ra.it);
 }
 
 // Batched source / record: one block (z) per shot; the step index comes from a device
-// counter that k_advance moves on, so a captured sequence of steps can be replayed.
+// counter, so a captured sequence of steps can be replayed.
 template <class P>
-__global__ void k_source_batch(const SourceArgs *tab, const int *itp)
+__global__ void k_source_batch(const SourceArgs *tab, const int *itp, int off)
 {
   const SourceArgs &sa = tab[blockIdx.x];
-  const int it = *itp;
+  const int it = *itp + off;
   if (!sa.wavelet || it >= sa.nt_w) return;
   source_cell<P>(sa, it);
 }
 template <class P>
-__global__ void k_record_batch(const RecordArgs *tab, const int *itp)
+__global__ void k_record_batch(const RecordArgs *tab, bool vel, const int *itp, int off)
 {
   const RecordArgs &ra = tab[blockIdx.z];
-  const int it = *itp;
+  const int it = *itp + off;
   if (!ra.traces || it >= ra.nt_max) return;
-  record_one<P>(ra, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, (int)blockIdx.y, it);
+  record_block<P>(ra, blockIdx.x, vel ? 0 : ra.nvel, ra.ncomp, it);
 }
-__global__ void k_advance(int *itp)
+__global__ void k_advance(int *itp, int d)
 {
-  if (threadIdx.x == 0) atomicAdd(itp, 1);
+  if (threadIdx.x == 0) atomicAdd(itp, d);
 }
-__global__ void k_set_counter(int *itp, int v)
+__global__ void k_set_counter(int *itp, int v, int end)
 {
-  if (threadIdx.x == 0) atomicExch(itp, v);
+  if (threadIdx.x == 0) itp[0] = v, itp[1] = end, itp[2] = v;
 }
 
 // In-place multiply of an FP16M tau or p field (lo: its tagged residual pointer).
@@ -1126,7 +1192,8 @@ __global__ void k_rescale4(S *p, int64_t nrec, double f0, double f1, double f2, 
 }
 
 template <class P, int ORDER, bool VEL>
-hipError_t launch_step(const StepArgs &in, LaunchShape sh, hipStream_t s)
+hipError_t launch_step(const StepArgs &in, LaunchShape sh, hipStream_t s, const RecordArgs *rec,
+                       const SourceArgs *src)
 {
   StepArgs a = in;
   const int h = ORDER / 2;
@@ -1135,48 +1202,61 @@ hipError_t launch_step(const StepArgs &in, LaunchShape sh, hipStream_t s)
   if (sh.zchunk <= 0) return hipErrorInvalidValue;
   set_tiles(a, sh, h);
   dim3 block(sh.bx, sh.by, 1);
-  dim3 grid((unsigned)(((a.ntiles + 7) / 8) * 8));
+  FuseArgs u{};
+  u.tile_blocks = ((a.ntiles + 7) / 8) * 8;
+  u.record = rec && rec->nrec > 0 && rec->c1 > rec->c0;
+  u.source = src != nullptr;
+  if (u.record) u.rec = *rec;
+  if (u.source) u.src = *src;
+  const int64_t rb = u.record ? (rec->nrec + sh.bx * sh.by - 1) / (sh.bx * sh.by) : 0;
+  dim3 grid((unsigned)(u.tile_blocks + rb));
   if (VEL)
-    hipLaunchKernelGGL((k_velocity<P, ORDER>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((k_velocity<P, ORDER>), grid, block, 0, s, a, u);
   else
-    hipLaunchKernelGGL((k_stress<P, ORDER>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((k_stress<P, ORDER>), grid, block, 0, s, a, u);
   return hipGetLastError();
 }
 
 template <bool VEL, int ORDER>
-hipError_t dispatch_order(int prec, const StepArgs &a, LaunchShape sh, hipStream_t s)
+hipError_t dispatch_order(int prec, const StepArgs &a, LaunchShape sh, hipStream_t s, const RecordArgs *rec,
+                          const SourceArgs *src)
 {
   switch (prec) {
-    case PREC_FP32: return launch_step<P32, ORDER, VEL>(a, sh, s);
-    case PREC_FP16: return launch_step<P16, ORDER, VEL>(a, sh, s);
-    case PREC_FP16C: return launch_step<P16C, ORDER, VEL>(a, sh, s);
-    case PREC_FP16T: return launch_step<P16T, ORDER, VEL>(a, sh, s);
-    case PREC_FP16M: return launch_step<P16M, ORDER, VEL>(a, sh, s);
-    case PREC_FP64: return launch_step<P64, ORDER, VEL>(a, sh, s);
+    case PREC_FP32: return launch_step<P32, ORDER, VEL>(a, sh, s, rec, src);
+    case PREC_FP16: return launch_step<P16, ORDER, VEL>(a, sh, s, rec, src);
+    case PREC_FP16C: return launch_step<P16C, ORDER, VEL>(a, sh, s, rec, src);
+    case PREC_FP16T: return launch_step<P16T, ORDER, VEL>(a, sh, s, rec, src);
+    case PREC_FP16M: return launch_step<P16M, ORDER, VEL>(a, sh, s, rec, src);
+    case PREC_FP64: return launch_step<P64, ORDER, VEL>(a, sh, s, rec, src);
   }
   return hipErrorInvalidValue;
 }
 
 template <bool VEL>
-hipError_t dispatch(int prec, int order, const StepArgs &a, LaunchShape sh, hipStream_t s)
+hipError_t dispatch(int prec, int order, const StepArgs &a, LaunchShape sh, hipStream_t s,
+                    const RecordArgs *rec, const SourceArgs *src)
 {
   if (sh.bx * sh.by > 256 || sh.bx <= 0 || sh.by <= 0) return hipErrorInvalidValue;
-  if (order == 2) return dispatch_order<VEL, 2>(prec, a, sh, s);
-  if (order == 4) return dispatch_order<VEL, 4>(prec, a, sh, s);
+  if (order == 2) return dispatch_order<VEL, 2>(prec, a, sh, s, rec, src);
+  if (order == 4) return dispatch_order<VEL, 4>(prec, a, sh, s, rec, src);
   return hipErrorInvalidValue;
 }
 
 }  // namespace
 
-hipError_t launch_step_batch(int prec, int order, bool vel, const BatchArgs &b, LaunchShape sh,
-                             int blocks, hipStream_t s)
+hipError_t launch_step_batch(int prec, int order, bool vel, const BatchArgs &in, LaunchShape sh,
+                             int blocks, int64_t max_nrec, hipStream_t s)
 {
   if (sh.bx * sh.by > 256 || sh.bx <= 0 || sh.by <= 0 || blocks <= 0 || blocks % 8) return hipErrorInvalidValue;
-  if (b.total_tiles <= 0) return hipSuccess;
-  dim3 grid((unsigned)blocks), block(sh.bx, sh.by, 1);
+  BatchArgs b = in;
+  b.tile_blocks = blocks;
+  b.rec_blocks = (int)((max_nrec + sh.bx * sh.by - 1) / (sh.bx * sh.by));
+  dim3 grid((unsigned)(blocks + b.rec_blocks * b.nshots)), block(sh.bx, sh.by, 1);
 #define BIOT_BATCH_CASE(PP, OO)                                                                 \
-  if (vel) hipLaunchKernelGGL((k_step_batch<PP, OO, true>), grid, block, 0, s, b);              \
-  else hipLaunchKernelGGL((k_step_batch<PP, OO, false>), grid, block, 0, s, b);
+  if (vel && b.queue) hipLaunchKernelGGL((k_step_batch<PP, OO, true, true>), grid, block, 0, s, b);   \
+  else if (vel) hipLaunchKernelGGL((k_step_batch<PP, OO, true, false>), grid, block, 0, s, b);  \
+  else if (b.queue) hipLaunchKernelGGL((k_step_batch<PP, OO, false, true>), grid, block, 0, s, b);    \
+  else hipLaunchKernelGGL((k_step_batch<PP, OO, false, false>), grid, block, 0, s, b);
   if (order != 2 && order != 4) return hipErrorInvalidValue;
   switch (prec) {
     case PREC_FP32:
@@ -1203,57 +1283,59 @@ hipError_t launch_step_batch(int prec, int order, bool vel, const BatchArgs &b, 
   return hipGetLastError();
 }
 
-hipError_t launch_source_batch(int prec, const SourceArgs *tab, int nshots, const int *it, hipStream_t s)
+hipError_t launch_source_batch(int prec, const SourceArgs *tab, int nshots, const int *it, int off, hipStream_t s)
 {
   if (nshots <= 0) return hipSuccess;
   switch (prec) {
-    case PREC_FP32: hipLaunchKernelGGL(k_source_batch<P32>, dim3(nshots), dim3(64), 0, s, tab, it); break;
-    case PREC_FP16: hipLaunchKernelGGL(k_source_batch<P16>, dim3(nshots), dim3(64), 0, s, tab, it); break;
-    case PREC_FP16C: hipLaunchKernelGGL(k_source_batch<P16C>, dim3(nshots), dim3(64), 0, s, tab, it); break;
-    case PREC_FP16T: hipLaunchKernelGGL(k_source_batch<P16T>, dim3(nshots), dim3(64), 0, s, tab, it); break;
-    case PREC_FP16M: hipLaunchKernelGGL(k_source_batch<P16M>, dim3(nshots), dim3(64), 0, s, tab, it); break;
-    case PREC_FP64: hipLaunchKernelGGL(k_source_batch<P64>, dim3(nshots), dim3(64), 0, s, tab, it); break;
+    case PREC_FP32: hipLaunchKernelGGL(k_source_batch<P32>, dim3(nshots), dim3(64), 0, s, tab, it, off); break;
+    case PREC_FP16: hipLaunchKernelGGL(k_source_batch<P16>, dim3(nshots), dim3(64), 0, s, tab, it, off); break;
+    case PREC_FP16C: hipLaunchKernelGGL(k_source_batch<P16C>, dim3(nshots), dim3(64), 0, s, tab, it, off); break;
+    case PREC_FP16T: hipLaunchKernelGGL(k_source_batch<P16T>, dim3(nshots), dim3(64), 0, s, tab, it, off); break;
+    case PREC_FP16M: hipLaunchKernelGGL(k_source_batch<P16M>, dim3(nshots), dim3(64), 0, s, tab, it, off); break;
+    case PREC_FP64: hipLaunchKernelGGL(k_source_batch<P64>, dim3(nshots), dim3(64), 0, s, tab, it, off); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
 
 hipError_t launch_record_batch(int prec, const RecordArgs *tab, int nshots, int64_t max_nrec,
-                               int max_ncomp, const int *it, hipStream_t s)
+                               bool vel, const int *it, int off, hipStream_t s)
 {
-  if (nshots <= 0 || max_nrec <= 0 || max_ncomp <= 0) return hipSuccess;
-  dim3 grid((unsigned)((max_nrec + 255) / 256), (unsigned)max_ncomp, (unsigned)nshots), block(256);
+  if (nshots <= 0 || max_nrec <= 0) return hipSuccess;
+  dim3 grid((unsigned)((max_nrec + 255) / 256), 1u, (unsigned)nshots), block(256);
   switch (prec) {
-    case PREC_FP32: hipLaunchKernelGGL(k_record_batch<P32>, grid, block, 0, s, tab, it); break;
-    case PREC_FP16: hipLaunchKernelGGL(k_record_batch<P16>, grid, block, 0, s, tab, it); break;
-    case PREC_FP16C: hipLaunchKernelGGL(k_record_batch<P16C>, grid, block, 0, s, tab, it); break;
-    case PREC_FP16T: hipLaunchKernelGGL(k_record_batch<P16T>, grid, block, 0, s, tab, it); break;
-    case PREC_FP16M: hipLaunchKernelGGL(k_record_batch<P16M>, grid, block, 0, s, tab, it); break;
-    case PREC_FP64: hipLaunchKernelGGL(k_record_batch<P64>, grid, block, 0, s, tab, it); break;
+    case PREC_FP32: hipLaunchKernelGGL(k_record_batch<P32>, grid, block, 0, s, tab, vel, it, off); break;
+    case PREC_FP16: hipLaunchKernelGGL(k_record_batch<P16>, grid, block, 0, s, tab, vel, it, off); break;
+    case PREC_FP16C: hipLaunchKernelGGL(k_record_batch<P16C>, grid, block, 0, s, tab, vel, it, off); break;
+    case PREC_FP16T: hipLaunchKernelGGL(k_record_batch<P16T>, grid, block, 0, s, tab, vel, it, off); break;
+    case PREC_FP16M: hipLaunchKernelGGL(k_record_batch<P16M>, grid, block, 0, s, tab, vel, it, off); break;
+    case PREC_FP64: hipLaunchKernelGGL(k_record_batch<P64>, grid, block, 0, s, tab, vel, it, off); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
 
-hipError_t launch_advance(int *it, hipStream_t s)
+hipError_t launch_advance(int *it, int d, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, s, it);
+  hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, s, it, d);
   return hipGetLastError();
 }
 
-hipError_t launch_set_counter(int *it, int v, hipStream_t s)
+hipError_t launch_set_counter(int *it, int v, int end, hipStream_t s)
 {
-  hipLaunchKernelGGL(k_set_counter, dim3(1), dim3(64), 0, s, it, v);
+  hipLaunchKernelGGL(k_set_counter, dim3(1), dim3(64), 0, s, it, v, end);
   return hipGetLastError();
 }
 
-hipError_t launch_velocity(int prec, int order, const StepArgs &args, LaunchShape sh, hipStream_t s)
+hipError_t launch_velocity(int prec, int order, const StepArgs &args, LaunchShape sh, hipStream_t s,
+                           const RecordArgs *rec)
 {
-  return dispatch<true>(prec, order, args, sh, s);
+  return dispatch<true>(prec, order, args, sh, s, rec, nullptr);
 }
-hipError_t launch_stress(int prec, int order, const StepArgs &args, LaunchShape sh, hipStream_t s)
+hipError_t launch_stress(int prec, int order, const StepArgs &args, LaunchShape sh, hipStream_t s,
+                         const RecordArgs *rec, const SourceArgs *src)
 {
-  return dispatch<false>(prec, order, args, sh, s);
+  return dispatch<false>(prec, order, args, sh, s, rec, src);
 }
 
 hipError_t launch_source(int prec, const SourceArgs &a, hipStream_t s)
@@ -1367,8 +1449,8 @@ hipError_t launch_rescale4(int prec, void *p, int64_t nrec, const double f[4], h
 
 hipError_t launch_record(int prec, const RecordArgs &a, hipStream_t s)
 {
-  if (a.nrec <= 0 || a.ncomp <= 0) return hipSuccess;
-  dim3 block(256), grid((unsigned)((a.nrec + 255) / 256), (unsigned)a.ncomp);
+  if (a.nrec <= 0 || a.c1 <= a.c0) return hipSuccess;
+  dim3 block(256), grid((unsigned)((a.nrec + 255) / 256));
   switch (prec) {
     case PREC_FP32: hipLaunchKernelGGL(k_record<P32>, grid, block, 0, s, a); break;
     case PREC_FP16: hipLaunchKernelGGL(k_record<P16>, grid, block, 0, s, a); break;
