@@ -902,8 +902,20 @@ __device__ __forceinline__ void source_field(const SA &sa, int f, int it)
   using A = typename P::A;
   const u32 c = (u32)sa.cell;
   const bool cf = (P::cmask >> f) & 1u;
-  const A amp = (A)sa.wavelet[it] * (A)sa.inv_scale[f];
-  store_raw<P>(sa.f[f], sa.lo[f], cf, c, load_raw<P>(sa.f[f], sa.lo[f], cf, c) + amp);
+  const A w = (A)sa.wavelet[it], inv = (A)sa.inv_scale[f];
+  const A old = load_raw<P>(sa.f[f], sa.lo[f], cf, c);
+  // one rounding or two, written out, so that the value does not depend on which launch adds it
+  A x;
+  if constexpr (P::comp && !P::packed) {
+#pragma clang fp contract(off)
+    const A amp = w * inv;
+    x = old + amp;
+  } else if constexpr (std::is_same<A, double>::value) {
+    x = fma(w, inv, old);
+  } else {
+    x = fmaf(w, inv, old);
+  }
+  store_raw<P>(sa.f[f], sa.lo[f], cf, c, x);
 }
 // one lane per field
 template <class P>
@@ -918,6 +930,7 @@ __device__ __forceinline__ void source_cell(const SourceArgs &sa, int it)
 template <class P, class SA>
 __device__ __forceinline__ void source_owner(const SA &sa, int it)
 {
+#pragma unroll 1
   for (int f = 0; f < NFIELD; ++f)
     if (sa.mask & (1u << f)) source_field<P>(sa, f, it);
 }
