@@ -287,6 +287,7 @@ biot_handle::~biot_handle()
   if (d_coef) (void)hipFree(d_coef);
   if (d_kpack) (void)hipFree(d_kpack);
   if (d_flag) (void)hipFree(d_flag);
+  if (h_slice) (void)hipHostFree(h_slice);
   for (auto *p : d_carry)
     if (p) (void)hipFree(p);
   for (auto &ax : d_prof)

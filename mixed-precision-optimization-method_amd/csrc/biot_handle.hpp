@@ -26,6 +26,7 @@ struct biot_handle {
   void *d_coef = nullptr;            // 22 * n (FP16M: the medium records, 18 bytes per cell)
   void *d_kpack = nullptr;           // the coefficients packed per cell (velocity, then stress block)
   void *d_carry[3] = {nullptr, nullptr, nullptr};
+  float *h_slice = nullptr;          // pinned, nx * nz: the slice of biot_snapshot_xz (made on first use)
   int *d_flag = nullptr;             // first step with a non-finite receiver sample
                                      // (biot::NONFINITE_NONE: none since the last clear)
   void *d_prof[3][4] = {};           // e_int, a_int, e_half, a_half per axis
