@@ -718,7 +718,7 @@ std::string tune_key(const biot_handle *h)
   for (auto &ch : arch)
     if (ch == ' ') ch = '_';
   char buf[256];
-  snprintf(buf, sizeof buf, "v4 %s p%d o%d %dx%dx%d", arch.c_str(), h->prec, h->g.order, h->g.nx,
+  snprintf(buf, sizeof buf, "v5 %s p%d o%d %dx%dx%d", arch.c_str(), h->prec, h->g.order, h->g.nx,
            h->g.ny, h->g.nz);
   return buf;
 }

@@ -122,6 +122,7 @@ struct StepArgs {
   int64_t sy, sz;            // strides
   int zchunk;
   int gx, gy, gz, ntiles;    // tile grid (x-y tiles of the block shape, z chunks)
+  int xg;                    // consecutive tiles an XCD takes at a time (xcd_run)
   int src[3];                // the source cell (no cell's position: no source)
   int xy0;                   // one-row blocks: the plane cell the first tile starts at
   uint32_t nx_rcp;           // ceil(2^32 / nx)
@@ -136,6 +137,26 @@ inline size_t carry_bytes(int prec) { return prec == PREC_FP64 ? 8 : prec == PRE
 struct LaunchShape {
   int bx, by, zchunk;
 };
+// Workgroup b of a 1-D grid goes to XCD b % 8.  Each XCD takes runs of g consecutive tiles, run
+// after run dealt out to the eight in turn, so that the rows neighbouring tiles both read meet in
+// one L2 while all XCDs work in the same planes of every array: with one contiguous eighth of the
+// tiles each, they streamed from eight places of each of the 30-odd arrays at once.  256^3 FP32,
+// velocity + stress, 256-cell tiles of 4 planes: eighths 934 us, runs of 1 tile 886, of 4, 8, 16 and
+// 32 tiles 859-862 (8 at 2 planes: 843), of 64 862, of 256 886; 512x512x384 FP32 5.54 ms in eighths,
+// 4.88 in runs of 8, FP16M at 16 planes 3.04 and 2.83 ms.  A run is 2048 cells; with few tiles it is
+// shorter, for eight runs an XCD.  Grids whose arrays about fit the eight L2s (half a million
+// cells) keep contiguous eighths, whose rows meet in one L2 from step to step (64^3 FP32, 200 steps:
+// 4.2 ms, in runs 4.5 ms).
+inline int xcd_run(int64_t ntiles, int threads, int64_t cells)
+{
+  if (cells <= (int64_t)1 << 19) return (int)((ntiles + 7) / 8 > 0 ? (ntiles + 7) / 8 : 1);
+  const int64_t g = ntiles / 64, most = 2048 / threads;
+  return (int)(g < 1 ? 1 : g > most ? most : g);
+}
+// the slots of one XCD for n tiles in runs of g: local slot m of XCD x is tile xcd_tile(x, m, g)
+// (those past n are empty)
+inline int64_t xcd_slots(int64_t n, int g) { return (n + 8 * (int64_t)g - 1) / (8 * (int64_t)g) * g; }
+__host__ __device__ inline int xcd_tile(int x, int m, int g) { return (m / g * 8 + x) * g + m % g; }
 // the tile grid of shape sh over the update box (h cells off every face): rectangles of bx x by
 // cells, or for by = 1 runs of bx consecutive cells of the x-y plane, the first starting on a
 // 64-cell boundary of the plane
@@ -153,6 +174,7 @@ inline void set_tiles(StepArgs &a, LaunchShape sh, int h)
   }
   a.gz = (a.nz - 2 * h + a.zchunk - 1) / a.zchunk;
   a.ntiles = a.gx * a.gy * a.gz;
+  a.xg = xcd_run(a.ntiles, sh.bx * sh.by, (int64_t)a.nx * a.ny * a.nz);
 }
 
 struct SourceArgs {
@@ -235,6 +257,7 @@ struct BatchArgs {
   const StepArgs *shots;    // device, one per shot (gx, gy, gz, zchunk set for the shape)
   const int *tile_start;    // device, nshots + 1 prefix sums of the shots' tile counts
   int nshots, total_tiles;
+  int xg;                   // consecutive tiles an XCD takes at a time (xcd_run; set by the launcher)
   int *queue;               // device, 16 ints (zero between launches): per XCD group the tile
                             // counter and the count of finished blocks; null: one block per tile
   // the work around the half step, as FuseArgs per shot: step it[0] + off, the sources of steps

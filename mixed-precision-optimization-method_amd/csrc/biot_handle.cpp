@@ -358,22 +358,24 @@ void biot_handle::fill_args(StepArgs &a) const
 }
 
 // The tile shape without the autotuner, from the number of waves one z plane a thread would make
-// (64 consecutive cells of an x-y plane each).  Small grids need one or two planes a thread: their
-// waves are all resident at once, so a longer march only makes the launch a longer chain of
-// memory round trips (64^3 FP32, velocity + stress: 24 us at 1 plane, 61 us at 16; 45x38x53 order
-// 2: 15 us, 51 us).  With more waves than fit (about 3000 at 130 VGPRs) a longer march saves the
-// re-read z halo: 3 planes from 24 k waves on (157x131x173 FP16T 143 us, 176 us at 16; 128^3 FP32
-// 110 us, 119 us at 16), 4 (8 for 16-bit fields) from 128 k (256^3 FP32 852 us, 873 us at 16) and
-// 16 from 1 M (512x512x384 FP16M 2.77 ms, 2.97 ms at 4; FP32 5.09 ms, 5.22 ms at 4).  Four waves
-// of one block share the L1 rows of the y differences; below 16 k waves single-wave blocks spread
-// better (99x110x83 FP64 103 us against 106 us; 128^3 114 us against 110 us).
+// (64 consecutive cells of an x-y plane each).  Small grids need one plane a thread: their waves
+// are all resident at once, so a longer march only makes the launch a longer chain of memory round
+// trips (64^3 FP32, velocity + stress: 24-25 us at 1 and 2 planes, 61 us at 16; 45x38x53 order 2: 17
+// us, 51 us).  With more waves than fit (about 3000 at 130 VGPRs) a longer march saves the re-read z
+// halo.  4- and 8-byte fields are best at 2 planes whatever their size (128^3 FP32 108 us, 121 us at
+// 16; 512x512x384 4.46 ms, 4.57 ms at 16), 16-bit fields, whose kernels issue more instructions a
+// byte, at more planes the larger they are (96x80x89 FP16M 34 us at 2; 157x131x173 FP16T 143 us at 2
+// and 3, 176 at 16; 192x192x160 FP16 144 us at 4, 151 at 2; 512x512x384 FP16M 2.67 ms at 16, 2.75 at
+// 4).  Four waves of one block share the L1 rows of the y differences; below 16 k waves single-wave
+// blocks spread better (99x110x83 FP64 102 us against 104 us; 128^3 FP32 115 us against 108 us).
 LaunchShape default_shape(int prec, int64_t plane_waves)
 {
+  const bool narrow = field_bytes(prec) == 2;
   int zc = 1;
   if (plane_waves > 4096) zc = 2;
-  if (plane_waves > 24576) zc = 3;
-  if (plane_waves > 131072) zc = field_bytes(prec) == 2 ? 8 : 4;
-  if (plane_waves > 1048576) zc = 16;
+  if (narrow && plane_waves > 24576) zc = 3;
+  if (narrow && plane_waves > 65536) zc = 4;
+  if (narrow && plane_waves > 1048576) zc = 16;
   return LaunchShape{plane_waves > 16384 ? 256 : 64, 1, zc};
 }
 int64_t plane_waves(const biot_grid &g)

@@ -467,16 +467,11 @@ __device__ __forceinline__ int slab_pos(int i, int n, int Lw, int Rw)
   return -1;
 }
 
-// XCD-aware tile assignment.  The dispatcher hands workgroup b of a 1-D grid to XCD
-// b % 8 in order; each XCD here gets one contiguous range of tiles, x fastest then y then
-// z, so the y- and z-adjacent tiles whose halos overlap are processed by the same XCD,
-// close in time, and the halo re-reads hit that XCD's L2.
+// the workgroup's tile, x fastest then y then z, dealt out to the XCDs in runs (xcd_run)
 template <class AT>
 __device__ __forceinline__ bool tile_of(const AT &a, int &tx, int &ty, int &tz)
 {
-  const int b = blockIdx.x;
-  const int per = (a.ntiles + 7) >> 3;
-  const int t = (b & 7) * per + (b >> 3);
+  const int t = xcd_tile(blockIdx.x & 7, blockIdx.x >> 3, a.xg);
   if (t >= a.ntiles) return false;
   tx = t % a.gx;
   const int r = t / a.gx;
@@ -1006,8 +1001,8 @@ __global__ void __launch_bounds__(256) k_stress(const StepArgs a, const FuseArgs
 }
 
 // Batched forms: one launch covers the tiles of every shot.  The shots' tile lists are
-// concatenated (tile_start[s] = first global tile of shot s); each XCD takes one contiguous range
-// of that list, so a shot's neighbouring tiles share an L2.  The argument tables are read-only for
+// concatenated (tile_start[s] = first global tile of shot s) and dealt out to the XCDs in runs, as
+// a single grid's.  The argument tables are read-only for
 // a launch and indexed uniformly per block: read them through the constant address space, so the
 // compiler keeps them in scalar registers (as it does kernel arguments) instead of a VGPR pair per
 // pointer.
@@ -1040,8 +1035,7 @@ __device__ __forceinline__ void batch_tile(const BatchArgs &b, int t)
     if (b1.src && sa.wavelet && it < sa.nt_w && it < ((CInt *)b1.it)[1]) source_owner<P>(sa, it);
   }
 }
-// QUEUE false: one block per tile, workgroup b on XCD b % 8, XCD group x owning the contiguous tile
-// range [begin, end).  QUEUE: a smaller grid whose blocks take their group's next tile from the
+// QUEUE false: one block per tile slot of its XCD (workgroup b on XCD b % 8).  QUEUE: a smaller grid whose blocks take their group's next tile from the
 // group's counter (one atomic a tile, the next one claimed while the current one runs), so blocks
 // that drew cheap tiles take more.  Every block ends on one claim past the range; the last block
 // of the group to make it sets the group's two counters back to zero for the next launch (no
@@ -1061,11 +1055,9 @@ __global__ void __launch_bounds__(256) k_step_batch(const BatchArgs b)
     return;
   }
   const int x = blockIdx.x & 7;
-  const int per = (b.total_tiles + 7) >> 3;
-  const int begin = x * per, end = min((x + 1) * per, b.total_tiles);
   if constexpr (!QUEUE) {
-    const int t = begin + (blockIdx.x >> 3);
-    if (t < end) batch_tile<P, ORDER, VEL>(b, t);
+    const int t = xcd_tile(x, blockIdx.x >> 3, b.xg);
+    if (t < b.total_tiles) batch_tile<P, ORDER, VEL>(b, t);
   } else {
     // every thread of the block reaches each barrier: the claims are the block's
     __shared__ int s_next;
@@ -1073,13 +1065,14 @@ __global__ void __launch_bounds__(256) k_step_batch(const BatchArgs b)
     int *ctr = b.queue + x, *done = b.queue + 8 + x;
     if (lead) s_next = atomicAdd(ctr, 1);
     __syncthreads();
-    int t = begin + s_next;
-    while (t < end) {
+    // a group's slots ascend in tiles, so its first slot past the list is its end
+    int t = xcd_tile(x, s_next, b.xg);
+    while (t < b.total_tiles) {
       __syncthreads();  // every thread has read s_next
       if (lead) s_next = atomicAdd(ctr, 1);
       batch_tile<P, ORDER, VEL>(b, t);
       __syncthreads();  // the next claim is in s_next
-      t = begin + s_next;
+      t = xcd_tile(x, s_next, b.xg);
     }
     if (lead && atomicAdd(done, 1) == (b.tile_blocks >> 3) - 1) {
       atomicExch(ctr, 0);
@@ -1216,7 +1209,7 @@ hipError_t launch_step(const StepArgs &in, LaunchShape sh, hipStream_t s, const 
   set_tiles(a, sh, h);
   dim3 block(sh.bx, sh.by, 1);
   FuseArgs u{};
-  u.tile_blocks = ((a.ntiles + 7) / 8) * 8;
+  u.tile_blocks = (int)(8 * xcd_slots(a.ntiles, a.xg));
   u.record = rec && rec->nrec > 0 && rec->c1 > rec->c0;
   u.source = src != nullptr;
   if (u.record) u.rec = *rec;
@@ -1262,9 +1255,10 @@ hipError_t launch_step_batch(int prec, int order, bool vel, const BatchArgs &in,
 {
   if (sh.bx * sh.by > 256 || sh.bx <= 0 || sh.by <= 0 || blocks <= 0 || blocks % 8) return hipErrorInvalidValue;
   BatchArgs b = in;
-  b.tile_blocks = blocks;
+  b.xg = xcd_run(b.total_tiles, sh.bx * sh.by, (int64_t)b.total_tiles * sh.bx * sh.by * sh.zchunk);
+  b.tile_blocks = b.queue ? blocks : (int)(8 * xcd_slots(b.total_tiles, b.xg));
   b.rec_blocks = (int)((max_nrec + sh.bx * sh.by - 1) / (sh.bx * sh.by));
-  dim3 grid((unsigned)(blocks + b.rec_blocks * b.nshots)), block(sh.bx, sh.by, 1);
+  dim3 grid((unsigned)(b.tile_blocks + b.rec_blocks * b.nshots)), block(sh.bx, sh.by, 1);
 #define BIOT_BATCH_CASE(PP, OO)                                                                 \
   if (vel && b.queue) hipLaunchKernelGGL((k_step_batch<PP, OO, true, true>), grid, block, 0, s, b);   \
   else if (vel) hipLaunchKernelGGL((k_step_batch<PP, OO, true, false>), grid, block, 0, s, b);  \
