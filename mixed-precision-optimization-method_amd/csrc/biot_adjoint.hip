@@ -6,8 +6,8 @@
 //                       q' = W1 q - W2 sum D' - W3 D's;  v' = v + U1 sum D' - U2 (q' - q)
 //   stress half step    E = delta(v', q'); E' = (1+a) E + c_T; c_T <- e (c_T + 2 a E)
 //                       p' = p - P1 div_u' - P2 div_w';  tau' = tau + S1 .. + S2 .. + S3 div_w'
-// (the folded C-PML carry, kernel.cu:188-196 algebraically).  Its transpose, applied
-// backward, is split into two passes per half step:
+// (the folded C-PML carry, kernel.cu:188-196 algebraically).  Its transpose, applied backward, has
+// two parts per half step:
 //   local  : adjoints of the twelve post-PML derivatives from the adjoint state at the cell,
 //            C-PML carry adjoints  lambda_E = (1+a) lambda_E' + 2 a e lambda_c,
 //            lambda_c <- lambda_E' + e lambda_c, the cell-local field adjoints, and the FP64
@@ -15,6 +15,18 @@
 //            forward derivatives recomputed from the stored states;
 //   gather : lambda_f(c) += sum_m w_m G(c - o_m), the transposed staggered differences,
 //            written per cell so the result is deterministic (no atomics).
+// A gather ends with the cell's new adjoint values, which are all that the next local part reads
+// of them, so a backward step is two passes: the gather of step n+1's velocity half with the local
+// part of step n's stress half (adj_stress), then the gather of that with the local part of step
+// n's velocity half (adj_velocity).
+// The derivative adjoints G between the passes: outside the absorbing slabs G is lambda_E', of
+// which the stress half has 7 different ones and the velocity half 6, kept as full arrays; the
+// derivatives along an axis whose slab the cell lies in are four records of G, laid out as the
+// carries are.
+// The passes are bound by their bytes: 137 values a cell and step (FP32: 548 B) and 144 B a slab
+// membership, where four passes with twelve full arrays of G moved 175 and 96 B.  Per step, before and
+// now: 128^3 FP32 343 and 325 us (about 4.1 TB/s), 192^3 1198 and 1018 us, 128^3 FP64 721 and 665, 90^3
+// FP16M 236 and 107, 128^3 FP16T 687 and 320.
 // With 16-bit storage everything runs in storage units (fields divided by their scales,
 // coefficients as the kernels apply them); the host converts dJ/dK with the per-array factor.
 #include <hip/hip_runtime.h>
@@ -40,19 +52,29 @@ __device__ __forceinline__ const T &at(const void *base, u32 idx)
   return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + idx * (u32)sizeof(T));
 }
 
-// derivative tables: field, direction (= damped axis), forward(1)/backward(0) difference,
-// carry slot on that axis, half-node (1) / integer-node (0) profile
-struct Der {
-  int field, dir, fwd, slot, half;
-};
-// velocity half step: x1 x2 x3 s1 y1 y2 y3 s2 z1 z2 z3 s3 (kernel.cu:172-185, 188-216)
-__constant__ Der VDER[12] = {{6, 0, 1, 0, 1},  {9, 1, 0, 0, 0},  {10, 2, 0, 0, 0}, {12, 0, 1, 1, 1},
-                             {7, 1, 1, 1, 1},  {9, 0, 0, 2, 0},  {11, 2, 0, 1, 0}, {12, 1, 1, 2, 1},
-                             {8, 2, 1, 2, 1},  {10, 0, 0, 3, 0}, {11, 1, 0, 3, 0}, {12, 2, 1, 3, 1}};
-// stress half step: uxx uyy uzz wx wy wz uxy uyx uxz uzx uyz uzy (kernel.cu:430-482)
-__constant__ Der TDER[12] = {{0, 0, 0, 4, 0}, {1, 1, 0, 4, 0}, {2, 2, 0, 4, 0}, {3, 0, 0, 5, 0},
-                             {4, 1, 0, 5, 0}, {5, 2, 0, 5, 0}, {0, 1, 1, 6, 1}, {1, 0, 1, 6, 1},
-                             {0, 2, 1, 6, 1}, {2, 0, 1, 7, 1}, {1, 2, 1, 7, 1}, {2, 1, 1, 7, 1}};
+// The twelve derivatives of a half step by axis and carry slot (kernel.cu:172-185, 188-216;
+// 430-482): the field they difference, and whether forward (on the half-node profile) or backward
+// (integer nodes).  Velocity half: x1 s1 y2 z2 | x2 y1 s2 z3 | x3 y3 z1 s3; stress half: uxx wx uyx
+// uzx | uyy wy uxy uzy | uzz wz uxz uyz.
+__device__ constexpr int der_field(bool vel, int ax, int m)
+{
+  constexpr int v[3][4] = {{6, 12, 9, 10}, {9, 7, 12, 11}, {10, 11, 8, 12}};
+  constexpr int t[3][4] = {{0, 3, 1, 2}, {1, 4, 0, 2}, {2, 5, 0, 1}};
+  return vel ? v[ax][m] : t[ax][m];
+}
+__device__ constexpr bool der_fwd(bool vel, int ax, int m)
+{
+  constexpr bool v[3][4] = {{true, true, false, false}, {false, true, true, false}, {false, false, true, true}};
+  return vel ? v[ax][m] : m >= 2;
+}
+// the full array (AdjArgs gv / gt) that holds the derivative's G outside its slab.  Velocity half:
+// the three S and the three Ds; stress half: uxx uyy uzz, div w, and the three shears xy xz yz.
+__device__ constexpr int der_base(bool vel, int ax, int m)
+{
+  constexpr int v[3][4] = {{0, 3, 1, 2}, {0, 1, 4, 2}, {0, 1, 2, 5}};
+  constexpr int t[3][4] = {{0, 3, 4, 5}, {1, 3, 4, 6}, {2, 3, 5, 6}};
+  return vel ? v[ax][m] : t[ax][m];
+}
 
 // storage type S -> arithmetic type A (also the C-PML carry type)
 template <typename S>
@@ -64,12 +86,16 @@ struct AdjT {
   static constexpr bool res = false;
   static constexpr bool pk = false;
 };
-// FP16T / FP16C states: binary16 fields and coefficients, an int8 residual on tau and p
-// (FP16C: also on v; value = h + r ulp(h)/256, as the forward kernels store it), float C-PML
-// carries
-struct H16R {};
-template <>
-struct AdjT<H16R> {
+// FP16T / FP16C states: binary16 fields and coefficients, an int8 residual on the fields of MASK
+// (FP16T tau and p, FP16C also v; value = h + r ulp(h)/256, as the forward kernels store it), float
+// C-PML carries.  The mask is part of the type: tested at run time it put a branch around each of
+// the 96 taps of a step (128^3 FP16T: 631 us a step, 292 without).
+template <uint32_t MASK>
+struct H16R {
+  static constexpr uint32_t mask = MASK;
+};
+template <uint32_t MASK>
+struct AdjT<H16R<MASK>> {
   using A = float;
   using C = float;
   using T = _Float16;
@@ -126,34 +152,31 @@ __device__ __forceinline__ const void *fw_carry(const AT &a, int q, int ax)
 {
   return a.slots + (uint64_t)q * a.sb + a.coff[ax];
 }
-// the residuals of field f in state q (FP16T tau and p, FP16C also v), or null; for FP16M
-// the state's record array (256-byte aligned) with the field's nibble in the low 3 bits
-template <typename S, class AT>
+// the residuals of field f in state q (FP16T, FP16C)
+template <class AT>
 __device__ __forceinline__ const int8_t *fw_lo(const AT &a, int q, int f)
 {
-  if (!a.loff || !((a.lomask >> f) & 1u)) return nullptr;
-  if constexpr (AdjT<S>::pk)
-    return reinterpret_cast<const int8_t *>(a.slots + (uint64_t)q * a.sb + a.loff + (uint64_t)pk_slot(f));
   return reinterpret_cast<const int8_t *>(a.slots + (uint64_t)q * a.sb + a.loff +
                                           (uint64_t)f * (uint64_t)a.nx * a.ny * a.nz);
 }
 
-template <typename S, int ORDER>
-__device__ __forceinline__ typename AdjT<S>::A diff(const void *f, const int8_t *lo, u32 c, u32 s, int fwd)
+// staggered difference of forward field f of state q at cell c, stride s (f and fwd fold to
+// constants).  FP16M: the residual record of a point is addressed from the one record array, so the
+// fields differenced there share its load.
+template <typename S, int ORDER, class AT>
+__device__ __forceinline__ typename AdjT<S>::A diff(const AT &a, int q, int f, u32 c, u32 s, bool fwd)
 {
   using A = typename AdjT<S>::A;
   using T = typename AdjT<S>::T;
+  const void *fp = fw_field(a, q, f);
   auto L = [&](u32 idx) {
-    const T h = at<T>(f, idx);
+    const T h = at<T>(fp, idx);
     if constexpr (AdjT<S>::res) {
-      if (lo) return (A)h + (A)lo[idx] * res_unit(h);
+      if ((S::mask >> f) & 1u) return (A)h + (A)fw_lo(a, q, f)[idx] * res_unit(h);
     }
     if constexpr (AdjT<S>::pk) {
-      if (lo) {
-        const uintptr_t t = reinterpret_cast<uintptr_t>(lo);
-        const int sl = (int)(t & 7u);
-        return (A)pk_join((float)h, pk_nib(at<u32>(reinterpret_cast<const void *>(t - sl), idx), sl));
-      }
+      if ((PK_FIELDS >> f) & 1u)
+        return (A)pk_join((float)h, pk_nib(at<u32>(a.slots + (uint64_t)q * a.sb + a.loff, idx), pk_slot(f)));
     }
     return (A)h;
   };
@@ -166,49 +189,90 @@ __device__ __forceinline__ typename AdjT<S>::A diff(const void *f, const int8_t 
   }
 }
 
-// transposed difference gathered at c from the derivative-adjoint array G
-template <typename A, int ORDER>
-__device__ __forceinline__ A diffT(const void *G, u32 c, u32 s, int fwd)
+template <int AX, class AT>
+__device__ __forceinline__ u32 stride(const AT &a)
 {
-  auto L = [&](u32 idx) { return at<A>(G, idx); };
-  if (fwd) {
-    if constexpr (ORDER == 2) return L(c - s) - L(c);
-    return A(9.0 / 8.0) * (L(c - s) - L(c)) + A(-1.0 / 24.0) * (L(c - 2 * s) - L(c + s));
+  return AX == 0 ? 1u : AX == 1 ? (u32)a.sy : (u32)a.sz;
+}
+// slab cell index on axis AX of the cell ci moved to position `pos` on that axis, or -1 outside
+// the slabs
+template <int AX, class AT>
+__device__ __forceinline__ int slab_cell(const AT &a, const CellIdx &ci, int pos)
+{
+  const int nn = AX == 0 ? a.nx : (AX == 1 ? a.ny : a.nz);
+  int p;
+  if (pos < a.L[AX]) p = pos;
+  else if (pos >= nn - a.R[AX]) p = a.L[AX] + pos - (nn - a.R[AX]);
+  else return -1;
+  const int w = a.L[AX] + a.R[AX];
+  if (AX == 0) return p + w * (ci.j + a.ny * ci.k);
+  if (AX == 1) return ci.i + a.nx * (p + w * ci.k);
+  return ci.i + a.nx * (ci.j + a.ny * p);
+}
+// the record of four values of slab cell o of group g (0: velocity half, 1: stress half) in an
+// array laid out as the carries are
+template <typename E>
+__device__ __forceinline__ void rec_load(E (&v)[4], const void *base, u32 g, u32 o, u32 sl)
+{
+  typedef E V4 __attribute__((ext_vector_type(4)));
+  const V4 r = *reinterpret_cast<const V4 *>(reinterpret_cast<const char *>(base) + (g * sl + o) * (u32)(4 * sizeof(E)));
+  v[0] = r.x, v[1] = r.y, v[2] = r.z, v[3] = r.w;
+}
+template <typename E>
+__device__ __forceinline__ void rec_store(const E (&v)[4], void *base, u32 g, u32 o, u32 sl)
+{
+  typedef E V4 __attribute__((ext_vector_type(4)));
+  V4 r;
+  r.x = v[0], r.y = v[1], r.z = v[2], r.w = v[3];
+  *reinterpret_cast<V4 *>(reinterpret_cast<char *>(base) + (g * sl + o) * (u32)(4 * sizeof(E))) = r;
+}
+
+// The transposed differences along axis AX of the four derivatives of a half step at cell ci:
+// out[m] from G at the cells -h..h along the axis, each from the full array outside the axis's
+// slabs and from the slab's record inside.  Away from the slabs (the whole stencil outside) there
+// is nothing to choose.
+template <typename A, int ORDER, bool VEL, int AX, class AT>
+__device__ __forceinline__ void gather_axis(const AT &a, const CellIdx &ci, A (&out)[4])
+{
+  constexpr int h = ORDER / 2;
+  const u32 s = stride<AX>(a);
+  const int pos = AX == 0 ? ci.i : (AX == 1 ? ci.j : ci.k);
+  const int nn = AX == 0 ? a.nx : (AX == 1 ? a.ny : a.nz);
+  A v[4][2 * h + 1];
+  auto base = [&](int m, int o) {
+    return at<A>(VEL ? a.gv[der_base(true, AX, m)] : a.gt[der_base(false, AX, m)], ci.c + (u32)o * s);
+  };
+  if (pos - h < a.L[AX] || pos + h >= nn - a.R[AX]) {
+#pragma unroll
+    for (int o = -h; o <= h; ++o) {
+      const int sc = slab_cell<AX>(a, ci, pos + o);
+      A r[4];
+      if (sc >= 0) {
+        rec_load(r, a.gs[AX], VEL ? 0u : 1u, (u32)sc, (u32)a.slab[AX]);
+      } else {
+#pragma unroll
+        for (int m = 0; m < 4; ++m) r[m] = base(m, o);
+      }
+#pragma unroll
+      for (int m = 0; m < 4; ++m) v[m][o + h] = r[m];
+    }
   } else {
-    if constexpr (ORDER == 2) return L(c) - L(c + s);
-    return A(9.0 / 8.0) * (L(c) - L(c + s)) + A(-1.0 / 24.0) * (L(c - s) - L(c + 2 * s));
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int o = -h; o <= h; ++o)
+        if (der_fwd(VEL, AX, m) ? o < h : o > -h) v[m][o + h] = base(m, o);
   }
-}
-
-__device__ __forceinline__ int slab_pos(int i, int n, int Lw, int Rw)
-{
-  if (i < Lw) return i;
-  if (i >= n - Rw) return Lw + i - (n - Rw);
-  return -1;
-}
-
-// carry element index of slot `slot` on axis `ax` at cell ci, or -1 outside that slab (records
-// of four carries per slab cell: slots 0..3, then 4..7)
-template <class AT>
-__device__ __forceinline__ long long carry_idx(const AT &a, int ax, int slot, const CellIdx &ci)
-{
-  const int pos = ax == 0 ? ci.i : (ax == 1 ? ci.j : ci.k);
-  const int nn = ax == 0 ? a.nx : (ax == 1 ? a.ny : a.nz);
-  const int p = slab_pos(pos, nn, a.L[ax], a.R[ax]);
-  if (p < 0) return -1;
-  const u32 w = (u32)(a.L[ax] + a.R[ax]);
-  u32 o;
-  if (ax == 0) o = (u32)p + w * ((u32)ci.j + (u32)a.ny * (u32)ci.k);
-  else if (ax == 1) o = (u32)ci.i + (u32)a.nx * ((u32)p + w * (u32)ci.k);
-  else o = (u32)ci.i + (u32)a.nx * ((u32)ci.j + (u32)a.ny * (u32)p);
-  return (long long)((u32)(slot >> 2) * 4u * (u32)a.slab[ax] + 4u * o + (u32)(slot & 3));
-}
-
-template <typename A, class AT>
-__device__ __forceinline__ A profv(const AT &a, int ax, int q, const CellIdx &ci)
-{
-  const int pos = ax == 0 ? ci.i : (ax == 1 ? ci.j : ci.k);
-  return at<A>(a.prof[ax][q], (u32)pos);
+#pragma unroll
+  for (int m = 0; m < 4; ++m) {
+    auto G = [&](int o) { return v[m][o + h]; };
+    if constexpr (ORDER == 2) {
+      out[m] = der_fwd(VEL, AX, m) ? G(-1) - G(0) : G(0) - G(1);
+    } else {
+      out[m] = der_fwd(VEL, AX, m) ? A(9.0 / 8.0) * (G(-1) - G(0)) + A(-1.0 / 24.0) * (G(-h) - G(1))
+                                   : A(9.0 / 8.0) * (G(0) - G(1)) + A(-1.0 / 24.0) * (G(-1) - G(h));
+    }
+  }
 }
 
 // the N coefficients K[k0..k0+N) of cell c from the packed copy (storage units, times the
@@ -256,130 +320,178 @@ __device__ __forceinline__ void gstore(const AT &a, void *p, u32 c, int k0, cons
   }
 }
 
-// Loads of one derivative-table entry: the forward derivative E (fields of state qf) and, in
-// the entry's absorbing slab, the profile values, the forward carry (state qc) and the carry
-// adjoint.  Every kernel below issues all of its loads before its first store: the compiler
-// cannot prove the arrays distinct and never moves a load above a store, so this order keeps
-// a cell's loads in flight together (one memory round trip instead of one per store).
+// contraction written out where the compiler has a choice, so that a gradient does not depend on
+// how the passes are arranged
+__device__ __forceinline__ float fmadd(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double fmadd(double a, double b, double c) { return fma(a, b, c); }
 template <typename A>
-struct PmlIn {
-  A E, e, aa, cf, lc;
-  long long ix;
-};
-template <typename S, int ORDER, class AT>
-__device__ __forceinline__ void pml_load(const AT &a, const Der &D, const CellIdx &ci, int qf, int qc,
-                                         PmlIn<typename AdjT<S>::A> &r)
+__device__ __forceinline__ A product(A a, A b)
 {
-  using A = typename AdjT<S>::A;
-  const u32 st[3] = {1u, (u32)a.sy, (u32)a.sz};
-  r.E = diff<S, ORDER>(fw_field(a, qf, D.field), fw_lo<S>(a, qf, D.field), ci.c, st[D.dir], D.fwd);
-  r.ix = carry_idx(a, D.dir, D.slot, ci);
-  r.e = r.aa = r.cf = r.lc = A(0);
-  if (r.ix >= 0) {
-    r.e = profv<A>(a, D.dir, D.half ? 2 : 0, ci);
-    r.aa = profv<A>(a, D.dir, D.half ? 3 : 1, ci);
-    r.cf = (A)at<typename AdjT<S>::C>(fw_carry(a, qc, D.dir), (u32)r.ix);
-    r.lc = at<A>(a.lcarry[D.dir], (u32)r.ix);
-  }
-}
-// post-PML forward derivative fwdEp, derivative adjoint G and the updated carry adjoint r.lc
-template <typename A>
-__device__ __forceinline__ void pml_apply(PmlIn<A> &r, A lamEp, A &fwdEp, A &G)
-{
-  if (r.ix < 0) {
-    fwdEp = r.E;
-    G = lamEp;
-    return;
-  }
-  fwdEp = (A(1) + r.aa) * r.E + r.cf;
-  G = (A(1) + r.aa) * lamEp + A(2) * r.aa * r.e * r.lc;
-  r.lc = lamEp + r.e * r.lc;
-}
-template <typename A, class AT>
-__device__ __forceinline__ void pml_store(const AT &a, const Der &D, const PmlIn<A> &r)
-{
-  if (r.ix >= 0) at<A>(a.lcarry[D.dir], (u32)r.ix) = r.lc;
+#pragma clang fp contract(off)
+  return a * b;
 }
 
-template <typename S, int ORDER, class AT>
-__device__ __forceinline__ void adj_stress_local(const AT &a, int q, u32 t)
+// The four derivatives of one axis in the local part of a half step: the forward derivatives E
+// (fields of state qf) and, in the axis's slab, its profile values, the forward carries (state qc)
+// and the carry adjoints, a record each.  Both passes issue all of their loads before their first
+// store: the compiler cannot prove the arrays distinct and never moves a load above a store, so
+// this order keeps a cell's loads in flight together (one memory round trip instead of one per
+// store).
+template <typename S, int ORDER, bool VEL, int AX>
+struct AxisLocal {
+  using A = typename AdjT<S>::A;
+  A E[4], e[2], aa[2], cf[4], lc[4], g[4];
+  int sc;
+  template <class AT>
+  __device__ __forceinline__ void load(const AT &a, const CellIdx &ci, int qf, int qc)
+  {
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+      E[m] = diff<S, ORDER>(a, qf, der_field(VEL, AX, m), ci.c, stride<AX>(a), der_fwd(VEL, AX, m));
+    const int pos = AX == 0 ? ci.i : (AX == 1 ? ci.j : ci.k);
+    sc = slab_cell<AX>(a, ci, pos);
+    if (sc >= 0) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {  // integer, half nodes
+        e[b] = at<A>(a.prof[AX][2 * b], (u32)pos);
+        aa[b] = at<A>(a.prof[AX][2 * b + 1], (u32)pos);
+      }
+      typename AdjT<S>::C c4[4];
+      rec_load(c4, fw_carry(a, qc, AX), VEL ? 0u : 1u, (u32)sc, (u32)a.slab[AX]);
+      rec_load(lc, a.lcarry[AX], VEL ? 0u : 1u, (u32)sc, (u32)a.slab[AX]);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) cf[m] = (A)c4[m];
+    }
+  }
+  // E becomes the post-PML forward derivatives, lc the updated carry adjoints, g the derivative
+  // adjoints (in the slab) of lE, the adjoints of the post-PML derivatives
+  __device__ __forceinline__ void apply(const A (&lE)[4])
+  {
+    if (sc < 0) return;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      const int b = der_fwd(VEL, AX, m) ? 1 : 0;
+      const A one = A(1) + aa[b], two = A(2) * aa[b] * e[b];
+      E[m] = fmadd(one, E[m], cf[m]);
+      g[m] = fmadd(one, lE[m], product(two, lc[m]));
+      lc[m] = fmadd(e[b], lc[m], lE[m]);
+    }
+  }
+  template <class AT>
+  __device__ __forceinline__ void store(const AT &a)
+  {
+    if (sc < 0) return;
+    rec_store(g, a.gs[AX], VEL ? 0u : 1u, (u32)sc, (u32)a.slab[AX]);
+    rec_store(lc, a.lcarry[AX], VEL ? 0u : 1u, (u32)sc, (u32)a.slab[AX]);
+  }
+};
+
+// The adjoint sources of step it at cell c added to the adjoints l[m] of fields F0 + m, one rounding
+// for the sample and one for the sum, as a kernel of its own adds them.
+template <typename A, int F0, int N, class IT>
+__device__ __forceinline__ void inject(const IT &j, u32 c, int it, A (&l)[N])
+{
+#pragma clang fp contract(off)
+  if (!((j.has[c >> 5] >> (c & 31u)) & 1u)) return;
+  int lo = 0, hi = j.ncells - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (j.cells[mid] < c) lo = mid + 1;
+    else hi = mid;
+  }
+  for (u32 e = j.first[lo]; e < j.first[lo + 1]; ++e) {
+    const int64_t r = j.ids[e];
+#pragma unroll
+    for (int m = 0; m < N; ++m) {
+      const int ci = j.comp[F0 + m];
+      if (ci < 0) continue;
+      const float v = j.src[((int64_t)ci * j.nt + it) * j.nrec + r] * j.scale[F0 + m];
+      l[m] = l[m] + (A)v;
+    }
+  }
+}
+
+// The loads of one axis at a time: left to itself the compiler issues a pass's hundred loads at
+// once and keeps 200-218 registers for them, two waves a SIMD (FP64: one).  Ended phase by phase
+// they take 127 and 165 (four and three waves), and the passes are faster: 192^3 FP32 996 -> 882 us a
+// step, 128^3 FP64 689 -> 629.  (Capping the registers instead spills: 128^3 FP32 302 -> 602 us.)
+__device__ __forceinline__ void phase() { __builtin_amdgcn_sched_barrier(0); }
+
+// lambda(tau, p) += transposed differences of the velocity-half G of the step after; then the local
+// part of the stress half of state q's step
+template <typename S, int ORDER, class AT, class IT>
+__device__ __forceinline__ void adj_stress(const AT &a, const IT &j, int q, int it, u32 t)
 {
   using A = typename AdjT<S>::A;
   constexpr int h = ORDER / 2;
   CellIdx ci;
   if (t >= a.nupd || !cell_of(a, h, t, ci)) return;
   const u32 c = ci.c;
-  const A ltxx = at<A>(a.lam[6], c), ltyy = at<A>(a.lam[7], c), ltzz = at<A>(a.lam[8], c);
-  const A ltxy = at<A>(a.lam[9], c), ltxz = at<A>(a.lam[10], c), ltyz = at<A>(a.lam[11], c);
-  const A lp = at<A>(a.lam[12], c);
+  A l[7];  // txx tyy tzz txy txz tyz p
+#pragma unroll
+  for (int f = 0; f < 7; ++f) l[f] = at<A>(a.lam[6 + f], c);
+  A gx[4], gy[4], gz[4];  // x1 s1 y2 z2 | x2 y1 s2 z3 | x3 y3 z1 s3
+  gather_axis<A, ORDER, true, 0>(a, ci, gx);
+  phase();
+  gather_axis<A, ORDER, true, 1>(a, ci, gy);
+  phase();
+  gather_axis<A, ORDER, true, 2>(a, ci, gz);
+  l[0] += gx[0], l[1] += gy[1], l[2] += gz[2];
+  l[3] += gy[0] + gx[2], l[4] += gz[0] + gx[3], l[5] += gz[1] + gy[3];
+  l[6] += gx[1] + gy[2] + gz[3];
+  inject<A, 6>(j, c, it, l);
+  const A ltxx = l[0], ltyy = l[1], ltzz = l[2], ltxy = l[3], ltxz = l[4], ltyz = l[5], lp = l[6];
+  phase();
+  AxisLocal<S, ORDER, false, 0> X;  // uxx wx uyx uzx
+  AxisLocal<S, ORDER, false, 1> Y;  // uyy wy uxy uzy
+  AxisLocal<S, ORDER, false, 2> Z;  // uzz wz uxz uyz
+  // velocities of state q+1 (after the velocity half step), carries of state q
+  X.load(a, ci, q + 1, q);
+  phase();
+  Y.load(a, ci, q + 1, q);
+  phase();
+  Z.load(a, ci, q + 1, q);
+  phase();
   A kt[8];  // K[14..21]: P1 P2 S1 S2 S3 Sxy Sxz Syz
   kblock<S, 8>(a, a.kt, c, K_P1, kt);
-  const A P1 = kt[0], P2 = kt[1], S1 = kt[2], S2 = kt[3], S3 = kt[4];
-  const A Sxy = kt[5], Sxz = kt[6], Syz = kt[7];
-  PmlIn<A> in[12];
-#pragma unroll
-  for (int d = 0; d < 12; ++d)  // velocities of state q+1 (after the velocity half step), carries of state q
-    pml_load<S, ORDER>(a, TDER[d], ci, q + 1, q, in[d]);
   double g[8];  // sums of K[14..21]
   gload<A, 8>(a, a.gpt, c, K_P1, g);
-
-  A lE[12];
-  lE[0] = S2 * ltxx + S1 * (ltyy + ltzz) - P1 * lp;
-  lE[1] = S2 * ltyy + S1 * (ltxx + ltzz) - P1 * lp;
-  lE[2] = S2 * ltzz + S1 * (ltxx + ltyy) - P1 * lp;
-  lE[3] = lE[4] = lE[5] = S3 * (ltxx + ltyy + ltzz) - P2 * lp;
-  lE[6] = lE[7] = Sxy * ltxy;
-  lE[8] = lE[9] = Sxz * ltxz;
-  lE[10] = lE[11] = Syz * ltyz;
-  A E[12], G[12];
-#pragma unroll
-  for (int d = 0; d < 12; ++d) pml_apply(in[d], lE[d], E[d], G[d]);
+  const A P1 = kt[0], P2 = kt[1], S1 = kt[2], S2 = kt[3], S3 = kt[4];
+  const A Sxy = kt[5], Sxz = kt[6], Syz = kt[7];
+  const A lxx = S2 * ltxx + S1 * (ltyy + ltzz) - P1 * lp;
+  const A lyy = S2 * ltyy + S1 * (ltxx + ltzz) - P1 * lp;
+  const A lzz = S2 * ltzz + S1 * (ltxx + ltyy) - P1 * lp;
+  const A lw = S3 * (ltxx + ltyy + ltzz) - P2 * lp;
+  const A lxy = Sxy * ltxy, lxz = Sxz * ltxz, lyz = Syz * ltyz;
+  X.apply({lxx, lw, lxy, lxz});
+  Y.apply({lyy, lw, lxy, lyz});
+  Z.apply({lzz, lw, lxz, lyz});
   // FP64 gradient sums: dJ/dK += lambda(output) x (forward term), kernel.cu:484-490
-  const double divu = (double)E[0] + E[1] + E[2], divw = (double)E[3] + E[4] + E[5];
+  const double divu = (double)X.E[0] + Y.E[0] + Z.E[0], divw = (double)X.E[1] + Y.E[1] + Z.E[1];
   g[0] += -(double)lp * divu;
   g[1] += -(double)lp * divw;
-  g[2] += (double)ltxx * (E[1] + E[2]) + (double)ltyy * (E[0] + E[2]) + (double)ltzz * (E[0] + E[1]);
-  g[3] += (double)ltxx * E[0] + (double)ltyy * E[1] + (double)ltzz * E[2];
+  g[2] += (double)ltxx * (Y.E[0] + Z.E[0]) + (double)ltyy * (X.E[0] + Z.E[0]) + (double)ltzz * (X.E[0] + Y.E[0]);
+  g[3] += (double)ltxx * X.E[0] + (double)ltyy * Y.E[0] + (double)ltzz * Z.E[0];
   g[4] += ((double)ltxx + ltyy + ltzz) * divw;
-  g[5] += (double)ltxy * (E[6] + E[7]);
-  g[6] += (double)ltxz * (E[8] + E[9]);
-  g[7] += (double)ltyz * (E[10] + E[11]);
+  g[5] += (double)ltxy * (Y.E[2] + X.E[2]);
+  g[6] += (double)ltxz * (Z.E[2] + X.E[3]);
+  g[7] += (double)ltyz * (Z.E[3] + Y.E[3]);
+  // stores
 #pragma unroll
-  for (int d = 0; d < 12; ++d) {
-    at<A>(a.G[d], c) = G[d];
-    pml_store(a, TDER[d], in[d]);
-  }
+  for (int f = 0; f < 7; ++f) at<A>(a.lam[6 + f], c) = l[f];
+  const A lE[7] = {lxx, lyy, lzz, lw, lxy, lxz, lyz};
+#pragma unroll
+  for (int d = 0; d < 7; ++d) at<A>(a.gt[d], c) = lE[d];
+  X.store(a);
+  Y.store(a);
+  Z.store(a);
   gstore<A, 8>(a, a.gpt, c, K_P1, g);
 }
 
-// lambda(v', q') += transposed differences of the stress-side derivative adjoints
-template <typename S, int ORDER, class AT>
-__device__ __forceinline__ void adj_stress_gather(const AT &a, int, u32 t)
-{
-  using A = typename AdjT<S>::A;
-  constexpr int h = ORDER / 2;
-  CellIdx ci;
-  if (t >= a.nupd || !cell_of(a, h, t, ci)) return;
-  const u32 c = ci.c, sx = 1, sy = (u32)a.sy, sz = (u32)a.sz;
-  const A l0 = at<A>(a.lam[0], c) + (diffT<A, ORDER>(a.G[0], c, sx, 0) + diffT<A, ORDER>(a.G[6], c, sy, 1) +
-                                     diffT<A, ORDER>(a.G[8], c, sz, 1));
-  const A l1 = at<A>(a.lam[1], c) + (diffT<A, ORDER>(a.G[1], c, sy, 0) + diffT<A, ORDER>(a.G[7], c, sx, 1) +
-                                     diffT<A, ORDER>(a.G[10], c, sz, 1));
-  const A l2 = at<A>(a.lam[2], c) + (diffT<A, ORDER>(a.G[2], c, sz, 0) + diffT<A, ORDER>(a.G[9], c, sx, 1) +
-                                     diffT<A, ORDER>(a.G[11], c, sy, 1));
-  const A l3 = at<A>(a.lam[3], c) + diffT<A, ORDER>(a.G[3], c, sx, 0);
-  const A l4 = at<A>(a.lam[4], c) + diffT<A, ORDER>(a.G[4], c, sy, 0);
-  const A l5 = at<A>(a.lam[5], c) + diffT<A, ORDER>(a.G[5], c, sz, 0);
-  at<A>(a.lam[0], c) = l0;
-  at<A>(a.lam[1], c) = l1;
-  at<A>(a.lam[2], c) = l2;
-  at<A>(a.lam[3], c) = l3;
-  at<A>(a.lam[4], c) = l4;
-  at<A>(a.lam[5], c) = l5;
-}
-
-template <typename S, int ORDER, class AT>
-__device__ __forceinline__ void adj_velocity_local(const AT &a, int q, u32 t)
+// lambda(v', q') += transposed differences of the stress-half G; then the local part of the
+// velocity half of state q's step
+template <typename S, int ORDER, class AT, class IT>
+__device__ __forceinline__ void adj_velocity(const AT &a, const IT &j, int q, int it, u32 t)
 {
   using A = typename AdjT<S>::A;
   constexpr int h = ORDER / 2;
@@ -389,105 +501,82 @@ __device__ __forceinline__ void adj_velocity_local(const AT &a, int q, u32 t)
   constexpr int kU1[3] = {K_U1X, K_U1Y, K_U1Z}, kU2[3] = {K_U2X, K_U2Y, K_U2Z};
   constexpr int kW1[3] = {K_W1X, K_W1Y, K_W1Z}, kW2[3] = {K_W2X, K_W2Y, K_W2Z};
   constexpr int kW3[3] = {K_W3X, K_W3Y, K_W3Y};  // qz takes W3y (kernel.cu:220)
-  // loads: adjoint state, coefficients, forward q of states q and q+1, derivative-table
-  // entries, gradient sums
+  A l[6], lv[3], lq[3];  // vx vy vz qx qy qz
+#pragma unroll
+  for (int m = 0; m < 6; ++m) l[m] = at<A>(a.lam[m], c);
+  inject<A, 0>(j, c, it, l);
+  A gx[4], gy[4], gz[4];  // uxx wx uyx uzx | uyy wy uxy uzy | uzz wz uxz uyz
+  gather_axis<A, ORDER, false, 0>(a, ci, gx);
+  phase();
+  gather_axis<A, ORDER, false, 1>(a, ci, gy);
+  phase();
+  gather_axis<A, ORDER, false, 2>(a, ci, gz);
+  lv[0] = l[0] + (gx[0] + gy[2] + gz[2]);
+  lv[1] = l[1] + (gy[0] + gx[2] + gz[3]);
+  lv[2] = l[2] + (gz[0] + gx[3] + gy[3]);
+  lq[0] = l[3] + gx[1];
+  lq[1] = l[4] + gy[1];
+  lq[2] = l[5] + gz[1];
+  phase();
+  AxisLocal<S, ORDER, true, 0> X;  // x1 s1 y2 z2
+  AxisLocal<S, ORDER, true, 1> Y;  // x2 y1 s2 z3
+  AxisLocal<S, ORDER, true, 2> Z;  // x3 y3 z1 s3
+  X.load(a, ci, q, q);
+  phase();
+  Y.load(a, ci, q, q);
+  phase();
+  Z.load(a, ci, q, q);
+  phase();
   A kv[14];  // K[0..13]: U1 xyz, U2 xyz, W1 xyz, W2 xyz, W3x, W3y
   kblock<S, 14>(a, a.kv, c, 0, kv);
-  A lv[3], lq[3], U1[3], U2[3], W1[3], W2[3], W3[3];
-  double q0[3], q1[3], gU1[3], gU2[3], gW1[3], gW2[3];
+  double q0[3], q1[3];
 #pragma unroll
   for (int m = 0; m < 3; ++m) {
-    lv[m] = at<A>(a.lam[m], c);
-    lq[m] = at<A>(a.lam[3 + m], c);
-    U1[m] = kv[kU1[m]], U2[m] = kv[kU2[m]];
-    W1[m] = kv[kW1[m]], W2[m] = kv[kW2[m]], W3[m] = kv[kW3[m]];
     q0[m] = (double)at<typename AdjT<S>::T>(fw_field(a, q, 3 + m), c);  // q carries no residual
     q1[m] = (double)at<typename AdjT<S>::T>(fw_field(a, q + 1, 3 + m), c);
   }
-  PmlIn<A> in[12];
-#pragma unroll
-  for (int d = 0; d < 12; ++d) pml_load<S, ORDER>(a, VDER[d], ci, q, q, in[d]);
   double gv[14];  // sums of K[0..13]
   gload<A, 14>(a, a.gpv, c, 0, gv);
-#pragma unroll
-  for (int m = 0; m < 3; ++m) {
-    gU1[m] = gv[kU1[m]], gU2[m] = gv[kU2[m]];
-    gW1[m] = gv[kW1[m]], gW2[m] = gv[kW2[m]];
-  }
-  double gW3x = gv[K_W3X], gW3y = gv[K_W3Y];
-
   // per component: lambda_qe = lambda_q' - U2 lambda_v'; lambda_S = U1 lambda_v' - W2 lambda_qe;
   // lambda_Ds = -W3 lambda_qe (qz takes W3y, kernel.cu:220)
   A lS[3], lDs[3], lqe[3], lqn[3];
 #pragma unroll
   for (int m = 0; m < 3; ++m) {
-    lqe[m] = lq[m] - U2[m] * lv[m];
-    lS[m] = U1[m] * lv[m] - W2[m] * lqe[m];
-    lDs[m] = -W3[m] * lqe[m];
-    lqn[m] = U2[m] * lv[m] + W1[m] * lqe[m];  // lambda_q at step n (lambda_v is unchanged)
+    const A U1 = kv[kU1[m]], U2 = kv[kU2[m]], W1 = kv[kW1[m]], W2 = kv[kW2[m]], W3 = kv[kW3[m]];
+    lqe[m] = lq[m] - U2 * lv[m];
+    lS[m] = U1 * lv[m] - W2 * lqe[m];
+    lDs[m] = -W3 * lqe[m];
+    lqn[m] = U2 * lv[m] + W1 * lqe[m];  // lambda_q at step n (lambda_v is unchanged)
   }
-  // derivative order x1 x2 x3 s1 y1 y2 y3 s2 z1 z2 z3 s3
-  const A lD[12] = {lS[0], lS[0], lS[0], lDs[0], lS[1], lS[1], lS[1], lDs[1],
-                    lS[2], lS[2], lS[2], lDs[2]};
-  A D[12], G[12];
-#pragma unroll
-  for (int d = 0; d < 12; ++d) pml_apply(in[d], lD[d], D[d], G[d]);
+  X.apply({lS[0], lDs[0], lS[1], lS[2]});
+  Y.apply({lS[0], lS[1], lDs[1], lS[2]});
+  Z.apply({lS[0], lS[1], lS[2], lDs[2]});
   // FP64 gradient sums with the forward terms of kernel.cu:218-225
-  const double Ssum[3] = {(double)D[0] + D[1] + D[2], (double)D[5] + D[4] + D[6],
-                          (double)D[9] + D[10] + D[8]};
-  const double Ds[3] = {(double)D[3], (double)D[7], (double)D[11]};
+  const double Ssum[3] = {(double)X.E[0] + Y.E[0] + Z.E[0], (double)X.E[2] + Y.E[1] + Z.E[1],
+                          (double)X.E[3] + Y.E[3] + Z.E[2]};
+  const double Ds[3] = {(double)X.E[1], (double)Y.E[2], (double)Z.E[3]};
 #pragma unroll
   for (int m = 0; m < 3; ++m) {
-    gU1[m] += (double)lv[m] * Ssum[m];
-    gU2[m] += -(double)lv[m] * (q1[m] - q0[m]);
-    gW1[m] += (double)lqe[m] * q0[m];
-    gW2[m] += -(double)lqe[m] * Ssum[m];
+    gv[kU1[m]] += (double)lv[m] * Ssum[m];
+    gv[kU2[m]] += -(double)lv[m] * (q1[m] - q0[m]);
+    gv[kW1[m]] += (double)lqe[m] * q0[m];
+    gv[kW2[m]] += -(double)lqe[m] * Ssum[m];
   }
-  gW3x += -(double)lqe[0] * Ds[0];
-  gW3y += -(double)lqe[1] * Ds[1];  // qy's term, then qz's, into the one W3y sum
-  gW3y += -(double)lqe[2] * Ds[2];
+  gv[K_W3X] += -(double)lqe[0] * Ds[0];
+  gv[K_W3Y] += -(double)lqe[1] * Ds[1];  // qy's term, then qz's, into the one W3y sum
+  gv[K_W3Y] += -(double)lqe[2] * Ds[2];
   // stores
 #pragma unroll
-  for (int m = 0; m < 3; ++m) at<A>(a.lam[3 + m], c) = lqn[m];
-#pragma unroll
-  for (int d = 0; d < 12; ++d) {
-    at<A>(a.G[d], c) = G[d];
-    pml_store(a, VDER[d], in[d]);
-  }
-#pragma unroll
   for (int m = 0; m < 3; ++m) {
-    gv[kU1[m]] = gU1[m], gv[kU2[m]] = gU2[m];
-    gv[kW1[m]] = gW1[m], gv[kW2[m]] = gW2[m];
+    at<A>(a.lam[m], c) = lv[m];
+    at<A>(a.lam[3 + m], c) = lqn[m];
+    at<A>(a.gv[m], c) = lS[m];
+    at<A>(a.gv[3 + m], c) = lDs[m];
   }
-  gv[K_W3X] = gW3x;
-  gv[K_W3Y] = gW3y;
+  X.store(a);
+  Y.store(a);
+  Z.store(a);
   gstore<A, 14>(a, a.gpv, c, 0, gv);
-}
-
-// lambda(tau, p) += transposed differences of the velocity-side derivative adjoints
-template <typename S, int ORDER, class AT>
-__device__ __forceinline__ void adj_velocity_gather(const AT &a, int, u32 t)
-{
-  using A = typename AdjT<S>::A;
-  constexpr int h = ORDER / 2;
-  CellIdx ci;
-  if (t >= a.nupd || !cell_of(a, h, t, ci)) return;
-  const u32 c = ci.c, sx = 1, sy = (u32)a.sy, sz = (u32)a.sz;
-  const A l6 = at<A>(a.lam[6], c) + diffT<A, ORDER>(a.G[0], c, sx, 1);
-  const A l9 = at<A>(a.lam[9], c) + (diffT<A, ORDER>(a.G[1], c, sy, 0) + diffT<A, ORDER>(a.G[5], c, sx, 0));
-  const A l10 = at<A>(a.lam[10], c) + (diffT<A, ORDER>(a.G[2], c, sz, 0) + diffT<A, ORDER>(a.G[9], c, sx, 0));
-  const A l7 = at<A>(a.lam[7], c) + diffT<A, ORDER>(a.G[4], c, sy, 1);
-  const A l11 = at<A>(a.lam[11], c) + (diffT<A, ORDER>(a.G[6], c, sz, 0) + diffT<A, ORDER>(a.G[10], c, sy, 0));
-  const A l8 = at<A>(a.lam[8], c) + diffT<A, ORDER>(a.G[8], c, sz, 1);
-  const A l12 = at<A>(a.lam[12], c) + (diffT<A, ORDER>(a.G[3], c, sx, 1) + diffT<A, ORDER>(a.G[7], c, sy, 1) +
-                                       diffT<A, ORDER>(a.G[11], c, sz, 1));
-  at<A>(a.lam[6], c) = l6;
-  at<A>(a.lam[9], c) = l9;
-  at<A>(a.lam[10], c) = l10;
-  at<A>(a.lam[7], c) = l7;
-  at<A>(a.lam[11], c) = l11;
-  at<A>(a.lam[8], c) = l8;
-  at<A>(a.lam[12], c) = l12;
 }
 
 // the float partial sums of a segment into the FP64 gradient sums, cleared for the next one
@@ -513,23 +602,20 @@ __device__ __forceinline__ void adj_flush(const AT &a, u32 t)
   packed::store<float, 8>(a.gpt, n, c, zero);
 }
 
-template <typename S, int ORDER, int WHICH, class AT>
-__device__ __forceinline__ void adj_pass(const AT &a, int q, u32 t)
+// WHICH 0: the stress pass, 1: the velocity pass, 2: the flush
+template <typename S, int ORDER, int WHICH, class AT, class IT>
+__device__ __forceinline__ void adj_pass(const AT &a, const IT &j, int q, int it, u32 t)
 {
-  if constexpr (WHICH == 0) adj_stress_local<S, ORDER>(a, q, t);
-  else if constexpr (WHICH == 1) adj_stress_gather<S, ORDER>(a, q, t);
-  else if constexpr (WHICH == 2) adj_velocity_local<S, ORDER>(a, q, t);
-  else if constexpr (WHICH == 3) adj_velocity_gather<S, ORDER>(a, q, t);
+  if constexpr (WHICH == 0) adj_stress<S, ORDER>(a, j, q, it, t);
+  else if constexpr (WHICH == 1) adj_velocity<S, ORDER>(a, j, q, it, t);
   else adj_flush<S, ORDER>(a, t);
 }
 
 // 256 cells a block, dealt out to the XCDs in runs of blocks as the forward kernels' tiles are
-// (xcd_run: the four passes of a 128^3 FP32 step 342 us in launch order, 308 us in runs of 8; 192^3
-// 1090 and 1025 us; 90^3 FP16M 237 and 216 us)
 template <typename S, int ORDER, int WHICH>
-__global__ void __launch_bounds__(256) k_adj(const AdjArgs a, int q, int xg)
+__global__ void __launch_bounds__(256) k_adj(const AdjArgs a, const InjectArgs j, int q, int it, int xg)
 {
-  adj_pass<S, ORDER, WHICH>(a, q, (u32)xcd_tile(blockIdx.x & 7, blockIdx.x >> 3, xg) * 256u + threadIdx.x);
+  adj_pass<S, ORDER, WHICH>(a, j, q, it, (u32)xcd_tile(blockIdx.x & 7, blockIdx.x >> 3, xg) * 256u + threadIdx.x);
 }
 
 // batched: argument tables read through the constant address space (uniform per block)
@@ -551,34 +637,15 @@ __device__ __forceinline__ int shot_of_block(const AdjBatch &b, int blk)
 }
 
 template <typename S, int ORDER, int WHICH>
-__global__ void __launch_bounds__(256) k_adj_batch(const AdjBatch b, int q, int xg)
+__global__ void __launch_bounds__(256) k_adj_batch(const AdjBatch b, int q, int it, int xg)
 {
   const int blk = xcd_tile(blockIdx.x & 7, blockIdx.x >> 3, xg);
   if (blk >= b.total_blocks) return;
   const int s = shot_of_block(b, blk);
   const CAdjArgs &a = ((CAdjArgs *)b.shots)[s];
+  const CInjectArgs &j = ((CInjectArgs *)b.inject)[s];
   const u32 t = (u32)(blk - ((CInt *)b.block_start)[s]) * 256u + threadIdx.x;
-  adj_pass<S, ORDER, WHICH>(a, q, t);
-}
-
-// lambda(recorded field at receiver) += scale x adjoint source sample of step it
-template <typename A, class IT>
-__device__ __forceinline__ void inject_one(const IT &a, int64_t r, int ci, int it)
-{
-  if (r >= a.nrec || ci >= a.ncomp) return;
-  const float v = a.src[((int64_t)ci * a.nt + it) * a.nrec + r] * a.scale[ci];
-  atomicAdd(&((A *)a.lam[a.comp[ci]])[a.rec[r]], (A)v);
-}
-template <typename A>
-__global__ void k_adj_inject(const InjectArgs a, int it)
-{
-  inject_one<A>(a, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, (int)blockIdx.y, it);
-}
-template <typename A>
-__global__ void k_adj_inject_batch(const InjectArgs *tab, int it)
-{
-  const CInjectArgs &a = ((CInjectArgs *)tab)[blockIdx.z];
-  inject_one<A>(a, (int64_t)blockIdx.x * blockDim.x + threadIdx.x, (int)blockIdx.y, it);
+  adj_pass<S, ORDER, WHICH>(a, j, q, it, t);
 }
 
 // J = 1/2 sum (d - obs)^2 in FP64, residual = d - obs
@@ -744,123 +811,84 @@ __global__ void __launch_bounds__(256) k_copy_batch(const CopyEntry *tab)
     ((uint8_t *)e.dst)[(words << 2) + threadIdx.x] = ((const uint8_t *)e.src)[(words << 2) + threadIdx.x];
 }
 
-template <typename S, int ORDER>
-hipError_t adj_launch(int which, const AdjArgs &a, int q, hipStream_t s)
-{
-  const int64_t n = ((int64_t)a.nupd + 255) / 256;
-  const int xg = xcd_run(n, 256, n * 256);
-  const dim3 blocks((unsigned)(8 * xcd_slots(n, xg)));
-  switch (which) {
-    case 0: hipLaunchKernelGGL((k_adj<S, ORDER, 0>), blocks, dim3(256), 0, s, a, q, xg); break;
-    case 1: hipLaunchKernelGGL((k_adj<S, ORDER, 1>), blocks, dim3(256), 0, s, a, q, xg); break;
-    case 2: hipLaunchKernelGGL((k_adj<S, ORDER, 2>), blocks, dim3(256), 0, s, a, q, xg); break;
-    case 3: hipLaunchKernelGGL((k_adj<S, ORDER, 3>), blocks, dim3(256), 0, s, a, q, xg); break;
-    case 4: hipLaunchKernelGGL((k_adj<S, ORDER, 4>), blocks, dim3(256), 0, s, a, q, xg); break;
-    default: return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
-}
-template <typename S, int ORDER>
-hipError_t adj_launch_batch(int which, const AdjBatch &b, int q, hipStream_t s)
-{
-  const int xg = xcd_run(b.total_blocks, 256, (int64_t)b.total_blocks * 256);
-  const dim3 blocks((unsigned)(8 * xcd_slots(b.total_blocks, xg)));
-  switch (which) {
-    case 0: hipLaunchKernelGGL((k_adj_batch<S, ORDER, 0>), blocks, dim3(256), 0, s, b, q, xg); break;
-    case 1: hipLaunchKernelGGL((k_adj_batch<S, ORDER, 1>), blocks, dim3(256), 0, s, b, q, xg); break;
-    case 2: hipLaunchKernelGGL((k_adj_batch<S, ORDER, 2>), blocks, dim3(256), 0, s, b, q, xg); break;
-    case 3: hipLaunchKernelGGL((k_adj_batch<S, ORDER, 3>), blocks, dim3(256), 0, s, b, q, xg); break;
-    case 4: hipLaunchKernelGGL((k_adj_batch<S, ORDER, 4>), blocks, dim3(256), 0, s, b, q, xg); break;
-    default: return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
-}
-
 struct SingleRun {
   const AdjArgs &a;
-  int q;
+  const InjectArgs &j;
+  int q, it;
   hipStream_t s;
-  template <typename S, int O>
-  hipError_t run(int which) { return adj_launch<S, O>(which, a, q, s); }
+  template <typename S, int O, int W>
+  void pass()
+  {
+    const int64_t n = ((int64_t)a.nupd + 255) / 256;
+    const int xg = xcd_run(n, 256, n * 256);
+    hipLaunchKernelGGL((k_adj<S, O, W>), dim3((unsigned)(8 * xcd_slots(n, xg))), dim3(256), 0, s, a, j, q, it, xg);
+  }
 };
 struct BatchRun {
   const AdjBatch &b;
-  int q;
+  int q, it;
   hipStream_t s;
-  template <typename S, int O>
-  hipError_t run(int which) { return adj_launch_batch<S, O>(which, b, q, s); }
+  template <typename S, int O, int W>
+  void pass()
+  {
+    const int xg = xcd_run(b.total_blocks, 256, (int64_t)b.total_blocks * 256);
+    hipLaunchKernelGGL((k_adj_batch<S, O, W>), dim3((unsigned)(8 * xcd_slots(b.total_blocks, xg))), dim3(256), 0, s, b,
+                       q, it, xg);
+  }
 };
 
-// passes first..last-1 (0-3: the adjoint step, 4: the flush), in order, for the storage
-// type of prec
+template <typename S, int O, class F>
+hipError_t run_passes(F f, bool flush)
+{
+  if (flush) {
+    f.template pass<S, O, 2>();
+  } else {
+    f.template pass<S, O, 0>();
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    f.template pass<S, O, 1>();
+  }
+  return hipGetLastError();
+}
+// the passes for the storage type of prec
 template <class F>
-hipError_t passes(int prec, int order, F f, int first, int last)
+hipError_t passes(int prec, int order, F f, bool flush)
 {
   if (order != 2 && order != 4) return hipErrorInvalidValue;
-  for (int which = first; which < last; ++which) {
-    hipError_t e;
-    if (prec == PREC_FP32) e = order == 2 ? f.template run<float, 2>(which) : f.template run<float, 4>(which);
-    else if (prec == PREC_FP64) e = order == 2 ? f.template run<double, 2>(which) : f.template run<double, 4>(which);
-    else if (prec == PREC_FP16) e = order == 2 ? f.template run<_Float16, 2>(which) : f.template run<_Float16, 4>(which);
-    else if (prec == PREC_FP16T || prec == PREC_FP16C)
-      e = order == 2 ? f.template run<H16R, 2>(which) : f.template run<H16R, 4>(which);
-    else if (prec == PREC_FP16M)
-      e = order == 2 ? f.template run<H16P, 2>(which) : f.template run<H16P, 4>(which);
-    else return hipErrorInvalidValue;
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
+  if (prec == PREC_FP32) return order == 2 ? run_passes<float, 2>(f, flush) : run_passes<float, 4>(f, flush);
+  if (prec == PREC_FP64) return order == 2 ? run_passes<double, 2>(f, flush) : run_passes<double, 4>(f, flush);
+  if (prec == PREC_FP16) return order == 2 ? run_passes<_Float16, 2>(f, flush) : run_passes<_Float16, 4>(f, flush);
+  if (prec == PREC_FP16T)
+    return order == 2 ? run_passes<H16R<COMP_FIELDS_T>, 2>(f, flush) : run_passes<H16R<COMP_FIELDS_T>, 4>(f, flush);
+  if (prec == PREC_FP16C)
+    return order == 2 ? run_passes<H16R<COMP_FIELDS_C>, 2>(f, flush) : run_passes<H16R<COMP_FIELDS_C>, 4>(f, flush);
+  if (prec == PREC_FP16M) return order == 2 ? run_passes<H16P, 2>(f, flush) : run_passes<H16P, 4>(f, flush);
+  return hipErrorInvalidValue;
 }
-
 }  // namespace
 
-hipError_t launch_adjoint_step(int prec, int order, const AdjArgs &a, int q, hipStream_t s)
+hipError_t launch_adjoint_step(int prec, int order, const AdjArgs &a, const InjectArgs &j, int q, int it, hipStream_t s)
 {
   if (a.nupd == 0) return hipSuccess;
-  return passes(prec, order, SingleRun{a, q, s}, 0, 4);
+  return passes(prec, order, SingleRun{a, j, q, it, s}, false);
 }
 
 hipError_t launch_adjoint_flush(int prec, int order, const AdjArgs &a, hipStream_t s)
 {
   if (a.nupd == 0 || prec == PREC_FP64) return hipSuccess;
-  return passes(prec, order, SingleRun{a, 0, s}, 4, 5);
+  return passes(prec, order, SingleRun{a, InjectArgs{}, 0, 0, s}, true);
 }
 
 hipError_t launch_adjoint_flush_batch(int prec, int order, const AdjBatch &b, hipStream_t s)
 {
   if (b.total_blocks <= 0 || prec == PREC_FP64) return hipSuccess;
-  return passes(prec, order, BatchRun{b, 0, s}, 4, 5);
+  return passes(prec, order, BatchRun{b, 0, 0, s}, true);
 }
 
-hipError_t launch_adjoint_step_batch(int prec, int order, const AdjBatch &b, int q, hipStream_t s)
+hipError_t launch_adjoint_step_batch(int prec, int order, const AdjBatch &b, int q, int it, hipStream_t s)
 {
   if (b.total_blocks <= 0) return hipSuccess;
-  return passes(prec, order, BatchRun{b, q, s}, 0, 4);
-}
-
-hipError_t launch_adjoint_inject(int prec, const InjectArgs &a, int it, hipStream_t s)
-{
-  if (a.nrec <= 0 || a.ncomp <= 0) return hipSuccess;
-  dim3 grid((unsigned)((a.nrec + 255) / 256), (unsigned)a.ncomp);
-  if (prec == PREC_FP64) hipLaunchKernelGGL(k_adj_inject<double>, grid, dim3(256), 0, s, a, it);
-  else if (prec == PREC_FP32 || prec == PREC_FP16 || prec == PREC_FP16T || prec == PREC_FP16C ||
-           prec == PREC_FP16M)
-    hipLaunchKernelGGL(k_adj_inject<float>, grid, dim3(256), 0, s, a, it);
-  else return hipErrorInvalidValue;
-  return hipGetLastError();
-}
-
-hipError_t launch_adjoint_inject_batch(int prec, const InjectArgs *tab, int nshots, int64_t max_nrec,
-                                       int max_ncomp, int it, hipStream_t s)
-{
-  if (nshots <= 0 || max_nrec <= 0 || max_ncomp <= 0) return hipSuccess;
-  dim3 grid((unsigned)((max_nrec + 255) / 256), (unsigned)max_ncomp, (unsigned)nshots);
-  if (prec == PREC_FP64) hipLaunchKernelGGL(k_adj_inject_batch<double>, grid, dim3(256), 0, s, tab, it);
-  else if (prec == PREC_FP32 || prec == PREC_FP16 || prec == PREC_FP16T || prec == PREC_FP16C ||
-           prec == PREC_FP16M)
-    hipLaunchKernelGGL(k_adj_inject_batch<float>, grid, dim3(256), 0, s, tab, it);
-  else return hipErrorInvalidValue;
-  return hipGetLastError();
+  return passes(prec, order, BatchRun{b, q, it, s}, false);
 }
 
 hipError_t launch_misfit(const void *d, bool d_double, const float *obs, float *res, int64_t n,

@@ -18,10 +18,12 @@ struct AdjArgs {
   uint64_t sb, fbytes, coff[3];
   uint64_t loff;             // offset in a state of the FP16T / FP16C residual arrays (int8, field f at
                              // f*n) or of FP16M's residual records (4 bytes per cell), else 0
-  uint32_t lomask;           // fields whose residual the adjoint reads (FP16T, FP16M tau, p; FP16C v, tau, p)
   void *lam[NFIELD];         // adjoint wavefields (arithmetic type), storage units
   void *lcarry[3];           // adjoint carries (arithmetic type), forward layout
-  void *G[12];               // derivative adjoints of the current half step (arithmetic type)
+  // derivative adjoints between the passes (arithmetic type): full arrays of the velocity half's 6
+  // (S, Ds of x, y, z) and the stress half's 7 (uxx, uyy, uzz, div w, xy, xz, yz), and per axis the
+  // records of the slab's own four (forward carry layout)
+  void *gv[6], *gt[7], *gs[3];
   double *grad[NKC];         // dJ/dK in storage units (multiply by the handle's kfac), FP64
   // per-step accumulation of dJ/dK: float partial sums over one checkpoint segment (FP32 and
   // FP16 handles; launch_adjoint_flush adds them into grad and clears them), grad itself on
@@ -42,21 +44,24 @@ struct AdjArgs {
   uint32_t nupd;             // cells of the update box
 };
 
+// The adjoint sources: a bit per cell tells the thread that updates a cell whether receivers sit
+// there, and the cells' sorted list which.
 struct InjectArgs {
-  void *lam[NFIELD];
-  const int64_t *rec;
+  const uint32_t *has;       // bit c: cell c holds receivers
+  const uint32_t *cells;     // the ncells cells that do, ascending
+  const uint32_t *first;     // ncells + 1: their first entries in ids
+  const uint32_t *ids;       // receivers by cell
+  int ncells;
   int64_t nrec;
-  int comp[NFIELD];
-  int ncomp;
-  float scale[NFIELD];
+  int comp[NFIELD];          // component that records field f, or -1
+  float scale[NFIELD];       // storage scale of field f (traces hold scale x stored value)
   const float *src;          // adjoint source [comp][nt][rec]
   int nt;
 };
 
-// adjoint of one full step (stress then velocity half step, two passes each) for segment
-// step q; prec is the storage precision (FP32, FP64 or FP16)
-hipError_t launch_adjoint_step(int prec, int order, const AdjArgs &a, int q, hipStream_t s);
-hipError_t launch_adjoint_inject(int prec, const InjectArgs &a, int it, hipStream_t s);
+// adjoint of one full step (the stress pass, then the velocity pass) for step it, segment step q,
+// with step it's adjoint sources; prec is the storage precision
+hipError_t launch_adjoint_step(int prec, int order, const AdjArgs &a, const InjectArgs &j, int q, int it, hipStream_t s);
 // grad += packed partial sums, partial sums = 0 over the update box (no-op on FP64 handles,
 // which sum into grad)
 hipError_t launch_adjoint_flush(int prec, int order, const AdjArgs &a, hipStream_t s);
@@ -71,11 +76,10 @@ struct AdjBatch {
   const AdjArgs *shots;
   const int *block_start;    // nshots + 1
   int nshots, total_blocks;
+  const InjectArgs *inject;  // one per shot
 };
-hipError_t launch_adjoint_step_batch(int prec, int order, const AdjBatch &b, int q, hipStream_t s);
+hipError_t launch_adjoint_step_batch(int prec, int order, const AdjBatch &b, int q, int it, hipStream_t s);
 hipError_t launch_adjoint_flush_batch(int prec, int order, const AdjBatch &b, hipStream_t s);
-hipError_t launch_adjoint_inject_batch(int prec, const InjectArgs *tab, int nshots, int64_t max_nrec,
-                                       int max_ncomp, int it, hipStream_t s);
 
 // Chain rule on the device: storage-unit coefficient gradients of one window (grad[k] times
 // kfac[k] gives dJ/dK) -> dJ/d(lambda, mu, alpha, M, rho, rho_f), written to (add: added into)

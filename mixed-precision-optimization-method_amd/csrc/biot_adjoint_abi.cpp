@@ -99,22 +99,32 @@ extern "C" int biot_forward_checkpointed(biot_handle *h, int32_t nt, int32_t eve
   for (uint32_t f = 0; f < NFIELD; ++f)
     if ((h->src_mask >> f) & 1u && !(f >= 6))
       return afail(h, BIOT_ERR_ARG, "the adjoint path supports sources on stresses and pressure only");
-  h->free_adjoint();
+  // The buffers of the last run serve one of the same length and spacing on the same model (a new
+  // model, source or receiver layout releases them): releasing and reserving the states of every
+  // run took 5-100 ms of a 96x80x89 gradient, and now and then a second.
+  const bool room = h->room_every == every && h->room_nt == nt;
+  h->ckpt_every = h->ckpt_nt = 0;
+  if (!room) h->free_adjoint();
   if (int rc = h->build_adjoint_coefs()) return rc;  // FP16M: the coefficient copy the adjoint reads
   const size_t sb = h->state_bytes();
   if (every == 1) {
     // every step's state, in one block the adjoint reads directly (no recomputation)
-    void *p = nullptr;
     const size_t bytes = sb * (size_t)(nt + 1);
-    if (hipMalloc(&p, bytes) != hipSuccess)
-      return afail(h, BIOT_ERR_NOMEM, "the %d step states (%zu bytes) do not fit; use every > 1", nt + 1, bytes);
-    h->ckpt.push_back(p);
+    if (!room) {
+      void *p = nullptr;
+      if (hipMalloc(&p, bytes) != hipSuccess)
+        return afail(h, BIOT_ERR_NOMEM, "the %d step states (%zu bytes) do not fit; use every > 1", nt + 1, bytes);
+      h->ckpt.push_back(p);
+      h->room_every = 1;
+      h->room_nt = nt;
+    }
+    char *p = (char *)h->ckpt[0];
     int rc = biot_reset(h);
     if (rc) return rc;
     AHIP(h, hipEventRecord(h->ev0, h->stream));
-    rc = h->enqueue_steps(nt, nullptr, (char *)p);
+    rc = h->enqueue_steps(nt, nullptr, p);
     if (rc) return rc;
-    h->save_state((char *)p + (size_t)nt * sb);
+    h->save_state(p + (size_t)nt * sb);
     AHIP(h, hipEventRecord(h->ev1, h->stream));
     AHIP(h, hipEventSynchronize(h->ev1));
     float ms = 0;
@@ -125,7 +135,7 @@ extern "C" int biot_forward_checkpointed(biot_handle *h, int32_t nt, int32_t eve
     return BIOT_OK;
   }
   const int nseg = (nt + every - 1) / every;
-  for (int s = 0; s < nseg; ++s) {
+  for (int s = 0; s < nseg && !room; ++s) {
     void *p = nullptr;
     if (hipMalloc(&p, sb) != hipSuccess) {
       h->free_adjoint();
@@ -133,6 +143,8 @@ extern "C" int biot_forward_checkpointed(biot_handle *h, int32_t nt, int32_t eve
     }
     h->ckpt.push_back(p);
   }
+  h->room_every = every;
+  h->room_nt = nt;
   int rc = biot_reset(h);
   if (rc) return rc;
   AHIP(h, hipEventRecord(h->ev0, h->stream));
@@ -217,8 +229,7 @@ extern "C" int biot_adjoint(biot_handle *h, const float *adj_source, double *con
     // 0), so both modes give the same gradients bit for bit.
     A.slots = (const char *)h->ckpt[0];
     for (int it = nt - 1; it >= 0; --it) {
-      AHIP(h, launch_adjoint_inject(h->prec, I, it, h->stream));
-      AHIP(h, launch_adjoint_step(h->prec, order, A, it, h->stream));
+      AHIP(h, launch_adjoint_step(h->prec, order, A, I, it, it, h->stream));
       if (it % kStoredFlushEvery == 0) AHIP(h, launch_adjoint_flush(h->prec, order, A, h->stream));
     }
   }
@@ -239,10 +250,7 @@ extern "C" int biot_adjoint(biot_handle *h, const float *adj_source, double *con
       AHIP(h, launch_stress(h->prec, order, st, h->shape, h->stream, nullptr, next ? &sa : nullptr));
     }
     h->save_state(slot(K));
-    for (int it = n0 + K - 1; it >= n0; --it) {
-      AHIP(h, launch_adjoint_inject(h->prec, I, it, h->stream));
-      AHIP(h, launch_adjoint_step(h->prec, order, A, it - n0, h->stream));
-    }
+    for (int it = n0 + K - 1; it >= n0; --it) AHIP(h, launch_adjoint_step(h->prec, order, A, I, it - n0, it, h->stream));
     AHIP(h, launch_adjoint_flush(h->prec, order, A, h->stream));  // the segment's float partial sums
   }
   AHIP(h, hipEventRecord(h->ev1, h->stream));

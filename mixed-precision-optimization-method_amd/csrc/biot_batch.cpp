@@ -52,7 +52,6 @@ struct biot_batch {
   int total_tiles = 0;
   int nactive = 0;                 // shots the current tables cover
   int64_t max_nrec = 0;
-  int max_ncomp = 0;
   bool fused = false;              // every shot's source and receivers can ride on the half steps
   bool built = false;
   // captured steps
@@ -325,7 +324,6 @@ int build_tables(biot_batch *b, int s0 = 0, int s1 = -1)
   std::vector<SourceArgs> src(S);
   std::vector<RecordArgs> rec(S);
   b->max_nrec = 0;
-  b->max_ncomp = 0;
   b->fused = true;
   const int h2 = b->cfg.order / 2;
   for (int i = 0; i < S; ++i) {
@@ -337,7 +335,6 @@ int build_tables(biot_batch *b, int s0 = 0, int s1 = -1)
     h->source_args(src[i]);
     h->record_args(rec[i]);
     b->max_nrec = std::max(b->max_nrec, h->nrec);
-    b->max_ncomp = std::max(b->max_ncomp, h->ncomp);
     b->fused = b->fused && !h->source_recorded() && (!h->src_mask || h->source_in_stress());
   }
   b->total_tiles = tiles[S];
@@ -693,7 +690,7 @@ int gradient_group(biot_batch *b, int s0, int s1, int nt, int every, const float
     if (h->d_gpart) BHIP(b, hipMemsetAsync(h->d_gpart, 0, (size_t)NKC * h->n * sizeof(float), b->stream));
   }
   // ---- segment recompute and adjoint sweep, all shots of the group per launch
-  const AdjBatch ab{b->d_adj, b->d_blocks, S, b->adj_blocks};
+  const AdjBatch ab{b->d_adj, b->d_blocks, S, b->adj_blocks, b->d_inj};
   for (int k = nseg - 1; k >= 0; --k) {
     const int n0 = k * every, K = std::min(every, nt - n0);
     BHIP(b, load_ckpt(k));
@@ -707,10 +704,7 @@ int gradient_group(biot_batch *b, int s0, int s1, int nt, int every, const float
       BHIP(b, launch_step_batch(prec, order, false, ba, b->shape, b->blocks, 0, b->stream));
     }
     BHIP(b, save_slot(K));
-    for (int it = n0 + K - 1; it >= n0; --it) {
-      BHIP(b, launch_adjoint_inject_batch(prec, b->d_inj, S, b->max_nrec, b->max_ncomp, it, b->stream));
-      BHIP(b, launch_adjoint_step_batch(prec, order, ab, it - n0, b->stream));
-    }
+    for (int it = n0 + K - 1; it >= n0; --it) BHIP(b, launch_adjoint_step_batch(prec, order, ab, it - n0, it, b->stream));
     BHIP(b, launch_adjoint_flush_batch(prec, order, ab, b->stream));
   }
   // ---- chain rule per shot into the model-grid gradient

@@ -124,9 +124,9 @@ int biot_handle::check_nonfinite()
 size_t biot_handle::lam_bytes() const
 {
   const size_t asz = prec == BIOT_FP64 ? 8 : 4;
-  size_t b = (size_t)NFIELD * n * asz + (size_t)12 * n * asz;
-  for (int ax = 0; ax < 3; ++ax) b += (size_t)NCARRY * slab[ax] * asz;
-  return b;
+  size_t b = (size_t)(NFIELD + 13) * n * asz;
+  for (int ax = 0; ax < 3; ++ax) b += 2 * round256((size_t)NCARRY * slab[ax] * asz);
+  return b + 256;
 }
 
 int biot_handle::alloc_adjoint(int every)
@@ -156,6 +156,39 @@ int biot_handle::alloc_adjoint(int every)
     err = "adjoint buffers do not fit in device memory";
     return BIOT_ERR_NOMEM;
   }
+  return build_inject();
+}
+
+int biot_handle::build_inject()
+{
+  if (d_inj) return BIOT_OK;
+  // receivers by cell, in list order within a cell
+  std::vector<uint32_t> ids(rec_cells.size());
+  for (size_t r = 0; r < ids.size(); ++r) ids[r] = (uint32_t)r;
+  std::stable_sort(ids.begin(), ids.end(), [&](uint32_t x, uint32_t y) { return rec_cells[x] < rec_cells[y]; });
+  const size_t words = ((size_t)n + 31) / 32;
+  std::vector<uint32_t> has(words, 0u), cells, first;
+  for (size_t e = 0; e < ids.size(); ++e) {
+    const uint32_t c = (uint32_t)rec_cells[ids[e]];
+    if (cells.empty() || cells.back() != c) {
+      cells.push_back(c);
+      first.push_back((uint32_t)e);
+      has[c >> 5] |= 1u << (c & 31u);
+    }
+  }
+  first.push_back((uint32_t)ids.size());
+  inj_cells = (int)cells.size();
+  std::vector<uint32_t> all(std::move(has));
+  for (const auto *v : {&cells, &first, &ids}) all.insert(all.end(), v->begin(), v->end());
+  if (hipMalloc((void **)&d_inj, all.size() * sizeof(uint32_t)) != hipSuccess) {
+    d_inj = nullptr;
+    err = "adjoint buffers do not fit in device memory";
+    return BIOT_ERR_NOMEM;
+  }
+  if (hipMemcpy(d_inj, all.data(), all.size() * sizeof(uint32_t), hipMemcpyHostToDevice) != hipSuccess) {
+    err = "receiver map upload failed";
+    return BIOT_ERR_HIP;
+  }
   return BIOT_OK;
 }
 
@@ -170,16 +203,25 @@ void biot_handle::adj_args(AdjArgs &A) const
   // FP16T / FP16C residual arrays, FP16M's residual records (tau and p)
   const bool res = prec == BIOT_FP16T || prec == BIOT_FP16C || prec == BIOT_FP16M;
   A.loff = res ? state_lo_off() : 0;
-  A.lomask = res ? comp_fields(prec) : 0u;
   for (int ax = 0; ax < 3; ++ax) A.coff[ax] = state_off(1 + ax);
+  // the adjoint fields, the derivative adjoints, then the slab records (vector accesses: each
+  // block 256-byte aligned)
   char *lp = (char *)d_lam;
-  for (int f = 0; f < NFIELD; ++f) A.lam[f] = lp + (size_t)f * n * asz;
-  lp += (size_t)NFIELD * n * asz;
+  auto next = [&](size_t count) {
+    char *p = lp;
+    lp += count * asz;
+    return p;
+  };
+  for (auto &p : A.lam) p = next(n);
+  for (auto &p : A.gv) p = next(n);
+  for (auto &p : A.gt) p = next(n);
+  lp = (char *)d_lam + round256((size_t)(lp - (char *)d_lam));
   for (int ax = 0; ax < 3; ++ax) {
+    const size_t b = round256((size_t)NCARRY * slab[ax] * asz);
     A.lcarry[ax] = lp;
-    lp += (size_t)NCARRY * slab[ax] * asz;
+    A.gs[ax] = lp + b;
+    lp += 2 * b;
   }
-  for (int d = 0; d < 12; ++d) A.G[d] = lp + (size_t)d * n * asz;
   for (int k = 0; k < NKC; ++k) {
     A.grad[k] = d_grad + (size_t)k * n;
     A.gacc[k] = prec == BIOT_FP64 ? (void *)A.grad[k] : (void *)(d_gpart + (size_t)k * n);
@@ -206,7 +248,7 @@ void biot_handle::adj_args(AdjArgs &A) const
 }
 
 // The six gradient outputs go over the float partial sums (88 n bytes, flushed by now) or, on
-// FP64 handles, over the adjoint wavefields (200 n bytes, no longer read).  The parameters take
+// FP64 handles, over the adjoint wavefields (208 n bytes, no longer read).  The parameters take
 // 64 n bytes of their own, uploaded on the side stream while the sweep runs; where that does
 // not fit, they go over the adjoint wavefields once the sweep is done.
 int biot_handle::chain_buffers(double *&par_dev, double *&out)
@@ -238,15 +280,17 @@ int biot_handle::chain_buffers(double *&par_dev, double *&out)
 
 void biot_handle::inject_args(InjectArgs &I) const
 {
-  const size_t asz = prec == BIOT_FP64 ? 8 : 4;
   std::memset(&I, 0, sizeof I);
-  for (int f = 0; f < NFIELD; ++f) I.lam[f] = (char *)d_lam + (size_t)f * n * asz;
-  I.rec = (const int64_t *)d_rec;
+  I.has = d_inj;
+  I.cells = I.has + ((size_t)n + 31) / 32;
+  I.first = I.cells + inj_cells;
+  I.ids = I.first + inj_cells + 1;
+  I.ncells = inj_cells;
   I.nrec = nrec;
-  I.ncomp = ncomp;
+  for (auto &c : I.comp) c = -1;
   for (int c = 0; c < ncomp; ++c) {
-    I.comp[c] = comp[c];
-    I.scale[c] = fscale[comp[c]];  // traces hold scale x stored value
+    I.comp[comp[c]] = c;
+    I.scale[comp[c]] = fscale[comp[c]];
   }
   I.src = d_adjsrc;
   I.nt = nt_max;
@@ -258,12 +302,13 @@ void biot_handle::free_adjoint()
   for (void *p : ckpt)
     if (p) (void)hipFree(p);
   ckpt.clear();
-  ckpt_every = ckpt_nt = 0;
+  ckpt_every = ckpt_nt = room_every = room_nt = 0;
   if (prec == BIOT_FP16M && d_kpack) {  // the adjoint's coefficient copy of the last parameters
     (void)hipFree(d_kpack);
     d_kpack = nullptr;
   }
-  for (void **p : {&d_slots, &d_lam, (void **)&d_grad, (void **)&d_gpart, (void **)&d_adjsrc, (void **)&d_par})
+  for (void **p : {&d_slots, &d_lam, (void **)&d_grad, (void **)&d_gpart, (void **)&d_adjsrc, (void **)&d_par,
+                   (void **)&d_inj})
     if (*p) {
       (void)hipFree(*p);
       *p = nullptr;

@@ -103,6 +103,7 @@ struct biot_handle {
   std::vector<double> K_last[biot::NKC];     // kernel coefficients built from par
   std::vector<void *> ckpt;                  // checkpoint states, every ckpt_every steps
   int ckpt_every = 0, ckpt_nt = 0;
+  int room_every = 0, room_nt = 0;           // the run the buffers of ckpt were allocated for
   // ckpt_every == 1: ckpt[0] is one block of ckpt_nt + 1 states, state it being step it's
   // state after its source (the last one the state after the run), which the adjoint reads
   // in place of segment recomputation
@@ -111,6 +112,8 @@ struct biot_handle {
   double *d_grad = nullptr;                  // 22 FP64 coefficient gradients
   float *d_gpart = nullptr;                  // 22 float per-segment partial sums (not FP64 handles)
   float *d_adjsrc = nullptr;                 // adjoint source traces
+  uint32_t *d_inj = nullptr;                 // which cells hold which receivers (InjectArgs)
+  int inj_cells = 0;
   double *d_par = nullptr;                   // the 8 parameter arrays of par, for the chain rule
   hipStream_t side = nullptr;                // uploads beside a running sweep (made on first use)
   size_t state_bytes() const;
@@ -137,7 +140,8 @@ struct biot_handle {
   int clear_nonfinite();                     // enqueue a clear of d_flag on the stream
   int check_nonfinite();                     // synchronize; BIOT_ERR_NONFINITE if it was set
   size_t lam_bytes() const;                  // adjoint wavefields, carries, derivative adjoints
-  int alloc_adjoint(int every);              // d_slots (every+1 states; none for 0), d_lam, d_grad, d_adjsrc
+  int alloc_adjoint(int every);              // d_slots (every+1 states; none for 0), d_lam, d_grad, d_adjsrc, d_inj
+  int build_inject();                        // d_inj from rec_cells
   void adj_args(biot::AdjArgs &A) const;     // after alloc_adjoint
   // the device copy of par and room for the 6 parameter gradients, for work queued on the stream
   // after the sweep that is queued now
