@@ -579,13 +579,13 @@ extern "C" int biot_reset(biot_handle *h)
 // ride on the two half-step launches (FuseArgs); the run's first source and its last step's
 // stresses and p have launches of their own, and so have all of them where a receiver samples
 // what the source changes.
-int biot_handle::enqueue_steps(int nsteps, hipEvent_t *marks, char *states)
+int biot_handle::enqueue_steps(int nsteps, hipEvent_t *marks, char *states, bool recording)
 {
-  const size_t sb = states ? state_bytes() : 0;
+  const uint64_t sb = state_bytes();
   SourceArgs sa;
-  source_args(sa);
+  source_args(sa, states);
   RecordArgs ra;
-  record_args(ra);
+  record_args(ra, states);
   const bool src_fused = source_in_stress(), rec_fused = !source_recorded();
   auto failed = [&](hipError_t e, const char *what) {
     return e == hipSuccess ? BIOT_OK : fail(this, BIOT_ERR_HIP, "%s launch: %s", what, hipGetErrorString(e));
@@ -595,33 +595,44 @@ int biot_handle::enqueue_steps(int nsteps, hipEvent_t *marks, char *states)
     ra.it = step;
     ra.c0 = first;
     ra.c1 = last;
-    return d_traces && step >= 0 && step < nt_max && last > first ? &ra : nullptr;
+    return recording && d_traces && step >= 0 && step < nt_max && last > first ? &ra : nullptr;
   };
   const int nvel = ra.nvel;
 
   StepArgs args;
-  fill_args(args);
+  fill_args(args, states);
 
   int rc = BIOT_OK;
   for (int s = 0; s < nsteps && !rc; ++s) {
-    if ((s == 0 || !src_fused) && has_source(it)) {
+    const int q = states ? s : -1;
+    // out of place, a source cell that no half step writes takes its value along
+    const bool carry = states && sa.outside && s > 0 && d_wavelet && src_mask;
+    if (((s == 0 || !src_fused) && has_source(it)) || carry) {
       sa.it = it;
+      sa.ooff = states ? (uint64_t)s * sb : 0;
+      sa.ioff = carry ? sa.ooff - sb : sa.ooff;
       if ((rc = failed(launch_source(prec, sa, stream), "source"))) break;
     }
-    if (states) save_state(states + (size_t)s * sb);
     if (marks) (void)hipEventRecord(marks[3 * s], stream);
     const RecordArgs *before = rec_fused && s > 0 ? record(it - 1, nvel, ncomp) : nullptr;
-    if ((rc = failed(launch_velocity(prec, g.order, args, shape, stream, before), "velocity"))) break;
+    if ((rc = failed(launch_velocity(prec, g.order, args, shape, stream, before, q), "velocity"))) break;
     if (marks) (void)hipEventRecord(marks[3 * s + 1], stream);
     const bool next = src_fused && s + 1 < nsteps && has_source(it + 1);
     sa.it = it + 1;
-    if ((rc = failed(launch_stress(prec, g.order, args, shape, stream, record(it, 0, nvel), next ? &sa : nullptr),
+    if ((rc = failed(launch_stress(prec, g.order, args, shape, stream, record(it, 0, nvel), next ? &sa : nullptr, q),
                      "stress")))
       break;
     if (marks) (void)hipEventRecord(marks[3 * s + 2], stream);
+    ra.off = states ? (uint64_t)(s + 1) * sb : 0;
     if (!rec_fused || s + 1 == nsteps)
       if (const RecordArgs *r = record(it, nvel, ncomp)) rc = failed(launch_record(prec, *r, stream), "record");
     ++it;
+  }
+  if (!rc && states && nsteps > 0 && sa.outside && d_wavelet && src_mask) {
+    sa.it = (int)wavelet.size();  // past the wavelet: the value alone
+    sa.ooff = (uint64_t)nsteps * sb;
+    sa.ioff = sa.ooff - sb;
+    rc = failed(launch_source(prec, sa, stream), "source");
   }
   return rc;
 }

@@ -115,16 +115,19 @@ extern "C" int biot_forward_checkpointed(biot_handle *h, int32_t nt, int32_t eve
       if (hipMalloc(&p, bytes) != hipSuccess)
         return afail(h, BIOT_ERR_NOMEM, "the %d step states (%zu bytes) do not fit; use every > 1", nt + 1, bytes);
       h->ckpt.push_back(p);
+      if (int rc = h->clear_borders((char *)p, nt + 1)) return rc;
       h->room_every = 1;
       h->room_nt = nt;
     }
+    // the steps go from one state to the next, and the last one is the handle's
     char *p = (char *)h->ckpt[0];
     int rc = biot_reset(h);
     if (rc) return rc;
     AHIP(h, hipEventRecord(h->ev0, h->stream));
+    AHIP(h, hipMemsetAsync(p, 0, sb, h->stream));
     rc = h->enqueue_steps(nt, nullptr, p);
     if (rc) return rc;
-    h->save_state(p + (size_t)nt * sb);
+    h->load_state(p + (size_t)nt * sb);
     AHIP(h, hipEventRecord(h->ev1, h->stream));
     AHIP(h, hipEventSynchronize(h->ev1));
     float ms = 0;
@@ -213,13 +216,7 @@ extern "C" int biot_adjoint(biot_handle *h, const float *adj_source, double *con
   h->adj_args(A);
   InjectArgs I;
   h->inject_args(I);
-  SourceArgs sa;
-  h->source_args(sa);
-  StepArgs st;
-  h->fill_args(st);
-  const bool src_fused = h->source_in_stress();
   const size_t sb = h->state_bytes();
-  auto slot = [&](int q) { return (char *)h->d_slots + (size_t)q * sb; };
 
   // ---- backward sweep over the checkpoint segments
   AHIP(h, hipEventRecord(h->ev0, h->stream));
@@ -236,20 +233,13 @@ extern "C" int biot_adjoint(biot_handle *h, const float *adj_source, double *con
   const int nseg = stored ? 0 : (int)h->ckpt.size();
   for (int s = nseg - 1; s >= 0; --s) {
     const int n0 = s * every, K = std::min(every, nt - n0);
-    h->load_state(h->ckpt[s]);
-    for (int q = 0; q < K; ++q) {
-      const int it = n0 + q;
-      if ((q == 0 || !src_fused) && h->has_source(it)) {
-        sa.it = it;
-        AHIP(h, launch_source(h->prec, sa, h->stream));
-      }
-      h->save_state(slot(q));  // state of step it after its source
-      AHIP(h, launch_velocity(h->prec, order, st, h->shape, h->stream));
-      const bool next = src_fused && q + 1 < K && h->has_source(it + 1);
-      sa.it = it + 1;
-      AHIP(h, launch_stress(h->prec, order, st, h->shape, h->stream, nullptr, next ? &sa : nullptr));
-    }
-    h->save_state(slot(K));
+    // the segment's steps again, from state to state
+    AHIP(h, hipMemcpyAsync(h->d_slots, h->ckpt[s], sb, hipMemcpyDeviceToDevice, h->stream));
+    const int at = h->it;
+    h->it = n0;
+    rc = h->enqueue_steps(K, nullptr, (char *)h->d_slots, false);
+    h->it = at;
+    if (rc) return rc;
     for (int it = n0 + K - 1; it >= n0; --it) AHIP(h, launch_adjoint_step(h->prec, order, A, I, it - n0, it, h->stream));
     AHIP(h, launch_adjoint_flush(h->prec, order, A, h->stream));  // the segment's float partial sums
   }

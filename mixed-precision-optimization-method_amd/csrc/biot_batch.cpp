@@ -63,6 +63,8 @@ struct biot_batch {
   int *d_blocks = nullptr;
   InjectArgs *d_inj = nullptr;
   CopyEntry *d_copy = nullptr;
+  StepArgs *d_step_s = nullptr;    // d_step and d_src over the segment states
+  SourceArgs *d_src_s = nullptr;
   int adj_blocks = 0;
   double *d_gout = nullptr;        // 6 model-grid arrays
   double *d_J = nullptr;
@@ -140,6 +142,8 @@ void biot_batch::free_gradient()
   dfree(d_blocks);
   dfree(d_inj);
   dfree(d_copy);
+  dfree(d_step_s);
+  dfree(d_src_s);
   dfree(d_gout);
   dfree(d_J);
 }
@@ -367,6 +371,7 @@ BatchArgs batch_args(const biot_batch *b)
   a.src = b->fused ? b->d_src : nullptr;
   a.rec = b->d_rec;
   a.it = b->d_it;
+  a.q = -1;
   return a;
 }
 
@@ -380,7 +385,7 @@ int enqueue_step(biot_batch *b, bool record, int off)
   BatchArgs ba = batch_args(b);
   ba.off = off;
   const int64_t rec = record && b->fused ? b->max_nrec : 0;
-  if (!b->fused) BHIP(b, launch_source_batch(prec, b->d_src, b->nactive, b->d_it, off, b->stream));
+  if (!b->fused) BHIP(b, launch_source_batch(prec, b->d_src, b->nactive, b->d_it, off, -1, b->stream));
   BHIP(b, launch_step_batch(prec, order, true, ba, b->shape, b->blocks, rec, b->stream));
   BHIP(b, launch_step_batch(prec, order, false, ba, b->shape, b->blocks, rec, b->stream));
   if (record && !b->fused)
@@ -393,7 +398,7 @@ int start_steps(biot_batch *b, int it, int n)
 {
   BHIP(b, launch_set_counter(b->d_it, it, it + n, b->stream));
   if (b->fused)
-    BHIP(b, launch_source_batch(b->cfg.precision, b->d_src, b->nactive, b->d_it, 0, b->stream));
+    BHIP(b, launch_source_batch(b->cfg.precision, b->d_src, b->nactive, b->d_it, 0, -1, b->stream));
   return BIOT_OK;
 }
 // the counter is past the run's last step (off: its distance from the counter)
@@ -633,41 +638,48 @@ int gradient_group(biot_batch *b, int s0, int s1, int nt, int every, const float
     BHIP(b, hipMemcpy(b->d_adj, adj.data(), S * sizeof(AdjArgs), hipMemcpyHostToDevice));
     BHIP(b, hipMemcpy(b->d_blocks, bs.data(), (S + 1) * sizeof(int), hipMemcpyHostToDevice));
     BHIP(b, hipMemcpy(b->d_inj, inj.data(), S * sizeof(InjectArgs), hipMemcpyHostToDevice));
-  }
-  // copy tables: [save ckpt k] nseg, [load ckpt k] nseg, [save slot q] every + 1; 5 pieces per shot
-  // (fields, the three carry blocks, the FP16T / FP16C residuals: 0 bytes on the other policies)
-  constexpr int NP = 5;
-  const int per = NP * S;
-  auto pieces = [&](biot_handle *h, char *state, bool to_state, CopyEntry *e) {
-    char *live[NP] = {(char *)h->d_fields, (char *)h->d_carry[0], (char *)h->d_carry[1], (char *)h->d_carry[2],
-                      (char *)h->d_lo};
-    const size_t bytes[NP] = {(size_t)NFIELD * h->n * h->esz, (size_t)NCARRY * h->slab[0] * h->csz,
-                              (size_t)NCARRY * h->slab[1] * h->csz, (size_t)NCARRY * h->slab[2] * h->csz,
-                              h->d_lo ? h->lo_bytes() : 0};
-    for (int p = 0; p < NP; ++p) {
-      char *st = state + (p < 4 ? h->state_off(p) : h->state_lo_off());
-      e[p].src = to_state ? (const void *)live[p] : (const void *)st;
-      e[p].dst = to_state ? (void *)st : (void *)live[p];
-      e[p].bytes = bytes[p];
-    }
-  };
-  {
-    std::vector<CopyEntry> tab((size_t)(2 * nseg + every + 1) * per);
+    // the half steps' and sources' arguments over the segment states
+    std::vector<StepArgs> st(S);
+    std::vector<SourceArgs> src(S);
     for (int i = 0; i < S; ++i) {
       biot_handle *h = b->shots[s0 + i].h;
+      h->fill_args(st[i], (char *)h->d_slots);
+      set_tiles(st[i], b->shape, order / 2);
+      h->source_args(src[i], (char *)h->d_slots);
+    }
+    BHIP(b, hipMalloc((void **)&b->d_step_s, S * sizeof(StepArgs)));
+    BHIP(b, hipMalloc((void **)&b->d_src_s, S * sizeof(SourceArgs)));
+    BHIP(b, hipMemcpy(b->d_step_s, st.data(), S * sizeof(StepArgs), hipMemcpyHostToDevice));
+    BHIP(b, hipMemcpy(b->d_src_s, src.data(), S * sizeof(SourceArgs), hipMemcpyHostToDevice));
+  }
+  // copy tables: [save ckpt k] nseg entries of 5 pieces per shot (fields, the three carry blocks,
+  // the residuals: 0 bytes on the policies without), [ckpt k to the first segment state] nseg of one
+  constexpr int NP = 5;
+  const int per = NP * S;
+  {
+    std::vector<CopyEntry> tab((size_t)nseg * (per + S));
+    for (int i = 0; i < S; ++i) {
+      biot_handle *h = b->shots[s0 + i].h;
+      char *live[NP] = {(char *)h->d_fields, (char *)h->d_carry[0], (char *)h->d_carry[1], (char *)h->d_carry[2],
+                        (char *)h->d_lo};
+      const size_t bytes[NP] = {(size_t)NFIELD * h->n * h->esz, (size_t)NCARRY * h->slab[0] * h->csz,
+                                (size_t)NCARRY * h->slab[1] * h->csz, (size_t)NCARRY * h->slab[2] * h->csz,
+                                h->d_lo ? h->lo_bytes() : 0};
       for (int k = 0; k < nseg; ++k) {
-        pieces(h, (char *)b->shots[s0 + i].ckpt[k], true, &tab[(size_t)k * per + NP * i]);
-        pieces(h, (char *)b->shots[s0 + i].ckpt[k], false, &tab[(size_t)(nseg + k) * per + NP * i]);
+        char *ckpt = (char *)b->shots[s0 + i].ckpt[k];
+        for (int p = 0; p < NP; ++p)
+          tab[(size_t)k * per + NP * i + p] =
+              CopyEntry{live[p], ckpt + (p < 4 ? h->state_off(p) : h->state_lo_off()), bytes[p]};
+        tab[(size_t)nseg * per + (size_t)k * S + i] = CopyEntry{ckpt, h->d_slots, h->state_bytes()};
       }
-      for (int q = 0; q <= every; ++q)
-        pieces(h, (char *)h->d_slots + (size_t)q * h->state_bytes(), true, &tab[(size_t)(2 * nseg + q) * per + NP * i]);
     }
     BHIP(b, hipMalloc((void **)&b->d_copy, tab.size() * sizeof(CopyEntry)));
     BHIP(b, hipMemcpy(b->d_copy, tab.data(), tab.size() * sizeof(CopyEntry), hipMemcpyHostToDevice));
   }
   auto save_ckpt = [&](int k) { return launch_copy_batch(b->d_copy + (size_t)k * per, per, b->stream); };
-  auto load_ckpt = [&](int k) { return launch_copy_batch(b->d_copy + (size_t)(nseg + k) * per, per, b->stream); };
-  auto save_slot = [&](int q) { return launch_copy_batch(b->d_copy + (size_t)(2 * nseg + q) * per, per, b->stream); };
+  auto load_ckpt = [&](int k) {
+    return launch_copy_batch(b->d_copy + (size_t)nseg * per + (size_t)k * S, S, b->stream);
+  };
   for (int i = s0; i < s1; ++i) {
     int r = biot_reset(b->shots[i].h);
     if (r) return hfail(b, b->shots[i].h, r, "reset");
@@ -694,16 +706,18 @@ int gradient_group(biot_batch *b, int s0, int s1, int nt, int every, const float
   for (int k = nseg - 1; k >= 0; --k) {
     const int n0 = k * every, K = std::min(every, nt - n0);
     BHIP(b, load_ckpt(k));
-    if ((rc = start_steps(b, n0, K))) return rc;
+    // the segment's steps again, from state to state; a shot's source that no stress launch can
+    // add has every shot's added by launches of their own
+    BHIP(b, launch_set_counter(b->d_it, n0, n0 + K, b->stream));
     for (int q = 0; q < K; ++q) {
-      if (!b->fused) BHIP(b, launch_source_batch(prec, b->d_src, S, b->d_it, q, b->stream));
-      BHIP(b, save_slot(q));
+      if (q == 0 || !b->fused) BHIP(b, launch_source_batch(prec, b->d_src_s, S, b->d_it, q, q, b->stream));
       BatchArgs ba = batch_args(b);
-      ba.off = q;
+      ba.shots = b->d_step_s;
+      ba.src = b->fused ? b->d_src_s : nullptr;
+      ba.off = ba.q = q;
       BHIP(b, launch_step_batch(prec, order, true, ba, b->shape, b->blocks, 0, b->stream));
       BHIP(b, launch_step_batch(prec, order, false, ba, b->shape, b->blocks, 0, b->stream));
     }
-    BHIP(b, save_slot(K));
     for (int it = n0 + K - 1; it >= n0; --it) BHIP(b, launch_adjoint_step_batch(prec, order, ab, it - n0, it, b->stream));
     BHIP(b, launch_adjoint_flush_batch(prec, order, ab, b->stream));
   }
@@ -754,6 +768,8 @@ void free_group(biot_batch *b, int s0, int s1)
   dfree(b->d_blocks);
   dfree(b->d_inj);
   dfree(b->d_copy);
+  dfree(b->d_step_s);
+  dfree(b->d_src_s);
 }
 
 }  // namespace

@@ -122,6 +122,7 @@ struct StepArgs {
   int64_t sy, sz;            // strides
   int zchunk;
   int gx, gy, gz, ntiles;    // tile grid (x-y tiles of the block shape, z chunks)
+  uint64_t sb;               // a run of states: bytes from one to the next
   int xg;                    // consecutive tiles an XCD takes at a time (xcd_run)
   int src[3];                // the source cell (no cell's position: no source)
   int xy0;                   // one-row blocks: the plane cell the first tile starts at
@@ -184,8 +185,11 @@ struct SourceArgs {
   uint32_t mask;
   const float *wavelet;     // device, one sample per step
   int it;
-  int nt_w;                 // wavelet samples (batched launches check the step against it)
+  int nt_w;                 // wavelet samples
   float inv_scale[NFIELD];  // 1 / storage scale per field
+  int outside;              // no half step writes the cell
+  uint64_t sb;              // a run of states: bytes from one to the next
+  uint64_t ioff, ooff;      // single launches: where the value is read and stored, bytes on
 };
 struct RecordArgs {
   const void *f[NFIELD];
@@ -202,6 +206,7 @@ struct RecordArgs {
   int *nonfinite;           // device: the first step with a non-finite sample (NONFINITE_NONE:
                             // none so far), or null
   int it, nt_max;
+  uint64_t off;             // single launches: the state's place, bytes on
 };
 // A half step's launch also does the work around it that touches only fields it leaves alone:
 // the velocity launch records the stresses and p of the step before, the stress launch the
@@ -213,14 +218,19 @@ struct FuseArgs {
   int tile_blocks;          // blocks of the tiles (set by the launcher); the others record
   int record;               // rec holds something to record
   int source;               // src is to be added (stress launch)
+  int q;                    // state of a run of states (OOP)
   RecordArgs rec;
   SourceArgs src;
 };
-// rec (c0, c1 and it set; may be null), src (it set; stress launch; may be null): see FuseArgs
+// rec (c0, c1 and it set; may be null), src (it set; stress launch; may be null): see FuseArgs;
+// q >= 0: out of place, state q of the run of states at the arguments' pointers to state q + 1
 hipError_t launch_velocity(int prec, int order, const StepArgs &args, LaunchShape shape, hipStream_t s,
-                           const RecordArgs *rec = nullptr);
+                           const RecordArgs *rec = nullptr, int q = -1);
 hipError_t launch_stress(int prec, int order, const StepArgs &args, LaunchShape shape, hipStream_t s,
-                         const RecordArgs *rec = nullptr, const SourceArgs *src = nullptr);
+                         const RecordArgs *rec = nullptr, const SourceArgs *src = nullptr, int q = -1);
+// zero values outside the update box of nstates states (loff: the residuals' place in a state)
+hipError_t launch_clear_border(int prec, void *slots, int nstates, uint64_t sb, uint64_t loff, int h, int nx, int ny,
+                               int nz, hipStream_t s);
 // the byte pattern a cleared non-finite flag holds (every byte 0x7F): larger than any step
 constexpr int NONFINITE_NONE = 0x7F7F7F7F;
 hipError_t launch_source(int prec, const SourceArgs &a, hipStream_t s);
@@ -267,14 +277,16 @@ struct BatchArgs {
   const RecordArgs *rec;
   const int *it;
   int off, tile_blocks, rec_blocks;
+  int q;                    // >= 0: out of place, as launch_velocity's; one block per tile, no recording
 };
 // blocks: the persistent grid size (a multiple of 8); max_nrec: the most receivers a shot has
 // (0: record nothing)
 hipError_t launch_step_batch(int prec, int order, bool vel, const BatchArgs &b, LaunchShape sh,
                              int blocks, int64_t max_nrec, hipStream_t s);
-// the sources of step it[0] + off; the components of step it[0] + off (vel: the velocities too,
+// the sources of step it[0] + off (to state q of each shot's run of states, or in place for q < 0);
+// the components of step it[0] + off (vel: the velocities too,
 // else the stresses and p alone)
-hipError_t launch_source_batch(int prec, const SourceArgs *tab, int nshots, const int *it, int off,
+hipError_t launch_source_batch(int prec, const SourceArgs *tab, int nshots, const int *it, int off, int q,
                                hipStream_t s);
 hipError_t launch_record_batch(int prec, const RecordArgs *tab, int nshots, int64_t max_nrec,
                                bool vel, const int *it, int off, hipStream_t s);

@@ -46,26 +46,32 @@ void biot_handle::load_state(const void *src)
   }
 }
 
-void biot_handle::source_args(SourceArgs &sa) const
+void biot_handle::source_args(SourceArgs &sa, char *states) const
 {
   std::memset(&sa, 0, sizeof sa);
+  StepArgs a;
+  fill_args(a, states);
   for (int f = 0; f < NFIELD; ++f) {
-    sa.f[f] = field_ptr(f);
-    sa.lo[f] = lo_ptr(f);
+    sa.f[f] = a.f[f];
+    sa.lo[f] = a.lo[f];
     sa.inv_scale[f] = 1.0f / fscale[f];
   }
   sa.cell = src_cell;
   sa.mask = src_mask;
   sa.wavelet = (const float *)d_wavelet;
   sa.nt_w = (int)wavelet.size();
+  sa.outside = source_outside();
+  sa.sb = state_bytes();
 }
 
-void biot_handle::record_args(RecordArgs &ra) const
+void biot_handle::record_args(RecordArgs &ra, char *states) const
 {
   std::memset(&ra, 0, sizeof ra);
+  StepArgs a;
+  fill_args(a, states);
   for (int f = 0; f < NFIELD; ++f) {
-    ra.f[f] = field_ptr(f);
-    ra.lo[f] = lo_ptr(f);
+    ra.f[f] = a.f[f];
+    ra.lo[f] = a.lo[f];
   }
   ra.rec = (const int64_t *)d_rec;
   ra.nrec = nrec;
@@ -88,12 +94,16 @@ bool biot_handle::source_recorded() const
          std::find(rec_cells.begin(), rec_cells.end(), src_cell) != rec_cells.end();
 }
 
-bool biot_handle::source_in_stress() const
+bool biot_handle::source_outside() const
 {
-  if (!d_wavelet || !src_mask || (src_mask & 0x3Fu) || source_recorded()) return false;
   const int h = g.order / 2;
   const int64_t i = src_cell % g.nx, j = src_cell / g.nx % g.ny, k = src_cell / ((int64_t)g.nx * g.ny);
-  return i >= h && i < g.nx - h && j >= h && j < g.ny - h && k >= h && k < g.nz - h;
+  return !(i >= h && i < g.nx - h && j >= h && j < g.ny - h && k >= h && k < g.nz - h);
+}
+
+bool biot_handle::source_in_stress() const
+{
+  return d_wavelet && src_mask && !(src_mask & 0x3Fu) && !source_recorded() && !source_outside();
 }
 
 int biot_handle::clear_nonfinite()
@@ -136,6 +146,7 @@ int biot_handle::alloc_adjoint(int every)
   // 32-bit byte offsets from its base, as the forward kernels do their arrays
   const int64_t asz = prec == BIOT_FP64 ? 8 : 4, lim = (int64_t)1 << 32;
   bool fits = n * asz < lim;
+  const bool new_slots = every > 0 && !d_slots;
   for (int ax = 0; ax < 3; ++ax) fits = fits && NCARRY * slab[ax] * asz < lim;
   if (!fits) {
     err = "grid too large for the adjoint (an adjoint array would exceed 4 GiB)";
@@ -156,7 +167,19 @@ int biot_handle::alloc_adjoint(int every)
     err = "adjoint buffers do not fit in device memory";
     return BIOT_ERR_NOMEM;
   }
+  if (new_slots)
+    if (int rc = clear_borders((char *)d_slots, every + 1)) return rc;
   return build_inject();
+}
+
+int biot_handle::clear_borders(char *states, int nstates)
+{
+  if (launch_clear_border(prec, states, nstates, state_bytes(), state_lo_off(), g.order / 2, g.nx, g.ny, g.nz,
+                          stream) == hipSuccess &&
+      hipStreamSynchronize(stream) == hipSuccess)
+    return BIOT_OK;
+  err = "clearing the states' outer cells failed";
+  return BIOT_ERR_HIP;
 }
 
 int biot_handle::build_inject()
@@ -365,13 +388,18 @@ int8_t *biot_handle::lo_ptr(int f) const
   return d_lo + (size_t)f * n;
 }
 
-void biot_handle::fill_args(StepArgs &a) const
+void biot_handle::fill_args(StepArgs &a, char *states) const
 {
   std::memset(&a, 0, sizeof a);
   for (int f = 0; f < NFIELD; ++f) {
     a.f[f] = field_ptr(f);
     a.lo[f] = lo_ptr(f);
+    if (states) {
+      a.f[f] = states + (size_t)f * n * esz;
+      if (a.lo[f]) a.lo[f] = (int8_t *)states + state_lo_off() + (a.lo[f] - d_lo);
+    }
   }
+  a.sb = state_bytes();
   for (int k = 0; k < NKC; ++k) {
     a.k[k] = (const char *)d_coef + (size_t)k * n * esz;
     a.ks[k] = ks[k];
@@ -386,7 +414,7 @@ void biot_handle::fill_args(StepArgs &a) const
     for (int q = 0; q < NMC; ++q) a.mc[q] = mc[q];
   }
   for (int ax = 0; ax < 3; ++ax) {
-    a.carry[ax] = d_carry[ax];
+    a.carry[ax] = states ? states + state_off(1 + ax) : (char *)d_carry[ax];
     a.slab[ax] = slab[ax];
     a.L[ax] = L[ax];
     a.R[ax] = R[ax];

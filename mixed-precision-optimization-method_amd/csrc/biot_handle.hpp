@@ -86,7 +86,8 @@ struct biot_handle {
   {
     return prec == BIOT_FP16 || prec == BIOT_FP16C || prec == BIOT_FP16T || prec == BIOT_FP16M;
   }
-  void fill_args(biot::StepArgs &a) const;
+  // the arguments over the handle's own arrays, or over the first of a run of states
+  void fill_args(biot::StepArgs &a, char *states = nullptr) const;
   int allocate();
   int upload_profiles();
   int upload_coefficients();
@@ -107,7 +108,7 @@ struct biot_handle {
   // ckpt_every == 1: ckpt[0] is one block of ckpt_nt + 1 states, state it being step it's
   // state after its source (the last one the state after the run), which the adjoint reads
   // in place of segment recomputation
-  void *d_slots = nullptr;                   // segment states (ckpt_every + 1)
+  void *d_slots = nullptr;                   // segment states (ckpt_every + 1), zero outside the update box
   void *d_lam = nullptr;                     // adjoint fields, carries, derivative adjoints
   double *d_grad = nullptr;                  // 22 FP64 coefficient gradients
   float *d_gpart = nullptr;                  // 22 float per-segment partial sums (not FP64 handles)
@@ -124,12 +125,15 @@ struct biot_handle {
   void free_adjoint();
   void forget_model();  // drop parameter-built coefficients and every adjoint buffer
   // marks: null, or 3 events per step recorded before velocity, between, after stress;
-  // states: null, or room for nsteps states, step s's state saved after its source
-  int enqueue_steps(int nsteps, hipEvent_t *marks, char *states = nullptr);
+  // states: null (in place), or a run of nsteps + 1 states, the first given: step s goes from state s,
+  // to which its source is added, to state s + 1.  record: false leaves the traces alone.
+  int enqueue_steps(int nsteps, hipEvent_t *marks, char *states = nullptr, bool record = true);
+  int clear_borders(char *states, int nstates);  // once for new states; on the stream
 
   // argument blocks shared by the single-grid and batched drivers
-  void source_args(biot::SourceArgs &sa) const;
-  void record_args(biot::RecordArgs &ra) const;  // every component
+  void source_args(biot::SourceArgs &sa, char *states = nullptr) const;
+  bool source_outside() const;               // no half step writes the source cell
+  void record_args(biot::RecordArgs &ra, char *states = nullptr) const;  // every component
   bool has_source(int step) const { return d_wavelet && src_mask && step < (int)wavelet.size(); }
   // whether a receiver records a stress or p at the source cell that the source changes: it then
   // has to be sampled before the next step's source is added

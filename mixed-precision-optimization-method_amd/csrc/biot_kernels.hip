@@ -242,19 +242,43 @@ __device__ __forceinline__ void store_raw(void *f, int8_t *lo, bool comp_f, u32 
     }
   }
 }
-template <class P, class AT>
-__device__ __forceinline__ typename P::A load_rt(const AT &a, int f, u32 idx)
+// One time-stepping state seen from a kernel: the arrays at the arguments' pointers (in place), or,
+// out of place (OOP), `off` bytes on: the kernel reads one state of a run of them and writes the
+// next.
+template <class AT, bool OOP>
+struct View {
+  const AT &a;
+  uint64_t off;
+  __device__ __forceinline__ void *f(int F) const
+  {
+    if constexpr (OOP) return reinterpret_cast<char *>(a.f[F]) + off;
+    else return a.f[F];
+  }
+  __device__ __forceinline__ int8_t *lo(int F) const
+  {
+    if constexpr (OOP) return a.lo[F] + off;
+    else return a.lo[F];
+  }
+  __device__ __forceinline__ void *carry(int ax) const
+  {
+    if constexpr (OOP) return reinterpret_cast<char *>(a.carry[ax]) + off;
+    else return a.carry[ax];
+  }
+};
+
+template <class P, class V>
+__device__ __forceinline__ typename P::A load_rt(const V &v, int f, u32 idx)
 {
-  return load_raw<P>(a.f[f], a.lo[f], (P::cmask >> f) & 1u, idx);
+  return load_raw<P>(v.f(f), v.lo(f), (P::cmask >> f) & 1u, idx);
 }
 // compile-time field index: the residual test folds away
 // (FP16M's tau and p read the whole residual record, from the base that field PK_FIRST's
 // pointer holds, so the fields of one stencil point share one record load)
-template <class P, int F, class AT>
-__device__ __forceinline__ typename P::A L(const AT &a, u32 idx)
+template <class P, int F, class V>
+__device__ __forceinline__ typename P::A L(const V &v, u32 idx)
 {
-  if constexpr (P::packed && ((PK_FIELDS >> F) & 1u)) return pk_at<F>(a.f[F], a.lo[PK_FIRST], idx);
-  else return load_rt<P>(a, F, idx);
+  if constexpr (P::packed && ((PK_FIELDS >> F) & 1u)) return pk_at<F>(v.f(F), v.lo(PK_FIRST), idx);
+  else return load_rt<P>(v, F, idx);
 }
 // FP16M and FP16T read their tau and p at a 4th-order stencil's outer taps (the pair with
 // weight 1/24 against the inner pair's 9/8) as the binary16 part, without the residual
@@ -263,22 +287,22 @@ template <class P, int F>
 constexpr bool outer16 = P::outer16 && ((P::cmask >> F) & 1u);
 // the value of field F at an outer tap: the binary16 part of FP16M's and FP16T's tau and p,
 // the full value of every other field
-template <class P, int F, class AT>
-__device__ __forceinline__ typename P::A LF(const AT &a, u32 idx)
+template <class P, int F, class V>
+__device__ __forceinline__ typename P::A LF(const V &v, u32 idx)
 {
-  if constexpr (outer16<P, F>) return pk_hi(a.f[F], idx);
-  else return L<P, F>(a, idx);
+  if constexpr (outer16<P, F>) return pk_hi(v.f(F), idx);
+  else return L<P, F>(v, idx);
 }
-template <class P, int F, bool NT, class AT>
-__device__ __forceinline__ typename P::A LO(const AT &a, u32 idx)
+template <class P, int F, bool NT, class V>
+__device__ __forceinline__ typename P::A LO(const V &v, u32 idx)
 {
-  if constexpr (P::packed && ((PK_FIELDS >> F) & 1u)) return pk_at<F>(a.f[F], a.lo[PK_FIRST], idx);
-  else return load_own<P, NT>(a.f[F], a.lo[F], (P::cmask >> F) & 1u, idx);
+  if constexpr (P::packed && ((PK_FIELDS >> F) & 1u)) return pk_at<F>(v.f(F), v.lo(PK_FIRST), idx);
+  else return load_own<P, NT>(v.f(F), v.lo(F), (P::cmask >> F) & 1u, idx);
 }
-template <class P, int F, bool NT, class AT>
-__device__ __forceinline__ void ST(const AT &a, u32 idx, typename P::A x)
+template <class P, int F, bool NT, class V>
+__device__ __forceinline__ void ST(const V &v, u32 idx, typename P::A x)
 {
-  store_raw<P, NT>(a.f[F], a.lo[F], (P::cmask >> F) & 1u, idx, x);
+  store_raw<P, NT>(v.f(F), v.lo(F), (P::cmask >> F) & 1u, idx, x);
 }
 
 // staggered difference across the centre of a 2h-point window w[0..2h-1]
@@ -293,38 +317,38 @@ __device__ __forceinline__ A dwin(const A *w)
 }
 
 // forward difference of field F at c + s/2 (value at c supplied)
-template <class P, int F, int ORDER, class AT>
-__device__ __forceinline__ typename P::A dfw(const AT &a, u32 c, u32 s, typename P::A fc)
+template <class P, int F, int ORDER, class V>
+__device__ __forceinline__ typename P::A dfw(const V &v, u32 c, u32 s, typename P::A fc)
 {
   using A = typename P::A;
   if constexpr (ORDER == 2) {
-    return L<P, F>(a, c + s) - fc;
+    return L<P, F>(v, c + s) - fc;
   } else {
     if constexpr (outer16<P, F>) {
       // FP16M, FP16T: both outer taps (c + 2s, c - s) as binary16, each an fma on the binary16 value
-      const float o2 = (float)at<_Float16>(a.f[F], c + 2 * s), o1 = (float)at<_Float16>(a.f[F], c - s);
-      return fmaf(A(-1.0 / 24.0), o2, fmaf(A(1.0 / 24.0), o1, A(9.0 / 8.0) * (L<P, F>(a, c + s) - fc)));
+      const float o2 = (float)at<_Float16>(v.f(F), c + 2 * s), o1 = (float)at<_Float16>(v.f(F), c - s);
+      return fmaf(A(-1.0 / 24.0), o2, fmaf(A(1.0 / 24.0), o1, A(9.0 / 8.0) * (L<P, F>(v, c + s) - fc)));
     } else {
-      return A(9.0 / 8.0) * (L<P, F>(a, c + s) - fc) +
-             A(-1.0 / 24.0) * (L<P, F>(a, c + 2 * s) - L<P, F>(a, c - s));
+      return A(9.0 / 8.0) * (L<P, F>(v, c + s) - fc) +
+             A(-1.0 / 24.0) * (L<P, F>(v, c + 2 * s) - L<P, F>(v, c - s));
     }
   }
 }
 // backward difference of field F at c - s/2 (value at c supplied)
-template <class P, int F, int ORDER, class AT>
-__device__ __forceinline__ typename P::A dbw(const AT &a, u32 c, u32 s, typename P::A fc)
+template <class P, int F, int ORDER, class V>
+__device__ __forceinline__ typename P::A dbw(const V &v, u32 c, u32 s, typename P::A fc)
 {
   using A = typename P::A;
   if constexpr (ORDER == 2) {
-    return fc - L<P, F>(a, c - s);
+    return fc - L<P, F>(v, c - s);
   } else {
     if constexpr (outer16<P, F>) {
       // FP16M, FP16T: both outer taps (c + s, c - 2s) as binary16, each an fma on the binary16 value
-      const float o1 = (float)at<_Float16>(a.f[F], c + s), o2 = (float)at<_Float16>(a.f[F], c - 2 * s);
-      return fmaf(A(-1.0 / 24.0), o1, fmaf(A(1.0 / 24.0), o2, A(9.0 / 8.0) * (fc - L<P, F>(a, c - s))));
+      const float o1 = (float)at<_Float16>(v.f(F), c + s), o2 = (float)at<_Float16>(v.f(F), c - 2 * s);
+      return fmaf(A(-1.0 / 24.0), o1, fmaf(A(1.0 / 24.0), o2, A(9.0 / 8.0) * (fc - L<P, F>(v, c - s))));
     } else {
-      return A(9.0 / 8.0) * (fc - L<P, F>(a, c - s)) +
-             A(-1.0 / 24.0) * (L<P, F>(a, c + s) - L<P, F>(a, c - 2 * s));
+      return A(9.0 / 8.0) * (fc - L<P, F>(v, c - s)) +
+             A(-1.0 / 24.0) * (L<P, F>(v, c + s) - L<P, F>(v, c - 2 * s));
     }
   }
 }
@@ -512,10 +536,11 @@ enum { FVX = 0, FVY, FVZ, FQX, FQY, FQZ, FTXX, FTYY, FTZZ, FTXY, FTXZ, FTYZ, FP 
 // one x-y tile of the update box, planes kb..ke-1 of z chunk tz
 // NT: the launch allows the policy's nontemporal accesses (the single-grid kernels; the
 // batched kernels, whose shot windows are reused from the caches, do not)
-template <class P, int ORDER, bool NT, class AT>
-__device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int tz)
+template <class P, int ORDER, bool NT, bool OOP, class AT>
+__device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int tz, uint64_t ioff, uint64_t ooff)
 {
   using A = typename P::A;
+  const View<AT, OOP> vi{a, ioff}, vo{a, ooff};
   constexpr int h = ORDER / 2;
   constexpr int W = 2 * h;
   int i, j;
@@ -554,14 +579,14 @@ __device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int t
   A wxz[W], wyz[W], wzz[W], wp[W];
 #pragma unroll
   for (int m = 0; m < W - 1; ++m) {
-    wxz[m] = L<P, FTXZ>(a, col + (u32)(kb - h + m) * sz);
-    wyz[m] = L<P, FTYZ>(a, col + (u32)(kb - h + m) * sz);
+    wxz[m] = L<P, FTXZ>(vi, col + (u32)(kb - h + m) * sz);
+    wyz[m] = L<P, FTYZ>(vi, col + (u32)(kb - h + m) * sz);
     if (zrec && m == W - 2) {
-      wzz[m] = LF<P, FTZZ>(a, col + (u32)(kb - h + 1 + m) * sz);
-      wp[m] = LF<P, FP>(a, col + (u32)(kb - h + 1 + m) * sz);
+      wzz[m] = LF<P, FTZZ>(vi, col + (u32)(kb - h + 1 + m) * sz);
+      wp[m] = LF<P, FP>(vi, col + (u32)(kb - h + 1 + m) * sz);
     } else {
-      wzz[m] = L<P, FTZZ>(a, col + (u32)(kb - h + 1 + m) * sz);
-      wp[m] = L<P, FP>(a, col + (u32)(kb - h + 1 + m) * sz);
+      wzz[m] = L<P, FTZZ>(vi, col + (u32)(kb - h + 1 + m) * sz);
+      wp[m] = L<P, FP>(vi, col + (u32)(kb - h + 1 + m) * sz);
     }
   }
 
@@ -571,7 +596,7 @@ __device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int t
   if constexpr (P::medium) mown = med_rec(a.mv, col + (u32)kb * sz);
   // FP16M at order 4: the cell's residual record, rotated along z like the moduli record
   u32 rown = 0u;
-  if constexpr (zrec) rown = at<u32>(a.lo[PK_FIRST], col + (u32)kb * sz);
+  if constexpr (zrec) rown = at<u32>(vi.lo(PK_FIRST), col + (u32)kb * sz);
 
   // Every load of a plane is written before the plane's first store.  The compiler cannot
   // prove the arrays distinct, so it never moves a load above a store; in this order all of
@@ -589,41 +614,41 @@ __device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int t
         // plane and the forward windows' plane k+1 (read as its binary16 part a plane
         // earlier), and is the next plane's own record.  The forward windows' new plane k+2
         // is an outer tap: its binary16 part.
-        const u32 r1 = at<u32>(a.lo[PK_FIRST], c + sz);
-        wxz[W - 1] = pk_rec<FTXZ>(a.f[FTXZ], r1, c + sz);
-        wyz[W - 1] = pk_rec<FTYZ>(a.f[FTYZ], r1, c + sz);
+        const u32 r1 = at<u32>(vi.lo(PK_FIRST), c + sz);
+        wxz[W - 1] = pk_rec<FTXZ>(vi.f(FTXZ), r1, c + sz);
+        wyz[W - 1] = pk_rec<FTYZ>(vi.f(FTYZ), r1, c + sz);
         wzz[W - 2] = pk_fill<FTZZ>(wzz[W - 2], r1);
         wp[W - 2] = pk_fill<FP>(wp[W - 2], r1);
-        wzz[W - 1] = pk_hi(a.f[FTZZ], c + 2u * sz);
-        wp[W - 1] = pk_hi(a.f[FP], c + 2u * sz);
-        txx_c = pk_rec<FTXX>(a.f[FTXX], rown, c);
-        tyy_c = pk_rec<FTYY>(a.f[FTYY], rown, c);
-        txy_c = pk_rec<FTXY>(a.f[FTXY], rown, c);
+        wzz[W - 1] = pk_hi(vi.f(FTZZ), c + 2u * sz);
+        wp[W - 1] = pk_hi(vi.f(FP), c + 2u * sz);
+        txx_c = pk_rec<FTXX>(vi.f(FTXX), rown, c);
+        tyy_c = pk_rec<FTYY>(vi.f(FTYY), rown, c);
+        txy_c = pk_rec<FTXY>(vi.f(FTXY), rown, c);
         rown = r1;
       } else {
-        wxz[W - 1] = L<P, FTXZ>(a, c + (u32)(h - 1) * sz);
-        wyz[W - 1] = L<P, FTYZ>(a, c + (u32)(h - 1) * sz);
-        wzz[W - 1] = L<P, FTZZ>(a, c + (u32)h * sz);
-        wp[W - 1] = L<P, FP>(a, c + (u32)h * sz);
-        txx_c = L<P, FTXX>(a, c), tyy_c = L<P, FTYY>(a, c), txy_c = L<P, FTXY>(a, c);
+        wxz[W - 1] = L<P, FTXZ>(vi, c + (u32)(h - 1) * sz);
+        wyz[W - 1] = L<P, FTYZ>(vi, c + (u32)(h - 1) * sz);
+        wzz[W - 1] = L<P, FTZZ>(vi, c + (u32)h * sz);
+        wp[W - 1] = L<P, FP>(vi, c + (u32)h * sz);
+        txx_c = L<P, FTXX>(vi, c), tyy_c = L<P, FTYY>(vi, c), txy_c = L<P, FTXY>(vi, c);
       }
       const A txz_c = wxz[h], tyz_c = wyz[h], p_c = wp[h - 1];
-      x1 = dfw<P, FTXX, ORDER>(a, c, 1u, txx_c);
-      x2 = dbw<P, FTXY, ORDER>(a, c, sy, txy_c);
+      x1 = dfw<P, FTXX, ORDER>(vi, c, 1u, txx_c);
+      x2 = dbw<P, FTXY, ORDER>(vi, c, sy, txy_c);
       x3 = dwin<ORDER>(wxz);
-      s1 = dfw<P, FP, ORDER>(a, c, 1u, p_c);
-      y1 = dfw<P, FTYY, ORDER>(a, c, sy, tyy_c);
-      y2 = dbw<P, FTXY, ORDER>(a, c, 1u, txy_c);
+      s1 = dfw<P, FP, ORDER>(vi, c, 1u, p_c);
+      y1 = dfw<P, FTYY, ORDER>(vi, c, sy, tyy_c);
+      y2 = dbw<P, FTXY, ORDER>(vi, c, 1u, txy_c);
       y3 = dwin<ORDER>(wyz);
-      s2 = dfw<P, FP, ORDER>(a, c, sy, p_c);
+      s2 = dfw<P, FP, ORDER>(vi, c, sy, p_c);
       z1 = dwin<ORDER>(wzz);
-      z2 = dbw<P, FTXZ, ORDER>(a, c, 1u, txz_c);
-      z3 = dbw<P, FTYZ, ORDER>(a, c, sy, tyz_c);
+      z2 = dbw<P, FTXZ, ORDER>(vi, c, 1u, txz_c);
+      z3 = dbw<P, FTYZ, ORDER>(vi, c, sy, tyz_c);
       s3 = dwin<ORDER>(wp);
     }
 
-    const A qx0 = LO<P, FQX, (P::nt_v && NT)>(a, c), qy0 = LO<P, FQY, (P::nt_v && NT)>(a, c), qz0 = LO<P, FQZ, (P::nt_v && NT)>(a, c);
-    const A vx0 = LO<P, FVX, (P::nt_v && NT)>(a, c), vy0 = LO<P, FVY, (P::nt_v && NT)>(a, c), vz0 = LO<P, FVZ, (P::nt_v && NT)>(a, c);
+    const A qx0 = LO<P, FQX, (P::nt_v && NT)>(vi, c), qy0 = LO<P, FQY, (P::nt_v && NT)>(vi, c), qz0 = LO<P, FQZ, (P::nt_v && NT)>(vi, c);
+    const A vx0 = LO<P, FVX, (P::nt_v && NT)>(vi, c), vy0 = LO<P, FVY, (P::nt_v && NT)>(vi, c), vz0 = LO<P, FVZ, (P::nt_v && NT)>(vi, c);
     A kv[14];  // K[0..13]: U1 xyz, U2 xyz, W1 xyz, W2 xyz, W3x, W3y
     dw2_t mn[3];
     if constexpr (P::medium) {
@@ -650,38 +675,38 @@ __device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int t
     A ezi = 0, azi = 0, ezh = 0, azh = 0;
     if (px >= 0) {
       ox = (u32)px + wxs * ((u32)j + ny * (u32)k);
-      carry_load(cx, a.carry[0], 0u, ox, sl0);
+      carry_load(cx, vi.carry(0), 0u, ox, sl0);
     }
     if (py >= 0) {
       oy = (u32)i + nx * ((u32)py + wys * (u32)k);
-      carry_load(cy, a.carry[1], 0u, oy, sl1);
+      carry_load(cy, vi.carry(1), 0u, oy, sl1);
     }
     if (pz >= 0) {
       ezi = prof<A>(a.prof[2][0], k), azi = prof<A>(a.prof[2][1], k);
       ezh = prof<A>(a.prof[2][2], k), azh = prof<A>(a.prof[2][3], k);
       oz = (u32)i + nx * ((u32)j + ny * (u32)pz);
-      carry_load(cz, a.carry[2], 0u, oz, sl2);
+      carry_load(cz, vi.carry(2), 0u, oz, sl2);
     }
     if (px >= 0) {
       x1 = pml<P>(cx[0], x1, exh, axh);
       s1 = pml<P>(cx[1], s1, exh, axh);
       y2 = pml<P>(cx[2], y2, exi, axi);
       z2 = pml<P>(cx[3], z2, exi, axi);
-      carry_store(cx, a.carry[0], 0u, ox, sl0);
+      carry_store(cx, vo.carry(0), 0u, ox, sl0);
     }
     if (py >= 0) {
       x2 = pml<P>(cy[0], x2, eyi, ayi);
       y1 = pml<P>(cy[1], y1, eyh, ayh);
       s2 = pml<P>(cy[2], s2, eyh, ayh);
       z3 = pml<P>(cy[3], z3, eyi, ayi);
-      carry_store(cy, a.carry[1], 0u, oy, sl1);
+      carry_store(cy, vo.carry(1), 0u, oy, sl1);
     }
     if (pz >= 0) {
       x3 = pml<P>(cz[0], x3, ezi, azi);
       y3 = pml<P>(cz[1], y3, ezi, azi);
       z1 = pml<P>(cz[2], z1, ezh, azh);
       s3 = pml<P>(cz[3], s3, ezh, azh);
-      carry_store(cz, a.carry[2], 0u, oz, sl2);
+      carry_store(cz, vo.carry(2), 0u, oz, sl2);
     }
 
     // relative fluid velocity (kernel.cu:218-220; qz takes W3y as the reference does) and
@@ -690,16 +715,16 @@ __device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int t
     const A qx1 = w1x * qx0 - w2x * sx - w3x * s1;
     const A qy1 = w1y * qy0 - w2y * sy_ - w3y * s2;
     const A qz1 = w1z * qz0 - w2z * sz_ - w3y * s3;
-    ST<P, FQX, (P::nt_v && NT)>(a, c, qx1);
-    ST<P, FQY, (P::nt_v && NT)>(a, c, qy1);
-    ST<P, FQZ, (P::nt_v && NT)>(a, c, qz1);
+    ST<P, FQX, (P::nt_v && NT)>(vo, c, qx1);
+    ST<P, FQY, (P::nt_v && NT)>(vo, c, qy1);
+    ST<P, FQZ, (P::nt_v && NT)>(vo, c, qz1);
     // the solid update sees q as stored (rounded), as the reference re-reads it; q is
     // never a compensated field, so the stored value is the plain storage rounding
     using S = typename P::S;
     const A qx1s = (A)(S)qx1, qy1s = (A)(S)qy1, qz1s = (A)(S)qz1;
-    ST<P, FVX, (P::nt_v && NT)>(a, c, vx0 + u1x * sx - u2x * (qx1s - qx0));
-    ST<P, FVY, (P::nt_v && NT)>(a, c, vy0 + u1y * sy_ - u2y * (qy1s - qy0));
-    ST<P, FVZ, (P::nt_v && NT)>(a, c, vz0 + u1z * sz_ - u2z * (qz1s - qz0));
+    ST<P, FVX, (P::nt_v && NT)>(vo, c, vx0 + u1x * sx - u2x * (qx1s - qx0));
+    ST<P, FVY, (P::nt_v && NT)>(vo, c, vy0 + u1y * sy_ - u2y * (qy1s - qy0));
+    ST<P, FVZ, (P::nt_v && NT)>(vo, c, vz0 + u1z * sz_ - u2z * (qz1s - qz0));
 
 #pragma unroll
     for (int m = 0; m < W - 1; ++m) {
@@ -716,10 +741,12 @@ __device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int t
 
 // one x-y tile of the update box, planes kb..ke-1 of z chunk tz; true in the thread that updated
 // the source cell
-template <class P, int ORDER, bool NT, class AT>
-__device__ __forceinline__ bool stress_tile(const AT &a, int tx, int ty, int tz)
+template <class P, int ORDER, bool NT, bool OOP, class AT>
+__device__ __forceinline__ bool stress_tile(const AT &a, int tx, int ty, int tz, uint64_t ioff, uint64_t ooff)
 {
   using A = typename P::A;
+  // the velocities of the step's own velocity half are in the state written
+  const View<AT, OOP> vi{a, ioff}, vo{a, ooff};
   constexpr int h = ORDER / 2;
   constexpr int W = 2 * h;
   int i, j;
@@ -755,10 +782,10 @@ __device__ __forceinline__ bool stress_tile(const AT &a, int tx, int ty, int tz)
   A wvz[W], wqz[W], wvx[W], wvy[W];
 #pragma unroll
   for (int m = 0; m < W - 1; ++m) {
-    wvz[m] = L<P, FVZ>(a, col + (u32)(kb - h + m) * sz);
-    wqz[m] = L<P, FQZ>(a, col + (u32)(kb - h + m) * sz);
-    wvx[m] = L<P, FVX>(a, col + (u32)(kb - h + 1 + m) * sz);
-    wvy[m] = L<P, FVY>(a, col + (u32)(kb - h + 1 + m) * sz);
+    wvz[m] = L<P, FVZ>(vo, col + (u32)(kb - h + m) * sz);
+    wqz[m] = L<P, FQZ>(vo, col + (u32)(kb - h + m) * sz);
+    wvx[m] = L<P, FVX>(vo, col + (u32)(kb - h + 1 + m) * sz);
+    wvy[m] = L<P, FVY>(vo, col + (u32)(kb - h + 1 + m) * sz);
   }
 
   // FP16M: the mu quad of the first plane, advanced along z by medium_stress
@@ -769,30 +796,30 @@ __device__ __forceinline__ bool stress_tile(const AT &a, int tx, int ty, int tz)
   using SC = typename P::SC;
   for (int k = kb; k < ke; ++k) {
     const u32 c = col + (u32)k * sz;
-    wvz[W - 1] = L<P, FVZ>(a, c + (u32)(h - 1) * sz);
-    wqz[W - 1] = L<P, FQZ>(a, c + (u32)(h - 1) * sz);
-    wvx[W - 1] = L<P, FVX>(a, c + (u32)h * sz);
-    wvy[W - 1] = L<P, FVY>(a, c + (u32)h * sz);
+    wvz[W - 1] = L<P, FVZ>(vo, c + (u32)(h - 1) * sz);
+    wqz[W - 1] = L<P, FQZ>(vo, c + (u32)(h - 1) * sz);
+    wvx[W - 1] = L<P, FVX>(vo, c + (u32)h * sz);
+    wvy[W - 1] = L<P, FVY>(vo, c + (u32)h * sz);
     const A vz_c = wvz[h], vx_c = wvx[h - 1], vy_c = wvy[h - 1];
-    const A qx_c = L<P, FQX>(a, c), qy_c = L<P, FQY>(a, c);
+    const A qx_c = L<P, FQX>(vo, c), qy_c = L<P, FQY>(vo, c);
 
     // twelve raw differences (kernel.cu:430-445 without 1/dx)
-    A uxx = dbw<P, FVX, ORDER>(a, c, 1u, vx_c);
-    A uyy = dbw<P, FVY, ORDER>(a, c, sy, vy_c);
+    A uxx = dbw<P, FVX, ORDER>(vo, c, 1u, vx_c);
+    A uyy = dbw<P, FVY, ORDER>(vo, c, sy, vy_c);
     A uzz = dwin<ORDER>(wvz);
-    A wx = dbw<P, FQX, ORDER>(a, c, 1u, qx_c);
-    A wy = dbw<P, FQY, ORDER>(a, c, sy, qy_c);
+    A wx = dbw<P, FQX, ORDER>(vo, c, 1u, qx_c);
+    A wy = dbw<P, FQY, ORDER>(vo, c, sy, qy_c);
     A wz = dwin<ORDER>(wqz);
-    A uxy = dfw<P, FVX, ORDER>(a, c, sy, vx_c);
-    A uyx = dfw<P, FVY, ORDER>(a, c, 1u, vy_c);
+    A uxy = dfw<P, FVX, ORDER>(vo, c, sy, vx_c);
+    A uyx = dfw<P, FVY, ORDER>(vo, c, 1u, vy_c);
     A uxz = dwin<ORDER>(wvx);
-    A uzx = dfw<P, FVZ, ORDER>(a, c, 1u, vz_c);
+    A uzx = dfw<P, FVZ, ORDER>(vo, c, 1u, vz_c);
     A uyz = dwin<ORDER>(wvy);
-    A uzy = dfw<P, FVZ, ORDER>(a, c, sy, vz_c);
+    A uzy = dfw<P, FVZ, ORDER>(vo, c, sy, vz_c);
 
-    const A p0 = LO<P, FP, (P::nt_t && NT)>(a, c), txx0 = LO<P, FTXX, (P::nt_t && NT)>(a, c), tyy0 = LO<P, FTYY, (P::nt_t && NT)>(a, c);
-    const A tzz0 = LO<P, FTZZ, (P::nt_t && NT)>(a, c), txy0 = LO<P, FTXY, (P::nt_t && NT)>(a, c), tyz0 = LO<P, FTYZ, (P::nt_t && NT)>(a, c);
-    const A txz0 = LO<P, FTXZ, (P::nt_t && NT)>(a, c);
+    const A p0 = LO<P, FP, (P::nt_t && NT)>(vi, c), txx0 = LO<P, FTXX, (P::nt_t && NT)>(vi, c), tyy0 = LO<P, FTYY, (P::nt_t && NT)>(vi, c);
+    const A tzz0 = LO<P, FTZZ, (P::nt_t && NT)>(vi, c), txy0 = LO<P, FTXY, (P::nt_t && NT)>(vi, c), tyz0 = LO<P, FTYZ, (P::nt_t && NT)>(vi, c);
+    const A txz0 = LO<P, FTXZ, (P::nt_t && NT)>(vi, c);
     A kt[8];  // K[14..21]: P1, P2, S1, S2, S3, Sxy, Sxz, Syz
     if constexpr (P::medium) medium_stress(a, c, sy, sz, rq, kt);
     else coef_block<P, 8>(a, a.kt, c, K_P1, kt);
@@ -807,38 +834,38 @@ __device__ __forceinline__ bool stress_tile(const AT &a, int tx, int ty, int tz)
     A ezi = 0, azi = 0, ezh = 0, azh = 0;
     if (px >= 0) {
       ox = (u32)px + wxs * ((u32)j + ny * (u32)k);
-      carry_load(cx, a.carry[0], 1u, ox, sl0);
+      carry_load(cx, vi.carry(0), 1u, ox, sl0);
     }
     if (py >= 0) {
       oy = (u32)i + nx * ((u32)py + wys * (u32)k);
-      carry_load(cy, a.carry[1], 1u, oy, sl1);
+      carry_load(cy, vi.carry(1), 1u, oy, sl1);
     }
     if (pz >= 0) {
       ezi = prof<A>(a.prof[2][0], k), azi = prof<A>(a.prof[2][1], k);
       ezh = prof<A>(a.prof[2][2], k), azh = prof<A>(a.prof[2][3], k);
       oz = (u32)i + nx * ((u32)j + ny * (u32)pz);
-      carry_load(cz, a.carry[2], 1u, oz, sl2);
+      carry_load(cz, vi.carry(2), 1u, oz, sl2);
     }
     if (px >= 0) {
       uxx = pml<P>(cx[0], uxx, exi, axi);
       wx = pml<P>(cx[1], wx, exi, axi);
       uyx = pml<P>(cx[2], uyx, exh, axh);
       uzx = pml<P>(cx[3], uzx, exh, axh);
-      carry_store(cx, a.carry[0], 1u, ox, sl0);
+      carry_store(cx, vo.carry(0), 1u, ox, sl0);
     }
     if (py >= 0) {
       uyy = pml<P>(cy[0], uyy, eyi, ayi);
       wy = pml<P>(cy[1], wy, eyi, ayi);
       uxy = pml<P>(cy[2], uxy, eyh, ayh);
       uzy = pml<P>(cy[3], uzy, eyh, ayh);
-      carry_store(cy, a.carry[1], 1u, oy, sl1);
+      carry_store(cy, vo.carry(1), 1u, oy, sl1);
     }
     if (pz >= 0) {
       uzz = pml<P>(cz[0], uzz, ezi, azi);
       wz = pml<P>(cz[1], wz, ezi, azi);
       uxz = pml<P>(cz[2], uxz, ezh, azh);
       uyz = pml<P>(cz[3], uyz, ezh, azh);
-      carry_store(cz, a.carry[2], 1u, oz, sl2);
+      carry_store(cz, vo.carry(2), 1u, oz, sl2);
     }
 
     // pore pressure and stresses (kernel.cu:484-490)
@@ -861,22 +888,22 @@ __device__ __forceinline__ bool stress_tile(const AT &a, int tx, int ty, int tz)
       pk_split(txzn, hb[pk_slot(FTXZ)], rb[pk_slot(FTXZ)]);
       pk_split(tyzn, hb[pk_slot(FTYZ)], rb[pk_slot(FTYZ)]);
       pk_split(pn, hb[pk_slot(FP)], rb[pk_slot(FP)]);
-      at<uint16_t>(a.f[FTXX], c) = hb[pk_slot(FTXX)];
-      at<uint16_t>(a.f[FTYY], c) = hb[pk_slot(FTYY)];
-      at<uint16_t>(a.f[FTZZ], c) = hb[pk_slot(FTZZ)];
-      at<uint16_t>(a.f[FTXY], c) = hb[pk_slot(FTXY)];
-      at<uint16_t>(a.f[FTXZ], c) = hb[pk_slot(FTXZ)];
-      at<uint16_t>(a.f[FTYZ], c) = hb[pk_slot(FTYZ)];
-      at<uint16_t>(a.f[FP], c) = hb[pk_slot(FP)];
-      at<u32>(a.lo[PK_FIRST], c) = pk_record(rb);
+      at<uint16_t>(vo.f(FTXX), c) = hb[pk_slot(FTXX)];
+      at<uint16_t>(vo.f(FTYY), c) = hb[pk_slot(FTYY)];
+      at<uint16_t>(vo.f(FTZZ), c) = hb[pk_slot(FTZZ)];
+      at<uint16_t>(vo.f(FTXY), c) = hb[pk_slot(FTXY)];
+      at<uint16_t>(vo.f(FTXZ), c) = hb[pk_slot(FTXZ)];
+      at<uint16_t>(vo.f(FTYZ), c) = hb[pk_slot(FTYZ)];
+      at<uint16_t>(vo.f(FP), c) = hb[pk_slot(FP)];
+      at<u32>(vo.lo(PK_FIRST), c) = pk_record(rb);
     } else {
-      ST<P, FP, (P::nt_t && NT)>(a, c, pn);
-      ST<P, FTXX, (P::nt_t && NT)>(a, c, txxn);
-      ST<P, FTYY, (P::nt_t && NT)>(a, c, tyyn);
-      ST<P, FTZZ, (P::nt_t && NT)>(a, c, tzzn);
-      ST<P, FTXY, (P::nt_t && NT)>(a, c, txyn);
-      ST<P, FTYZ, (P::nt_t && NT)>(a, c, tyzn);
-      ST<P, FTXZ, (P::nt_t && NT)>(a, c, txzn);
+      ST<P, FP, (P::nt_t && NT)>(vo, c, pn);
+      ST<P, FTXX, (P::nt_t && NT)>(vo, c, txxn);
+      ST<P, FTYY, (P::nt_t && NT)>(vo, c, tyyn);
+      ST<P, FTZZ, (P::nt_t && NT)>(vo, c, tzzn);
+      ST<P, FTXY, (P::nt_t && NT)>(vo, c, txyn);
+      ST<P, FTYZ, (P::nt_t && NT)>(vo, c, tyzn);
+      ST<P, FTXZ, (P::nt_t && NT)>(vo, c, txzn);
     }
 
 #pragma unroll
@@ -890,15 +917,18 @@ __device__ __forceinline__ bool stress_tile(const AT &a, int tx, int ty, int tz)
   return own;
 }
 
-// Source injection (kernel.cu:130-142) of step it into field f of the source cell.
+// Source injection (kernel.cu:130-142) of step it into field f of the source cell: the value at
+// ioff bytes on plus the sample, stored at ooff bytes on (the state's place in a run of states, 0 in
+// place); past the wavelet the value alone.
 template <class P, class SA>
-__device__ __forceinline__ void source_field(const SA &sa, int f, int it)
+__device__ __forceinline__ void source_field(const SA &sa, int f, int it, uint64_t ioff, uint64_t ooff)
 {
   using A = typename P::A;
   const u32 c = (u32)sa.cell;
   const bool cf = (P::cmask >> f) & 1u;
-  const A w = (A)sa.wavelet[it], inv = (A)sa.inv_scale[f];
-  const A old = load_raw<P>(sa.f[f], sa.lo[f], cf, c);
+  const A w = it < sa.nt_w ? (A)sa.wavelet[it] : A(0), inv = (A)sa.inv_scale[f];
+  char *p = reinterpret_cast<char *>(sa.f[f]);
+  const A old = load_raw<P>(p + ioff, sa.lo[f] + ioff, cf, c);
   // one rounding or two, written out, so that the value does not depend on which launch adds it
   A x;
   if constexpr (P::comp && !P::packed) {
@@ -910,33 +940,34 @@ __device__ __forceinline__ void source_field(const SA &sa, int f, int it)
   } else {
     x = fmaf(w, inv, old);
   }
-  store_raw<P>(sa.f[f], sa.lo[f], cf, c, x);
+  store_raw<P>(p + ooff, sa.lo[f] + ooff, cf, c, x);
 }
 // one lane per field
 template <class P>
-__device__ __forceinline__ void source_cell(const SourceArgs &sa, int it)
+__device__ __forceinline__ void source_cell(const SourceArgs &sa, int it, uint64_t ioff, uint64_t ooff)
 {
   const int f = threadIdx.x;
   if (f >= NFIELD || !(sa.mask & (1u << f))) return;
-  source_field<P>(sa, f, it);
+  source_field<P>(sa, f, it, ioff, ooff);
 }
 // After a tile of the stress half step: the thread that updated the source cell adds step it's
 // source to it.  No other thread of the launch reads or writes that cell's stresses.
 template <class P, class SA>
-__device__ __forceinline__ void source_owner(const SA &sa, int it)
+__device__ __forceinline__ void source_owner(const SA &sa, int it, uint64_t off)
 {
 #pragma unroll 1
   for (int f = 0; f < NFIELD; ++f)
-    if (sa.mask & (1u << f)) source_field<P>(sa, f, it);
+    if (sa.mask & (1u << f)) source_field<P>(sa, f, it, off, off);
 }
 
-// Receiver sampling: traces[comp][it][rec] = field value * storage scale.
+// Receiver sampling: traces[comp][it][rec] = field value * storage scale (of the state off bytes on).
 template <class P, class RA>
-__device__ __forceinline__ void record_one(const RA &ra, int64_t r, int ci, int it)
+__device__ __forceinline__ void record_one(const RA &ra, int64_t r, int ci, int it, uint64_t off)
 {
   const int f = ra.comp[ci];
   // the product of two floats is exact in double, so (float)v is the rounded float product
-  const double v = (double)load_raw<P>(ra.f[f], ra.lo[f], (P::cmask >> f) & 1u, (u32)ra.rec[r]) *
+  const double v = (double)load_raw<P>(reinterpret_cast<const char *>(ra.f[f]) + off, ra.lo[f] + off,
+                                       (P::cmask >> f) & 1u, (u32)ra.rec[r]) *
                    (double)ra.scale[ci];
   const int64_t o = ((int64_t)ci * ra.nt_max + it) * ra.nrec + r;
   const float vf = (float)v;
@@ -948,11 +979,11 @@ __device__ __forceinline__ void record_one(const RA &ra, int64_t r, int ci, int 
 }
 // components c0..c1-1 of the receiver a block-th thread of recording block b stands for
 template <class P, class RA>
-__device__ __forceinline__ void record_block(const RA &ra, int b, int c0, int c1, int it)
+__device__ __forceinline__ void record_block(const RA &ra, int b, int c0, int c1, int it, uint64_t off)
 {
   const int64_t r = (int64_t)b * (blockDim.x * blockDim.y) + threadIdx.y * blockDim.x + threadIdx.x;
   if (r >= ra.nrec) return;
-  for (int ci = c0; ci < c1; ++ci) record_one<P>(ra, r, ci, it);
+  for (int ci = c0; ci < c1; ++ci) record_one<P>(ra, r, ci, it, off);
 }
 
 // the constant address space: uniform reads through it stay in scalar registers
@@ -973,31 +1004,36 @@ __device__ __forceinline__ __attribute__((address_space(4))) const T *late_args(
   return (__attribute__((address_space(4))) const T *)p;
 }
 
-template <class P, int ORDER>
+// OOP: the half step reads state u.q of a run of states at the arguments' pointers and writes state
+// u.q + 1
+template <class P, int ORDER, bool OOP>
 __global__ void __launch_bounds__(256) k_velocity(const StepArgs a, const FuseArgs u)
 {
+  const uint64_t ioff = OOP ? (uint64_t)u.q * a.sb : 0, ooff = OOP ? ioff + a.sb : 0;
   if ((int)blockIdx.x >= u.tile_blocks) {
-    record_block<P>(u.rec, blockIdx.x - u.tile_blocks, u.rec.c0, u.rec.c1, u.rec.it);
+    record_block<P>(u.rec, blockIdx.x - u.tile_blocks, u.rec.c0, u.rec.c1, u.rec.it, ioff);
     return;
   }
   int tx, ty, tz;
   if (!tile_of(a, tx, ty, tz)) return;
-  velocity_tile<P, ORDER, true>(a, tx, ty, tz);
+  velocity_tile<P, ORDER, true, OOP>(a, tx, ty, tz, ioff, ooff);
 }
-template <class P, int ORDER>
+template <class P, int ORDER, bool OOP>
 __global__ void __launch_bounds__(256) k_stress(const StepArgs a, const FuseArgs u)
 {
+  const uint64_t ioff = OOP ? (uint64_t)u.q * a.sb : 0, ooff = OOP ? ioff + a.sb : 0;
   if ((int)blockIdx.x >= u.tile_blocks) {
-    record_block<P>(u.rec, blockIdx.x - u.tile_blocks, u.rec.c0, u.rec.c1, u.rec.it);
+    record_block<P>(u.rec, blockIdx.x - u.tile_blocks, u.rec.c0, u.rec.c1, u.rec.it, ooff);
     return;
   }
   int tx, ty, tz;
   if (!tile_of(a, tx, ty, tz)) return;
-  if (!stress_tile<P, ORDER, true>(a, tx, ty, tz)) return;
+  if (!stress_tile<P, ORDER, true, OOP>(a, tx, ty, tz, ioff, ooff)) return;
   // the arguments of what follows are read here, so that none of them is kept in scalar registers
   // over the plane loop (kept, they spilled 16 more of the FP16T kernel's)
-  CFuseArgs &u1 = *(CFuseArgs *)(late_args<StepArgs>() + 1);
-  if (u1.source) source_owner<P>(u1.src, u1.src.it);
+  CStepArgs *a1 = late_args<StepArgs>();
+  CFuseArgs &u1 = *(CFuseArgs *)(a1 + 1);
+  if (u1.source) source_owner<P>(u1.src, u1.src.it, OOP ? (uint64_t)(u1.q + 1) * a1->sb : 0);
 }
 
 // Batched forms: one launch covers the tiles of every shot.  The shots' tile lists are
@@ -1019,20 +1055,23 @@ __device__ __forceinline__ int shot_of(const BA &b, int t)
   return lo;
 }
 // tile t of the concatenated lists
-template <class P, int ORDER, bool VEL>
+template <class P, int ORDER, bool VEL, bool OOP>
 __device__ __forceinline__ void batch_tile(const BatchArgs &b, int t)
 {
   const int s = shot_of(b, t);
   const CStepArgs &a = ((CStepArgs *)b.shots)[s];
   const int lt = t - ((CInt *)b.tile_start)[s];
   const int tx = lt % a.gx, r = lt / a.gx, ty = r % a.gy, tz = r / a.gy;
+  const uint64_t ioff = OOP ? (uint64_t)b.q * a.sb : 0, ooff = OOP ? ioff + a.sb : 0;
   if constexpr (VEL) {
-    velocity_tile<P, ORDER, false>(a, tx, ty, tz);
-  } else if (stress_tile<P, ORDER, false>(a, tx, ty, tz)) {
+    velocity_tile<P, ORDER, false, OOP>(a, tx, ty, tz, ioff, ooff);
+  } else if (stress_tile<P, ORDER, false, OOP>(a, tx, ty, tz, ioff, ooff)) {
     CBatchArgs &b1 = *late_args<BatchArgs>();
-    CSourceArgs &sa = ((CSourceArgs *)b1.src)[shot_of(b1, t)];
+    const int s1 = shot_of(b1, t);
+    CSourceArgs &sa = ((CSourceArgs *)b1.src)[s1];
     const int it = ((CInt *)b1.it)[0] + b1.off + 1;
-    if (b1.src && sa.wavelet && it < sa.nt_w && it < ((CInt *)b1.it)[1]) source_owner<P>(sa, it);
+    if (b1.src && sa.wavelet && it < sa.nt_w && it < ((CInt *)b1.it)[1])
+      source_owner<P>(sa, it, OOP ? (uint64_t)(b1.q + 1) * ((CStepArgs *)b1.shots)[s1].sb : 0);
   }
 }
 // QUEUE false: one block per tile slot of its XCD (workgroup b on XCD b % 8).  QUEUE: a smaller grid whose blocks take their group's next tile from the
@@ -1042,22 +1081,23 @@ __device__ __forceinline__ void batch_tile(const BatchArgs &b, int t)
 // other block of the group touches them after its own last claim).  Two kernels, because one loop
 // for both kept the queue's state in scalar registers over the plane loop (6-35 of them spilled
 // at order 4; without the queue 0-5, and FP16's velocity kernel fits 5 waves a SIMD, not 4).
-template <class P, int ORDER, bool VEL, bool QUEUE>
+// OOP (one block per tile, recording nothing): state b.q of each shot's run of states to the next.
+template <class P, int ORDER, bool VEL, bool QUEUE, bool OOP>
 __global__ void __launch_bounds__(256) k_step_batch(const BatchArgs b)
 {
-  if ((int)blockIdx.x >= b.tile_blocks) {
+  if (!OOP && (int)blockIdx.x >= b.tile_blocks) {
     // velocity launch: the stresses and p of the step before; stress launch: the step's velocities
     const int rb = blockIdx.x - b.tile_blocks, s = rb / b.rec_blocks;
     const CRecordArgs &ra = ((CRecordArgs *)b.rec)[s];
     const int it = ((CInt *)b.it)[0] + b.off - (VEL ? 1 : 0);
     if (!ra.traces || it < ((CInt *)b.it)[2] || it >= ra.nt_max) return;
-    record_block<P>(ra, rb - s * b.rec_blocks, VEL ? ra.nvel : 0, VEL ? ra.ncomp : ra.nvel, it);
+    record_block<P>(ra, rb - s * b.rec_blocks, VEL ? ra.nvel : 0, VEL ? ra.ncomp : ra.nvel, it, 0);
     return;
   }
   const int x = blockIdx.x & 7;
   if constexpr (!QUEUE) {
     const int t = xcd_tile(x, blockIdx.x >> 3, b.xg);
-    if (t < b.total_tiles) batch_tile<P, ORDER, VEL>(b, t);
+    if (t < b.total_tiles) batch_tile<P, ORDER, VEL, OOP>(b, t);
   } else {
     // every thread of the block reaches each barrier: the claims are the block's
     __shared__ int s_next;
@@ -1070,7 +1110,7 @@ __global__ void __launch_bounds__(256) k_step_batch(const BatchArgs b)
     while (t < b.total_tiles) {
       __syncthreads();  // every thread has read s_next
       if (lead) s_next = atomicAdd(ctr, 1);
-      batch_tile<P, ORDER, VEL>(b, t);
+      batch_tile<P, ORDER, VEL, OOP>(b, t);
       __syncthreads();  // the next claim is in s_next
       t = xcd_tile(x, s_next, b.xg);
     }
@@ -1084,24 +1124,26 @@ __global__ void __launch_bounds__(256) k_step_batch(const BatchArgs b)
 template <class P>
 __global__ void k_source(const SourceArgs sa)
 {
-  source_cell<P>(sa, sa.it);
+  source_cell<P>(sa, sa.it, sa.ioff, sa.ooff);
 }
 
 template <class P>
 __global__ void k_record(const RecordArgs ra)
 {
-  record_block<P>(ra, blockIdx.x, ra.c0, ra.c1, ra.it);
+  record_block<P>(ra, blockIdx.x, ra.c0, ra.c1, ra.it, ra.off);
 }
 
 // Batched source / record: one block (z) per shot; the step index comes from a device
 // counter, so a captured sequence of steps can be replayed.
 template <class P>
-__global__ void k_source_batch(const SourceArgs *tab, const int *itp, int off)
+__global__ void k_source_batch(const SourceArgs *tab, const int *itp, int off, int q)
 {
   const SourceArgs &sa = tab[blockIdx.x];
   const int it = *itp + off;
-  if (!sa.wavelet || it >= sa.nt_w) return;
-  source_cell<P>(sa, it);
+  const bool carry = sa.outside && q > 0;  // no half step writes the cell: its value comes along here
+  if (!sa.wavelet || (it >= sa.nt_w && !carry)) return;
+  const uint64_t ooff = q < 0 ? 0 : (uint64_t)q * sa.sb;
+  source_cell<P>(sa, it, carry ? ooff - sa.sb : ooff, ooff);
 }
 template <class P>
 __global__ void k_record_batch(const RecordArgs *tab, bool vel, const int *itp, int off)
@@ -1109,7 +1151,7 @@ __global__ void k_record_batch(const RecordArgs *tab, bool vel, const int *itp, 
   const RecordArgs &ra = tab[blockIdx.z];
   const int it = *itp + off;
   if (!ra.traces || it >= ra.nt_max) return;
-  record_block<P>(ra, blockIdx.x, vel ? 0 : ra.nvel, ra.ncomp, it);
+  record_block<P>(ra, blockIdx.x, vel ? 0 : ra.nvel, ra.ncomp, it, 0);
 }
 __global__ void k_advance(int *itp, int d)
 {
@@ -1118,6 +1160,24 @@ __global__ void k_advance(int *itp, int d)
 __global__ void k_set_counter(int *itp, int v, int end)
 {
   if (threadIdx.x == 0) itp[0] = v, itp[1] = end, itp[2] = v;
+}
+
+// zero values in the cells outside the update box of every field (and residual) of nstates states:
+// the half steps read them there and write only inside
+template <int ESZ>
+__global__ void __launch_bounds__(256) k_clear_border(char *slots, uint64_t sb, uint64_t loff, int lsz, int h, int nx,
+                                                      int ny, int nz)
+{
+  const uint32_t n = (uint32_t)nx * ny * nz, c = blockIdx.x * 256u + threadIdx.x;
+  if (c >= n) return;
+  const int i = (int)(c % (uint32_t)nx), j = (int)(c / (uint32_t)nx % (uint32_t)ny), k = (int)(c / ((uint32_t)nx * ny));
+  if (i >= h && i < nx - h && j >= h && j < ny - h && k >= h && k < nz - h) return;
+  char *s = slots + (uint64_t)blockIdx.y * sb;
+  for (int f = 0; f < NFIELD; ++f)
+    for (int b = 0; b < ESZ; b += 2) *reinterpret_cast<uint16_t *>(s + ((uint64_t)f * n + c) * ESZ + b) = 0;
+  if (lsz == PK_RECORD) *reinterpret_cast<uint32_t *>(s + loff + (uint64_t)c * PK_RECORD) = 0u;
+  else if (lsz == 1)
+    for (int f = 0; f < NFIELD; ++f) s[loff + (uint64_t)f * n + c] = 0;
 }
 
 // In-place multiply of an FP16M tau or p field (lo: its tagged residual pointer).
@@ -1199,7 +1259,7 @@ __global__ void k_rescale4(S *p, int64_t nrec, double f0, double f1, double f2, 
 
 template <class P, int ORDER, bool VEL>
 hipError_t launch_step(const StepArgs &in, LaunchShape sh, hipStream_t s, const RecordArgs *rec,
-                       const SourceArgs *src)
+                       const SourceArgs *src, int q)
 {
   StepArgs a = in;
   const int h = ORDER / 2;
@@ -1212,39 +1272,40 @@ hipError_t launch_step(const StepArgs &in, LaunchShape sh, hipStream_t s, const 
   u.tile_blocks = (int)(8 * xcd_slots(a.ntiles, a.xg));
   u.record = rec && rec->nrec > 0 && rec->c1 > rec->c0;
   u.source = src != nullptr;
+  u.q = q;
   if (u.record) u.rec = *rec;
   if (u.source) u.src = *src;
   const int64_t rb = u.record ? (rec->nrec + sh.bx * sh.by - 1) / (sh.bx * sh.by) : 0;
   dim3 grid((unsigned)(u.tile_blocks + rb));
-  if (VEL)
-    hipLaunchKernelGGL((k_velocity<P, ORDER>), grid, block, 0, s, a, u);
-  else
-    hipLaunchKernelGGL((k_stress<P, ORDER>), grid, block, 0, s, a, u);
+  if (VEL && q >= 0) hipLaunchKernelGGL((k_velocity<P, ORDER, true>), grid, block, 0, s, a, u);
+  else if (VEL) hipLaunchKernelGGL((k_velocity<P, ORDER, false>), grid, block, 0, s, a, u);
+  else if (q >= 0) hipLaunchKernelGGL((k_stress<P, ORDER, true>), grid, block, 0, s, a, u);
+  else hipLaunchKernelGGL((k_stress<P, ORDER, false>), grid, block, 0, s, a, u);
   return hipGetLastError();
 }
 
 template <bool VEL, int ORDER>
 hipError_t dispatch_order(int prec, const StepArgs &a, LaunchShape sh, hipStream_t s, const RecordArgs *rec,
-                          const SourceArgs *src)
+                          const SourceArgs *src, int q)
 {
   switch (prec) {
-    case PREC_FP32: return launch_step<P32, ORDER, VEL>(a, sh, s, rec, src);
-    case PREC_FP16: return launch_step<P16, ORDER, VEL>(a, sh, s, rec, src);
-    case PREC_FP16C: return launch_step<P16C, ORDER, VEL>(a, sh, s, rec, src);
-    case PREC_FP16T: return launch_step<P16T, ORDER, VEL>(a, sh, s, rec, src);
-    case PREC_FP16M: return launch_step<P16M, ORDER, VEL>(a, sh, s, rec, src);
-    case PREC_FP64: return launch_step<P64, ORDER, VEL>(a, sh, s, rec, src);
+    case PREC_FP32: return launch_step<P32, ORDER, VEL>(a, sh, s, rec, src, q);
+    case PREC_FP16: return launch_step<P16, ORDER, VEL>(a, sh, s, rec, src, q);
+    case PREC_FP16C: return launch_step<P16C, ORDER, VEL>(a, sh, s, rec, src, q);
+    case PREC_FP16T: return launch_step<P16T, ORDER, VEL>(a, sh, s, rec, src, q);
+    case PREC_FP16M: return launch_step<P16M, ORDER, VEL>(a, sh, s, rec, src, q);
+    case PREC_FP64: return launch_step<P64, ORDER, VEL>(a, sh, s, rec, src, q);
   }
   return hipErrorInvalidValue;
 }
 
 template <bool VEL>
 hipError_t dispatch(int prec, int order, const StepArgs &a, LaunchShape sh, hipStream_t s,
-                    const RecordArgs *rec, const SourceArgs *src)
+                    const RecordArgs *rec, const SourceArgs *src, int q)
 {
   if (sh.bx * sh.by > 256 || sh.bx <= 0 || sh.by <= 0) return hipErrorInvalidValue;
-  if (order == 2) return dispatch_order<VEL, 2>(prec, a, sh, s, rec, src);
-  if (order == 4) return dispatch_order<VEL, 4>(prec, a, sh, s, rec, src);
+  if (order == 2) return dispatch_order<VEL, 2>(prec, a, sh, s, rec, src, q);
+  if (order == 4) return dispatch_order<VEL, 4>(prec, a, sh, s, rec, src, q);
   return hipErrorInvalidValue;
 }
 
@@ -1256,14 +1317,16 @@ hipError_t launch_step_batch(int prec, int order, bool vel, const BatchArgs &in,
   if (sh.bx * sh.by > 256 || sh.bx <= 0 || sh.by <= 0 || blocks <= 0 || blocks % 8) return hipErrorInvalidValue;
   BatchArgs b = in;
   b.xg = xcd_run(b.total_tiles, sh.bx * sh.by, (int64_t)b.total_tiles * sh.bx * sh.by * sh.zchunk);
+  if (b.q >= 0) b.queue = nullptr;
   b.tile_blocks = b.queue ? blocks : (int)(8 * xcd_slots(b.total_tiles, b.xg));
   b.rec_blocks = (int)((max_nrec + sh.bx * sh.by - 1) / (sh.bx * sh.by));
   dim3 grid((unsigned)(b.tile_blocks + b.rec_blocks * b.nshots)), block(sh.bx, sh.by, 1);
+#define BIOT_BATCH_LAUNCH(PP, OO, VV)                                                            \
+  if (b.q >= 0) hipLaunchKernelGGL((k_step_batch<PP, OO, VV, false, true>), grid, block, 0, s, b);      \
+  else if (b.queue) hipLaunchKernelGGL((k_step_batch<PP, OO, VV, true, false>), grid, block, 0, s, b);  \
+  else hipLaunchKernelGGL((k_step_batch<PP, OO, VV, false, false>), grid, block, 0, s, b);
 #define BIOT_BATCH_CASE(PP, OO)                                                                 \
-  if (vel && b.queue) hipLaunchKernelGGL((k_step_batch<PP, OO, true, true>), grid, block, 0, s, b);   \
-  else if (vel) hipLaunchKernelGGL((k_step_batch<PP, OO, true, false>), grid, block, 0, s, b);  \
-  else if (b.queue) hipLaunchKernelGGL((k_step_batch<PP, OO, false, true>), grid, block, 0, s, b);    \
-  else hipLaunchKernelGGL((k_step_batch<PP, OO, false, false>), grid, block, 0, s, b);
+  if (vel) { BIOT_BATCH_LAUNCH(PP, OO, true) } else { BIOT_BATCH_LAUNCH(PP, OO, false) }
   if (order != 2 && order != 4) return hipErrorInvalidValue;
   switch (prec) {
     case PREC_FP32:
@@ -1287,19 +1350,21 @@ hipError_t launch_step_batch(int prec, int order, bool vel, const BatchArgs &in,
     default: return hipErrorInvalidValue;
   }
 #undef BIOT_BATCH_CASE
+#undef BIOT_BATCH_LAUNCH
   return hipGetLastError();
 }
 
-hipError_t launch_source_batch(int prec, const SourceArgs *tab, int nshots, const int *it, int off, hipStream_t s)
+hipError_t launch_source_batch(int prec, const SourceArgs *tab, int nshots, const int *it, int off, int q,
+                               hipStream_t s)
 {
   if (nshots <= 0) return hipSuccess;
   switch (prec) {
-    case PREC_FP32: hipLaunchKernelGGL(k_source_batch<P32>, dim3(nshots), dim3(64), 0, s, tab, it, off); break;
-    case PREC_FP16: hipLaunchKernelGGL(k_source_batch<P16>, dim3(nshots), dim3(64), 0, s, tab, it, off); break;
-    case PREC_FP16C: hipLaunchKernelGGL(k_source_batch<P16C>, dim3(nshots), dim3(64), 0, s, tab, it, off); break;
-    case PREC_FP16T: hipLaunchKernelGGL(k_source_batch<P16T>, dim3(nshots), dim3(64), 0, s, tab, it, off); break;
-    case PREC_FP16M: hipLaunchKernelGGL(k_source_batch<P16M>, dim3(nshots), dim3(64), 0, s, tab, it, off); break;
-    case PREC_FP64: hipLaunchKernelGGL(k_source_batch<P64>, dim3(nshots), dim3(64), 0, s, tab, it, off); break;
+    case PREC_FP32: hipLaunchKernelGGL(k_source_batch<P32>, dim3(nshots), dim3(64), 0, s, tab, it, off, q); break;
+    case PREC_FP16: hipLaunchKernelGGL(k_source_batch<P16>, dim3(nshots), dim3(64), 0, s, tab, it, off, q); break;
+    case PREC_FP16C: hipLaunchKernelGGL(k_source_batch<P16C>, dim3(nshots), dim3(64), 0, s, tab, it, off, q); break;
+    case PREC_FP16T: hipLaunchKernelGGL(k_source_batch<P16T>, dim3(nshots), dim3(64), 0, s, tab, it, off, q); break;
+    case PREC_FP16M: hipLaunchKernelGGL(k_source_batch<P16M>, dim3(nshots), dim3(64), 0, s, tab, it, off, q); break;
+    case PREC_FP64: hipLaunchKernelGGL(k_source_batch<P64>, dim3(nshots), dim3(64), 0, s, tab, it, off, q); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -1335,14 +1400,14 @@ hipError_t launch_set_counter(int *it, int v, int end, hipStream_t s)
 }
 
 hipError_t launch_velocity(int prec, int order, const StepArgs &args, LaunchShape sh, hipStream_t s,
-                           const RecordArgs *rec)
+                           const RecordArgs *rec, int q)
 {
-  return dispatch<true>(prec, order, args, sh, s, rec, nullptr);
+  return dispatch<true>(prec, order, args, sh, s, rec, nullptr, q);
 }
 hipError_t launch_stress(int prec, int order, const StepArgs &args, LaunchShape sh, hipStream_t s,
-                         const RecordArgs *rec, const SourceArgs *src)
+                         const RecordArgs *rec, const SourceArgs *src, int q)
 {
-  return dispatch<false>(prec, order, args, sh, s, rec, src);
+  return dispatch<false>(prec, order, args, sh, s, rec, src, q);
 }
 
 hipError_t launch_source(int prec, const SourceArgs &a, hipStream_t s)
@@ -1357,6 +1422,25 @@ hipError_t launch_source(int prec, const SourceArgs &a, hipStream_t s)
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
+}
+
+hipError_t launch_clear_border(int prec, void *slots, int nstates, uint64_t sb, uint64_t loff, int h, int nx, int ny,
+                               int nz, hipStream_t s)
+{
+  const int lsz = prec == PREC_FP16M ? PK_RECORD : comp_fields(prec) ? 1 : 0;
+  const uint32_t blocks = (uint32_t)(((int64_t)nx * ny * nz + 255) / 256);
+  for (int q = 0; q < nstates; q += 32768) {  // the grid's y extent
+    const dim3 grid(blocks, (unsigned)std::min(nstates - q, 32768));
+    char *p = (char *)slots + (uint64_t)q * sb;
+    switch (field_bytes(prec)) {
+      case 2: hipLaunchKernelGGL(k_clear_border<2>, grid, dim3(256), 0, s, p, sb, loff, lsz, h, nx, ny, nz); break;
+      case 4: hipLaunchKernelGGL(k_clear_border<4>, grid, dim3(256), 0, s, p, sb, loff, lsz, h, nx, ny, nz); break;
+      default: hipLaunchKernelGGL(k_clear_border<8>, grid, dim3(256), 0, s, p, sb, loff, lsz, h, nx, ny, nz); break;
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_rescale(int prec, void *p, int8_t *lo, int64_t n, double f, hipStream_t s)
