@@ -729,8 +729,8 @@ std::string tune_key(const biot_handle *h)
   for (auto &ch : arch)
     if (ch == ' ') ch = '_';
   char buf[256];
-  snprintf(buf, sizeof buf, "v5 %s p%d o%d %dx%dx%d", arch.c_str(), h->prec, h->g.order, h->g.nx,
-           h->g.ny, h->g.nz);
+  snprintf(buf, sizeof buf, "v6 %s p%d%s o%d %dx%dx%d", arch.c_str(), h->prec, h->d_ids ? "r" : "", h->g.order,
+           h->g.nx, h->g.ny, h->g.nz);
   return buf;
 }
 bool tune_lookup(const std::string &key, LaunchShape &out)

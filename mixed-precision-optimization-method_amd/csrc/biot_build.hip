@@ -207,7 +207,105 @@ __global__ void __launch_bounds__(256) k_ref_to_kernel(RefArgs a)
   }
 }
 
+// A hash table of the distinct 22-value records, compared bit by bit: slot s holds the first cell
+// that claimed it, ids[c] the slot of cell c's record.  A wave works through its distinct records one
+// at a time (the lanes that hold the same one take its slot together), so a layered medium costs one
+// probe a wave and no contended atomics.  Every loop is bounded: a probe by 64 slots, the wave's by
+// its lanes (the first lane left is always resolved).
+template <typename S>
+struct DictWord {
+  using T = std::conditional_t<sizeof(S) == 8, unsigned long long, std::conditional_t<sizeof(S) == 4, uint32_t, uint16_t>>;
+};
+template <typename S>
+__global__ void __launch_bounds__(256) k_dict(DictArgs a)
+{
+  using W = typename DictWord<S>::T;
+  const W *coef = (const W *)a.coef;
+  const int lane = threadIdx.x & 63;
+  for (int64_t base = (int64_t)blockIdx.x * 256; base < a.n; base += (int64_t)gridDim.x * 256) {
+    const int64_t c = base + threadIdx.x;
+    const bool act = c < a.n;
+    W v[NKC];
+    uint32_t hash = 0x9E3779B9u;
+#pragma unroll
+    for (int k = 0; k < NKC; ++k) {
+      v[k] = act ? coef[(int64_t)k * a.n + c] : W(0);
+      uint32_t w = (uint32_t)v[k];
+      if constexpr (sizeof(S) == 8) w ^= (uint32_t)(v[k] >> 32) * 0xC2B2AE35u;
+      hash = (hash ^ w) * 0x85EBCA6Bu;
+      hash ^= hash >> 15;
+    }
+    unsigned long long todo = __ballot(act);
+    while (todo) {
+      if (__builtin_amdgcn_readfirstlane(
+              __hip_atomic_load(a.state + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
+        return;
+      const int lead = __ffsll(todo) - 1;
+      const uint32_t h = (uint32_t)__shfl((int)hash, lead);
+      for (uint32_t p = 0; (todo >> lead) & 1ull; ++p) {
+        if (p == 64) {
+          if (lane == 0) __hip_atomic_store(a.state + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          return;
+        }
+        const uint32_t s = (h + p) & (DICT_SLOTS - 1);
+        uint32_t r = __hip_atomic_load(a.slots + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (r == DICT_EMPTY && lane == lead) {
+          r = atomicCAS(a.slots + s, DICT_EMPTY, (uint32_t)c);
+          if (r == DICT_EMPTY) {
+            r = (uint32_t)c;
+            if (atomicAdd(a.state, 1u) >= DICT_MAX)
+              __hip_atomic_store(a.state + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          }
+        }
+        r = (uint32_t)__shfl((int)r, lead);
+        bool same = (todo >> lane) & 1ull;
+#pragma unroll
+        for (int k = 0; k < NKC; ++k) same = same && v[k] == coef[(int64_t)k * a.n + r];
+        if (same) a.ids[c] = (uint16_t)s;
+        todo &= ~__ballot(same);
+      }
+    }
+  }
+}
+// the records' values, one thread a slot
+template <typename S>
+__global__ void __launch_bounds__(256) k_dict_values(DictArgs a)
+{
+  const uint32_t s = blockIdx.x * 256 + threadIdx.x;
+  if (s >= DICT_SLOTS) return;
+  const uint32_t r = a.slots[s];
+  if (r == DICT_EMPTY) return;
+  const S *coef = (const S *)a.coef;
+  S *dv = (S *)a.dv + (size_t)s * 16, *dt = (S *)a.dt + (size_t)s * 8;
+  for (int k = 0; k < 14; ++k) dv[k] = coef[(int64_t)k * a.n + r];
+  for (int k = 14; k < NKC; ++k) dt[k - 14] = coef[(int64_t)k * a.n + r];
+}
+
 }  // namespace
+
+hipError_t launch_dict(int prec, const DictArgs &a, hipStream_t s)
+{
+  if (a.n <= 0) return hipSuccess;
+  const dim3 grid((unsigned)std::min<int64_t>((a.n + 255) / 256, 2048)), slots(DICT_SLOTS / 256), block(256);
+  switch (prec) {
+    case PREC_FP32:
+      hipLaunchKernelGGL(k_dict<float>, grid, block, 0, s, a);
+      hipLaunchKernelGGL(k_dict_values<float>, slots, block, 0, s, a);
+      break;
+    case PREC_FP64:
+      hipLaunchKernelGGL(k_dict<double>, grid, block, 0, s, a);
+      hipLaunchKernelGGL(k_dict_values<double>, slots, block, 0, s, a);
+      break;
+    case PREC_FP16:
+    case PREC_FP16C:
+    case PREC_FP16T:
+      hipLaunchKernelGGL(k_dict<_Float16>, grid, block, 0, s, a);
+      hipLaunchKernelGGL(k_dict_values<_Float16>, slots, block, 0, s, a);
+      break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
 
 hipError_t launch_moduli(const MediumArgs &m, int64_t n, hipStream_t s)
 {

@@ -106,6 +106,10 @@ struct StepArgs {
   // half step, kt K[14..21] of the stress half step, cell c at element c*14 / c*8 (addressed
   // in 64 bits: these arrays may span more than 4 GiB)
   const void *kv, *kt;
+  // a medium of few distinct cells (DictArgs): the cell's record, and the records' coefficients
+  // (storage type; record r at element 16 r of dv, 8 r of dt); null otherwise
+  const uint16_t *ids;
+  const void *dv, *dt;
   float ks[NKC];             // per-array scale (binary16 storage), 1 otherwise
   // FP16M: the medium records (mv: 4 binary16 values per cell, mt: 4), the cell shear
   // moduli (mu: binary16) and constants
@@ -305,6 +309,23 @@ hipError_t launch_rescale4(int prec, void *p, int64_t nrec, const double f[4], h
 hipError_t launch_slice_xz(int prec, const void *f, const int8_t *lo, bool comp, double scale, int j, int nx,
                            int ny, int nz, float *out, hipStream_t s);
 // per-cell packed copies kv (K[0..13]) and kt (K[14..21]) of the 22 coefficient arrays
+// The distinct coefficient records of a medium (biot_build.hip).  Layered and blocky media hold the
+// same 22 values in most of their cells: then a cell names its record in 2 bytes instead of streaming
+// 88 bytes (FP32) of coefficients a step (256^3 FP32, three layers, velocity + stress: 845 us streamed,
+// 680 us with records).  A medium with more than DICT_MAX different cells keeps the streamed arrays
+// alone; the scan stops where it finds that many.  A random mix of two rocks, 128 records in no order,
+// is still no slower than its streamed arrays (835 us), so the limit is the table's size, not its use:
+// 2048 records of 96 bytes (FP32) stay in an L2.
+constexpr uint32_t DICT_SLOTS = 4096, DICT_MAX = 2048, DICT_EMPTY = 0xFFFFFFFFu;
+struct DictArgs {
+  const void *coef;          // 22 * n stored coefficients
+  int64_t n;
+  uint16_t *ids;             // n
+  void *dv, *dt;             // DICT_SLOTS records of 16 and 8 stored values
+  uint32_t *slots;           // DICT_SLOTS: a cell with the record's values, or DICT_EMPTY
+  uint32_t *state;           // records found; 1 once there are too many (both cleared)
+};
+hipError_t launch_dict(int prec, const DictArgs &a, hipStream_t s);
 hipError_t launch_pack_coef(int prec, const void *soa, void *kv, void *kt, int64_t n, hipStream_t s);
 hipError_t launch_record(int prec, const RecordArgs &a, hipStream_t s);
 

@@ -354,6 +354,7 @@ biot_handle::~biot_handle()
   if (d_lo) (void)hipFree(d_lo);
   if (d_coef) (void)hipFree(d_coef);
   if (d_kpack) (void)hipFree(d_kpack);
+  drop_records();
   if (d_flag) (void)hipFree(d_flag);
   if (h_slice) (void)hipHostFree(h_slice);
   for (auto *p : d_carry)
@@ -406,6 +407,9 @@ void biot_handle::fill_args(StepArgs &a, char *states) const
   }
   a.kv = d_kpack;
   a.kt = d_kpack ? (const char *)d_kpack + (size_t)14 * n * esz : nullptr;
+  a.ids = d_ids;
+  a.dv = d_dict;
+  a.dt = d_dict ? (const char *)d_dict + (size_t)DICT_SLOTS * 16 * esz : nullptr;
   if (prec == BIOT_FP16M) {
     for (int k = 0; k < NKC; ++k) a.k[k] = nullptr;
     a.mv = d_coef;
@@ -748,8 +752,59 @@ int biot_handle::upload_from_ref(const float *d_ref)
     err = "coefficient conversion failed";
     return BIOT_ERR_HIP;
   }
-  if ((rc = pack_coefficients())) return rc;
+  if ((rc = pack_coefficients()) || (rc = find_records())) return rc;
   have_coef = true;
+  return BIOT_OK;
+}
+
+void biot_handle::drop_records()
+{
+  for (void **p : {(void **)&d_ids, &d_dict})
+    if (*p) {
+      (void)hipFree(*p);
+      *p = nullptr;
+    }
+}
+
+// Coefficients built from a medium or given by the caller; an inversion's (biot_set_params) differ
+// from cell to cell and are not looked through.  FP32 and FP64 kernels wait on memory whatever the
+// size, and gain at any (us a step, streamed arrays / records: 64^3 FP32 22.5 / 19.5, 160x144x129 152 /
+// 127, 256^3 851 / 689; FP64 64^3 42 / 33, 224^3 1254 / 1111).  The 16-bit kernels gain while the rest
+// of a step's arrays then about fit the 256 MB memory-side cache (160x144x129: FP16 92 / 79, FP16T 122 /
+// 87, FP16C 147 / 115; 192x192x160: FP16 161 / 142); past it they are bound by what they issue, and the
+// dependent load costs more than the bytes it saves (192x192x160: FP16T 212 / 221, FP16C 270 / 278;
+// 224^3: FP16 295 / 296, FP16C 499 / 514).  Without room for it the arrays are streamed as ever.
+int biot_handle::find_records()
+{
+  drop_records();
+  if (half() && n > (int64_t)1 << (prec == BIOT_FP16 ? 23 : 22)) return BIOT_OK;
+  const size_t values = (size_t)DICT_SLOTS * 24 * esz;
+  const size_t table = (size_t)DICT_SLOTS * sizeof(uint32_t);
+  if (hipMalloc((void **)&d_ids, (size_t)n * sizeof(uint16_t)) != hipSuccess ||
+      hipMalloc(&d_dict, values + table + 256) != hipSuccess) {
+    (void)hipGetLastError();
+    drop_records();
+    return BIOT_OK;
+  }
+  DictArgs a{};
+  a.coef = d_coef;
+  a.n = n;
+  a.ids = d_ids;
+  a.dv = d_dict;
+  a.dt = (char *)d_dict + (size_t)DICT_SLOTS * 16 * esz;
+  a.slots = (uint32_t *)((char *)d_dict + values);
+  a.state = (uint32_t *)((char *)d_dict + values + table);
+  uint32_t found[2] = {0, 0};
+  if (hipMemsetAsync(a.slots, 0xFF, table, stream) != hipSuccess ||
+      hipMemsetAsync(a.state, 0, sizeof found, stream) != hipSuccess ||
+      launch_dict(prec, a, stream) != hipSuccess ||
+      hipMemcpyAsync(found, a.state, sizeof found, hipMemcpyDeviceToHost, stream) != hipSuccess ||
+      hipStreamSynchronize(stream) != hipSuccess) {
+    drop_records();
+    err = "looking for the medium's distinct cells failed";
+    return BIOT_ERR_HIP;
+  }
+  if (found[1]) drop_records();
   return BIOT_OK;
 }
 
@@ -847,6 +902,7 @@ int biot_handle::upload_kernel_coefs(const std::vector<double> (&K_in)[NKC])
     have_coef = true;
     return BIOT_OK;
   }
+  drop_records();
   std::vector<double> K[NKC];
   for (int k = 0; k < NKC; ++k) {
     K[k] = K_in[k];

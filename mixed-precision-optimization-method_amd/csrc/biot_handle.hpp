@@ -25,6 +25,8 @@ struct biot_handle {
   int8_t *d_lo = nullptr;  // FP16C / FP16T residuals, 13 * n (compensated fields used); FP16M residual records, 4 * n
   void *d_coef = nullptr;            // 22 * n (FP16M: the medium records, 18 bytes per cell)
   void *d_kpack = nullptr;           // the coefficients packed per cell (velocity, then stress block)
+  uint16_t *d_ids = nullptr;         // a medium of few distinct cells: their records (StepArgs), else null
+  void *d_dict = nullptr;            // those records' values, and the table they were found in
   void *d_carry[3] = {nullptr, nullptr, nullptr};
   float *h_slice = nullptr;          // pinned, nx * nz: the slice of biot_snapshot_xz (made on first use)
   int *d_flag = nullptr;             // first step with a non-finite receiver sample
@@ -92,6 +94,8 @@ struct biot_handle {
   int upload_profiles();
   int upload_coefficients();
   int pack_coefficients();           // d_coef -> d_kpack
+  int find_records();                // d_coef -> d_ids, d_dict where the medium has few distinct cells
+  void drop_records();
   int build_adjoint_coefs();         // FP16M: d_kpack for the adjoint, from K_last
   int upload_kernel_coefs(const std::vector<double> (&K)[biot::NKC]);
   int upload_from_ref(const float *d_ref);      // 23 reference arrays on the device

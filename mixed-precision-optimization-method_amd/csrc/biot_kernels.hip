@@ -370,6 +370,26 @@ __device__ __forceinline__ void coef_block(const AT &a, const void *base, u32 c,
   }
 }
 
+// The N coefficients of record id of a medium of few distinct cells, at a stride of STRIDE stored
+// values: lanes of one record read the same 32 to 128 bytes, from the caches.
+template <class P, int N, int STRIDE, class AT>
+__device__ __forceinline__ void coef_record(const AT &a, const void *base, u32 id, int k0, typename P::A (&out)[N])
+{
+  using S = typename P::S;
+  using A = typename P::A;
+  constexpr int ND = N * (int)sizeof(S) / 4;
+  const char *p = reinterpret_cast<const char *>(base) + id * (u32)(STRIDE * sizeof(S));
+  uint32_t d[ND];
+#pragma unroll
+  for (int q = 0; q + 4 <= ND; q += 4) packed::ld_rec<4, false>(p + 4 * q, d + q);
+  packed::ld_rec<ND % 4, false>(p + 4 * (ND / 4 * 4), d + ND / 4 * 4);
+#pragma unroll
+  for (int e = 0; e < N; ++e) {
+    if constexpr (P::scaled) out[e] = (A)packed::value<S>(d, e) * a.ks[k0 + e];
+    else out[e] = (A)packed::value<S>(d, e);
+  }
+}
+
 // FP16M medium record of cell c: 4 binary16 values in 8 bytes (mv, mt)
 __device__ __forceinline__ float h2f(uint32_t d, int half)
 {
@@ -536,7 +556,8 @@ enum { FVX = 0, FVY, FVZ, FQX, FQY, FQZ, FTXX, FTYY, FTZZ, FTXY, FTXZ, FTYZ, FP 
 // one x-y tile of the update box, planes kb..ke-1 of z chunk tz
 // NT: the launch allows the policy's nontemporal accesses (the single-grid kernels; the
 // batched kernels, whose shot windows are reused from the caches, do not)
-template <class P, int ORDER, bool NT, bool OOP, class AT>
+// DICT: the coefficients come from the medium's records (StepArgs::ids)
+template <class P, int ORDER, bool NT, bool OOP, bool DICT, class AT>
 __device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int tz, uint64_t ioff, uint64_t ooff)
 {
   using A = typename P::A;
@@ -570,6 +591,10 @@ __device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int t
   const u32 wxs = (u32)(a.L[0] + a.R[0]), wys = (u32)(a.L[1] + a.R[1]);
   const u32 ny = (u32)a.ny, nx = (u32)a.nx;
   const u32 sl0 = (u32)a.slab[0], sl1 = (u32)a.slab[1], sl2 = (u32)a.slab[2];
+
+  // the cell's record, fetched a plane ahead: its values are then one load away, like the fields
+  u32 id1 = 0u;
+  if constexpr (DICT) id1 = at<uint16_t>(a.ids, col + (u32)kb * sz);
 
   // z windows: backward-differenced txz, tyz hold planes k-h..k+h-1,
   // forward-differenced tzz, p hold planes k-h+1..k+h.
@@ -605,6 +630,8 @@ __device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int t
   using SC = typename P::SC;
   for (int k = kb; k < ke; ++k) {
     const u32 c = col + (u32)k * sz;
+    const u32 id = id1;
+    if constexpr (DICT) id1 = at<uint16_t>(a.ids, c + sz);
     // twelve raw staggered differences (kernel.cu:172-185 without the 1/dx factor)
     A x1, x2, x3, s1, y1, y2, y3, s2, z1, z2, z3, s3;
     {
@@ -656,6 +683,8 @@ __device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int t
       mn[1] = med_rec(a.mv, c + sy);
       mn[2] = med_rec(a.mv, c + sz);
       medium_velocity(a, mown, mn, kv);
+    } else if constexpr (DICT) {
+      coef_record<P, 14, 16>(a, a.dv, id, 0, kv);
     } else {
       coef_block<P, 14>(a, a.kv, c, 0, kv);
     }
@@ -741,7 +770,7 @@ __device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int t
 
 // one x-y tile of the update box, planes kb..ke-1 of z chunk tz; true in the thread that updated
 // the source cell
-template <class P, int ORDER, bool NT, bool OOP, class AT>
+template <class P, int ORDER, bool NT, bool OOP, bool DICT, class AT>
 __device__ __forceinline__ bool stress_tile(const AT &a, int tx, int ty, int tz, uint64_t ioff, uint64_t ooff)
 {
   using A = typename P::A;
@@ -777,6 +806,10 @@ __device__ __forceinline__ bool stress_tile(const AT &a, int tx, int ty, int tz,
   const u32 ny = (u32)a.ny, nx = (u32)a.nx;
   const u32 sl0 = (u32)a.slab[0], sl1 = (u32)a.slab[1], sl2 = (u32)a.slab[2];
 
+  // the cell's record, fetched a plane ahead: its values are then one load away, like the fields
+  u32 id1 = 0u;
+  if constexpr (DICT) id1 = at<uint16_t>(a.ids, col + (u32)kb * sz);
+
   // z windows: backward-differenced vz, qz hold planes k-h..k+h-1,
   // forward-differenced vx, vy hold planes k-h+1..k+h.
   A wvz[W], wqz[W], wvx[W], wvy[W];
@@ -796,6 +829,8 @@ __device__ __forceinline__ bool stress_tile(const AT &a, int tx, int ty, int tz,
   using SC = typename P::SC;
   for (int k = kb; k < ke; ++k) {
     const u32 c = col + (u32)k * sz;
+    const u32 id = id1;
+    if constexpr (DICT) id1 = at<uint16_t>(a.ids, c + sz);
     wvz[W - 1] = L<P, FVZ>(vo, c + (u32)(h - 1) * sz);
     wqz[W - 1] = L<P, FQZ>(vo, c + (u32)(h - 1) * sz);
     wvx[W - 1] = L<P, FVX>(vo, c + (u32)h * sz);
@@ -822,6 +857,7 @@ __device__ __forceinline__ bool stress_tile(const AT &a, int tx, int ty, int tz,
     const A txz0 = LO<P, FTXZ, (P::nt_t && NT)>(vi, c);
     A kt[8];  // K[14..21]: P1, P2, S1, S2, S3, Sxy, Sxz, Syz
     if constexpr (P::medium) medium_stress(a, c, sy, sz, rq, kt);
+    else if constexpr (DICT) coef_record<P, 8, 8>(a, a.dt, id, K_P1, kt);
     else coef_block<P, 8>(a, a.kt, c, K_P1, kt);
     const A s1 = kt[K_S1 - K_P1], s2 = kt[K_S2 - K_P1], s3 = kt[K_S3 - K_P1];
     const A kp1 = kt[0], kp2 = kt[K_P2 - K_P1];
@@ -1006,7 +1042,7 @@ __device__ __forceinline__ __attribute__((address_space(4))) const T *late_args(
 
 // OOP: the half step reads state u.q of a run of states at the arguments' pointers and writes state
 // u.q + 1
-template <class P, int ORDER, bool OOP>
+template <class P, int ORDER, bool OOP, bool DICT>
 __global__ void __launch_bounds__(256) k_velocity(const StepArgs a, const FuseArgs u)
 {
   const uint64_t ioff = OOP ? (uint64_t)u.q * a.sb : 0, ooff = OOP ? ioff + a.sb : 0;
@@ -1016,9 +1052,9 @@ __global__ void __launch_bounds__(256) k_velocity(const StepArgs a, const FuseAr
   }
   int tx, ty, tz;
   if (!tile_of(a, tx, ty, tz)) return;
-  velocity_tile<P, ORDER, true, OOP>(a, tx, ty, tz, ioff, ooff);
+  velocity_tile<P, ORDER, true, OOP, DICT>(a, tx, ty, tz, ioff, ooff);
 }
-template <class P, int ORDER, bool OOP>
+template <class P, int ORDER, bool OOP, bool DICT>
 __global__ void __launch_bounds__(256) k_stress(const StepArgs a, const FuseArgs u)
 {
   const uint64_t ioff = OOP ? (uint64_t)u.q * a.sb : 0, ooff = OOP ? ioff + a.sb : 0;
@@ -1028,7 +1064,7 @@ __global__ void __launch_bounds__(256) k_stress(const StepArgs a, const FuseArgs
   }
   int tx, ty, tz;
   if (!tile_of(a, tx, ty, tz)) return;
-  if (!stress_tile<P, ORDER, true, OOP>(a, tx, ty, tz, ioff, ooff)) return;
+  if (!stress_tile<P, ORDER, true, OOP, DICT>(a, tx, ty, tz, ioff, ooff)) return;
   // the arguments of what follows are read here, so that none of them is kept in scalar registers
   // over the plane loop (kept, they spilled 16 more of the FP16T kernel's)
   CStepArgs *a1 = late_args<StepArgs>();
@@ -1064,8 +1100,8 @@ __device__ __forceinline__ void batch_tile(const BatchArgs &b, int t)
   const int tx = lt % a.gx, r = lt / a.gx, ty = r % a.gy, tz = r / a.gy;
   const uint64_t ioff = OOP ? (uint64_t)b.q * a.sb : 0, ooff = OOP ? ioff + a.sb : 0;
   if constexpr (VEL) {
-    velocity_tile<P, ORDER, false, OOP>(a, tx, ty, tz, ioff, ooff);
-  } else if (stress_tile<P, ORDER, false, OOP>(a, tx, ty, tz, ioff, ooff)) {
+    velocity_tile<P, ORDER, false, OOP, false>(a, tx, ty, tz, ioff, ooff);
+  } else if (stress_tile<P, ORDER, false, OOP, false>(a, tx, ty, tz, ioff, ooff)) {
     CBatchArgs &b1 = *late_args<BatchArgs>();
     const int s1 = shot_of(b1, t);
     CSourceArgs &sa = ((CSourceArgs *)b1.src)[s1];
@@ -1277,10 +1313,17 @@ hipError_t launch_step(const StepArgs &in, LaunchShape sh, hipStream_t s, const 
   if (u.source) u.src = *src;
   const int64_t rb = u.record ? (rec->nrec + sh.bx * sh.by - 1) / (sh.bx * sh.by) : 0;
   dim3 grid((unsigned)(u.tile_blocks + rb));
-  if (VEL && q >= 0) hipLaunchKernelGGL((k_velocity<P, ORDER, true>), grid, block, 0, s, a, u);
-  else if (VEL) hipLaunchKernelGGL((k_velocity<P, ORDER, false>), grid, block, 0, s, a, u);
-  else if (q >= 0) hipLaunchKernelGGL((k_stress<P, ORDER, true>), grid, block, 0, s, a, u);
-  else hipLaunchKernelGGL((k_stress<P, ORDER, false>), grid, block, 0, s, a, u);
+  if constexpr (!P::medium) {
+    if (q < 0 && a.ids) {
+      if (VEL) hipLaunchKernelGGL((k_velocity<P, ORDER, false, true>), grid, block, 0, s, a, u);
+      else hipLaunchKernelGGL((k_stress<P, ORDER, false, true>), grid, block, 0, s, a, u);
+      return hipGetLastError();
+    }
+  }
+  if (VEL && q >= 0) hipLaunchKernelGGL((k_velocity<P, ORDER, true, false>), grid, block, 0, s, a, u);
+  else if (VEL) hipLaunchKernelGGL((k_velocity<P, ORDER, false, false>), grid, block, 0, s, a, u);
+  else if (q >= 0) hipLaunchKernelGGL((k_stress<P, ORDER, true, false>), grid, block, 0, s, a, u);
+  else hipLaunchKernelGGL((k_stress<P, ORDER, false, false>), grid, block, 0, s, a, u);
   return hipGetLastError();
 }
 
