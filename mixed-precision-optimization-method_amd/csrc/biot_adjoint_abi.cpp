@@ -268,19 +268,23 @@ extern "C" int biot_adjoint(biot_handle *h, const float *adj_source, double *con
     c.Cp = s.Cp;
     c.Hinv = s.Hinv;
     AHIP(h, launch_chain(c, h->stream));
-    AHIP(h, hipStreamSynchronize(h->stream));
-    for (int q = 0; q < 6; ++q)
-      AHIP(h, hipMemcpy(grad_params[q], out + (size_t)q * n, (size_t)n * sizeof(double), hipMemcpyDeviceToHost));
+    std::vector<ReadBack::Piece> pieces;
+    for (int q = 0; q < 6; ++q) pieces.push_back({grad_params[q], out + (size_t)q * n, (size_t)n * sizeof(double)});
+    if (!h->back.read(pieces, h->g.device, h->stream)) return afail(h, BIOT_ERR_HIP, "reading the gradients failed");
   }
   AHIP(h, hipEventSynchronize(h->ev1));
   float ms = 0;
   AHIP(h, hipEventElapsedTime(&ms, h->ev0, h->ev1));
   h->last_ms = ms;
   // coefficient gradients: storage units times the per-array factor
+  std::vector<ReadBack::Piece> pieces;
+  for (int k = 0; k < NKC && grad_coef; ++k)
+    if (grad_coef[k]) pieces.push_back({grad_coef[k], h->d_grad + (size_t)k * n, (size_t)n * sizeof(double)});
+  if (!pieces.empty() && !h->back.read(pieces, h->g.device, h->stream))
+    return afail(h, BIOT_ERR_HIP, "reading the gradients failed");
   for (int k = 0; k < NKC && grad_coef; ++k) {
     double *g = grad_coef[k];
     if (!g) continue;
-    AHIP(h, hipMemcpy(g, h->d_grad + (size_t)k * n, (size_t)n * sizeof(double), hipMemcpyDeviceToHost));
     if (h->kfac[k] != 1.0)
       for (int64_t c = 0; c < n; ++c) g[c] *= h->kfac[k];
   }

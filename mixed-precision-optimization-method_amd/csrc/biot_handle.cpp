@@ -8,6 +8,8 @@
 #include <cstdlib>
 #include <cstring>
 #include <memory>
+#include <system_error>
+#include <thread>
 
 using namespace biot;
 
@@ -139,6 +141,60 @@ size_t biot_handle::lam_bytes() const
   return b + 256;
 }
 
+ReadBack::~ReadBack()
+{
+  if (pinned) (void)hipHostFree(pinned);
+}
+
+bool ReadBack::read(const std::vector<Piece> &pieces, int device, hipStream_t s)
+{
+  size_t chunks = 0;
+  for (const Piece &p : pieces) chunks += (p.bytes + CHUNK - 1) / CHUNK;
+  if (chunks > 1 && !pinned && hipHostMalloc((void **)&pinned, THREADS * CHUNK, hipHostMallocDefault) != hipSuccess) {
+    pinned = nullptr;
+    (void)hipGetLastError();
+  }
+  if (chunks <= 1 || !pinned) {
+    if (hipStreamSynchronize(s) != hipSuccess) return false;
+    for (const Piece &p : pieces)
+      if (p.bytes && hipMemcpy(p.dst, p.src, p.bytes, hipMemcpyDeviceToHost) != hipSuccess) return false;
+    return true;
+  }
+  std::atomic<size_t> next{0};
+  std::atomic<bool> ok{true};
+  auto work = [&](int t) {
+    char *mine = pinned + (size_t)t * CHUNK;
+    hipEvent_t ev = nullptr;
+    if ((t > 0 && hipSetDevice(device) != hipSuccess) ||
+        hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
+      ok = false;
+      return;
+    }
+    for (size_t c; ok && (c = next.fetch_add(1)) < chunks;) {
+      size_t q = 0;
+      for (size_t k; c >= (k = (pieces[q].bytes + CHUNK - 1) / CHUNK); ++q) c -= k;
+      const size_t off = c * CHUNK, len = std::min(CHUNK, pieces[q].bytes - off);
+      if (hipMemcpyAsync(mine, (const char *)pieces[q].src + off, len, hipMemcpyDeviceToHost, s) != hipSuccess ||
+          hipEventRecord(ev, s) != hipSuccess || hipEventSynchronize(ev) != hipSuccess) {
+        ok = false;
+        break;
+      }
+      std::memcpy((char *)pieces[q].dst + off, mine, len);
+    }
+    (void)hipEventDestroy(ev);
+  };
+  std::vector<std::thread> pool;
+  try {
+    for (int t = 1; t < THREADS && (size_t)t < chunks; ++t) pool.emplace_back(work, t);
+  } catch (const std::system_error &) {  // fewer threads, then
+  }
+  work(0);
+  for (auto &th : pool) th.join();
+  // a copy into the buffers that was queued before a failure ends before anyone uses them again
+  if (!ok) (void)hipStreamSynchronize(s);
+  return ok;
+}
+
 int biot_handle::alloc_adjoint(int every)
 {
   const int64_t m = (int64_t)ncomp * nt_max * nrec;
@@ -146,7 +202,13 @@ int biot_handle::alloc_adjoint(int every)
   // 32-bit byte offsets from its base, as the forward kernels do their arrays
   const int64_t asz = prec == BIOT_FP64 ? 8 : 4, lim = (int64_t)1 << 32;
   bool fits = n * asz < lim;
+  if (every > 0 && d_slots && slots_every != every) {
+    (void)hipStreamSynchronize(stream);
+    (void)hipFree(d_slots);
+    d_slots = nullptr;
+  }
   const bool new_slots = every > 0 && !d_slots;
+  if (new_slots) slots_every = every;
   for (int ax = 0; ax < 3; ++ax) fits = fits && NCARRY * slab[ax] * asz < lim;
   if (!fits) {
     err = "grid too large for the adjoint (an adjoint array would exceed 4 GiB)";
