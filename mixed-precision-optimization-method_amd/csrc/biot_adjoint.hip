@@ -129,17 +129,20 @@ struct CellIdx {
   u32 c;
 };
 
-// update-box cell t (x fastest)
+// the cell of thread t of block blk (AdjArgs: ADJ_BX consecutive cells of an x-y plane in ADJ_BZ
+// planes); false outside the update box
 template <class AT>
-__device__ __forceinline__ bool cell_of(const AT &a, int h, u32 t, CellIdx &ci)
+__device__ __forceinline__ bool cell_of(const AT &a, int h, u32 blk, u32 t, CellIdx &ci)
 {
-  const u32 ni = (u32)(a.nx - 2 * h), nj = (u32)(a.ny - 2 * h);
-  ci.i = h + (int)(t % ni);
-  const u32 r = t / ni;
-  ci.j = h + (int)(r % nj);
-  ci.k = h + (int)(r / nj);
-  ci.c = (u32)ci.i + (u32)ci.j * (u32)a.sy + (u32)ci.k * (u32)a.sz;
-  return ci.k < a.nz - h;
+  const u32 tz = blk / (u32)a.gx, tx = blk - tz * (u32)a.gx;
+  const u32 l = (u32)a.xy0 + tx * ADJ_BX + t % ADJ_BX;
+  u32 q = __umulhi(l, a.nx_rcp);
+  if (q * (u32)a.nx > l) --q;
+  ci.j = (int)q;
+  ci.i = (int)(l - q * (u32)a.nx);
+  ci.k = h + (int)(tz * ADJ_BZ + t / ADJ_BX);
+  ci.c = l + (u32)ci.k * (u32)a.sz;
+  return ci.i >= h && ci.i < a.nx - h && ci.j >= h && ci.j < a.ny - h && ci.k < a.nz - h;
 }
 
 template <class AT>
@@ -420,12 +423,12 @@ __device__ __forceinline__ void phase() { __builtin_amdgcn_sched_barrier(0); }
 // lambda(tau, p) += transposed differences of the velocity-half G of the step after; then the local
 // part of the stress half of state q's step
 template <typename S, int ORDER, class AT, class IT>
-__device__ __forceinline__ void adj_stress(const AT &a, const IT &j, int q, int it, u32 t)
+__device__ __forceinline__ void adj_stress(const AT &a, const IT &j, int q, int it, u32 blk, u32 t)
 {
   using A = typename AdjT<S>::A;
   constexpr int h = ORDER / 2;
   CellIdx ci;
-  if (t >= a.nupd || !cell_of(a, h, t, ci)) return;
+  if (!cell_of(a, h, blk, t, ci)) return;
   const u32 c = ci.c;
   A l[7];  // txx tyy tzz txy txz tyz p
 #pragma unroll
@@ -491,12 +494,12 @@ __device__ __forceinline__ void adj_stress(const AT &a, const IT &j, int q, int 
 // lambda(v', q') += transposed differences of the stress-half G; then the local part of the
 // velocity half of state q's step
 template <typename S, int ORDER, class AT, class IT>
-__device__ __forceinline__ void adj_velocity(const AT &a, const IT &j, int q, int it, u32 t)
+__device__ __forceinline__ void adj_velocity(const AT &a, const IT &j, int q, int it, u32 blk, u32 t)
 {
   using A = typename AdjT<S>::A;
   constexpr int h = ORDER / 2;
   CellIdx ci;
-  if (t >= a.nupd || !cell_of(a, h, t, ci)) return;
+  if (!cell_of(a, h, blk, t, ci)) return;
   const u32 c = ci.c;
   constexpr int kU1[3] = {K_U1X, K_U1Y, K_U1Z}, kU2[3] = {K_U2X, K_U2Y, K_U2Z};
   constexpr int kW1[3] = {K_W1X, K_W1Y, K_W1Z}, kW2[3] = {K_W2X, K_W2Y, K_W2Z};
@@ -581,11 +584,11 @@ __device__ __forceinline__ void adj_velocity(const AT &a, const IT &j, int q, in
 
 // the float partial sums of a segment into the FP64 gradient sums, cleared for the next one
 template <typename S, int ORDER, class AT>
-__device__ __forceinline__ void adj_flush(const AT &a, u32 t)
+__device__ __forceinline__ void adj_flush(const AT &a, u32 blk, u32 t)
 {
   constexpr int h = ORDER / 2;
   CellIdx ci;
-  if (t >= a.nupd || !cell_of(a, h, t, ci)) return;
+  if (!cell_of(a, h, blk, t, ci)) return;
   const u32 c = ci.c;
   const uint64_t n = (uint64_t)a.nx * a.ny * a.nz;
   uint32_t dv[14], dt[8];
@@ -604,18 +607,19 @@ __device__ __forceinline__ void adj_flush(const AT &a, u32 t)
 
 // WHICH 0: the stress pass, 1: the velocity pass, 2: the flush
 template <typename S, int ORDER, int WHICH, class AT, class IT>
-__device__ __forceinline__ void adj_pass(const AT &a, const IT &j, int q, int it, u32 t)
+__device__ __forceinline__ void adj_pass(const AT &a, const IT &j, int q, int it, u32 blk, u32 t)
 {
-  if constexpr (WHICH == 0) adj_stress<S, ORDER>(a, j, q, it, t);
-  else if constexpr (WHICH == 1) adj_velocity<S, ORDER>(a, j, q, it, t);
-  else adj_flush<S, ORDER>(a, t);
+  if constexpr (WHICH == 0) adj_stress<S, ORDER>(a, j, q, it, blk, t);
+  else if constexpr (WHICH == 1) adj_velocity<S, ORDER>(a, j, q, it, blk, t);
+  else adj_flush<S, ORDER>(a, blk, t);
 }
 
 // 256 cells a block, dealt out to the XCDs in runs of blocks as the forward kernels' tiles are
 template <typename S, int ORDER, int WHICH>
-__global__ void __launch_bounds__(256) k_adj(const AdjArgs a, const InjectArgs j, int q, int it, int xg)
+__global__ void __launch_bounds__(ADJ_BX * ADJ_BZ) k_adj(const AdjArgs a, const InjectArgs j, int q, int it, int xg)
 {
-  adj_pass<S, ORDER, WHICH>(a, j, q, it, (u32)xcd_tile(blockIdx.x & 7, blockIdx.x >> 3, xg) * 256u + threadIdx.x);
+  const u32 blk = (u32)xcd_tile(blockIdx.x & 7, blockIdx.x >> 3, xg);
+  if (blk < (u32)a.blocks) adj_pass<S, ORDER, WHICH>(a, j, q, it, blk, threadIdx.x);
 }
 
 // batched: argument tables read through the constant address space (uniform per block)
@@ -637,15 +641,14 @@ __device__ __forceinline__ int shot_of_block(const AdjBatch &b, int blk)
 }
 
 template <typename S, int ORDER, int WHICH>
-__global__ void __launch_bounds__(256) k_adj_batch(const AdjBatch b, int q, int it, int xg)
+__global__ void __launch_bounds__(ADJ_BX * ADJ_BZ) k_adj_batch(const AdjBatch b, int q, int it, int xg)
 {
   const int blk = xcd_tile(blockIdx.x & 7, blockIdx.x >> 3, xg);
   if (blk >= b.total_blocks) return;
   const int s = shot_of_block(b, blk);
   const CAdjArgs &a = ((CAdjArgs *)b.shots)[s];
   const CInjectArgs &j = ((CInjectArgs *)b.inject)[s];
-  const u32 t = (u32)(blk - ((CInt *)b.block_start)[s]) * 256u + threadIdx.x;
-  adj_pass<S, ORDER, WHICH>(a, j, q, it, t);
+  adj_pass<S, ORDER, WHICH>(a, j, q, it, (u32)(blk - ((CInt *)b.block_start)[s]), threadIdx.x);
 }
 
 // J = 1/2 sum (d - obs)^2 in FP64, residual = d - obs
@@ -819,9 +822,9 @@ struct SingleRun {
   template <typename S, int O, int W>
   void pass()
   {
-    const int64_t n = ((int64_t)a.nupd + 255) / 256;
-    const int xg = xcd_run(n, 256, n * 256);
-    hipLaunchKernelGGL((k_adj<S, O, W>), dim3((unsigned)(8 * xcd_slots(n, xg))), dim3(256), 0, s, a, j, q, it, xg);
+    const int xg = xcd_run(a.blocks, ADJ_BX * ADJ_BZ, (int64_t)a.blocks * ADJ_BX * ADJ_BZ);
+    hipLaunchKernelGGL((k_adj<S, O, W>), dim3((unsigned)(8 * xcd_slots(a.blocks, xg))), dim3(ADJ_BX * ADJ_BZ), 0, s, a,
+                       j, q, it, xg);
   }
 };
 struct BatchRun {
@@ -831,8 +834,8 @@ struct BatchRun {
   template <typename S, int O, int W>
   void pass()
   {
-    const int xg = xcd_run(b.total_blocks, 256, (int64_t)b.total_blocks * 256);
-    hipLaunchKernelGGL((k_adj_batch<S, O, W>), dim3((unsigned)(8 * xcd_slots(b.total_blocks, xg))), dim3(256), 0, s, b,
+    const int xg = xcd_run(b.total_blocks, ADJ_BX * ADJ_BZ, (int64_t)b.total_blocks * ADJ_BX * ADJ_BZ);
+    hipLaunchKernelGGL((k_adj_batch<S, O, W>), dim3((unsigned)(8 * xcd_slots(b.total_blocks, xg))), dim3(ADJ_BX * ADJ_BZ), 0, s, b,
                        q, it, xg);
   }
 };
@@ -869,13 +872,13 @@ hipError_t passes(int prec, int order, F f, bool flush)
 
 hipError_t launch_adjoint_step(int prec, int order, const AdjArgs &a, const InjectArgs &j, int q, int it, hipStream_t s)
 {
-  if (a.nupd == 0) return hipSuccess;
+  if (a.blocks == 0) return hipSuccess;
   return passes(prec, order, SingleRun{a, j, q, it, s}, false);
 }
 
 hipError_t launch_adjoint_flush(int prec, int order, const AdjArgs &a, hipStream_t s)
 {
-  if (a.nupd == 0 || prec == PREC_FP64) return hipSuccess;
+  if (a.blocks == 0 || prec == PREC_FP64) return hipSuccess;
   return passes(prec, order, SingleRun{a, InjectArgs{}, 0, 0, s}, true);
 }
 

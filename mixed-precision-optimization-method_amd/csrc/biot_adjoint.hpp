@@ -9,6 +9,14 @@
 
 namespace biot {
 
+// A block of the adjoint passes: ADJ_BX consecutive cells of an x-y plane, the plane's first block
+// starting on a 64-cell boundary, in ADJ_BZ planes.  Runs of the update box's own cells left every wave
+// two cells off its cache lines; with these the two passes take (us a step, before / after) 329 / 320 at
+// 128^3 FP32, 1023 / 1000 at 192^3 FP32, 100 / 92 at 96x80x89 FP16M, 284 / 280 at 110x99x83 FP64.  256
+// cells of one plane: 317, 986, 93, 281, and 2 % slower than before at 75^3 (128 x 2: 2 % faster); blocks
+// of 512 and blocks that end each axis's loads together, for the rows they share, are slower: the
+// passes are bound by the 360 and 265 bytes a cell (FP32) that they move, at 4.1 TB/s.
+constexpr uint32_t ADJ_BX = 128, ADJ_BZ = 2;
 // Per-grid adjoint arguments.  The forward states of a recomputed segment sit in `slots`
 // (state q at slots + q*sb: the fields block, field f at f*fbytes, then the carry blocks at
 // coff[0..2]); the adjoint step of segment step q reads state q (after its source) and the
@@ -41,7 +49,8 @@ struct AdjArgs {
   int L[3], R[3];
   int64_t slab[3];
   int64_t sy, sz;
-  uint32_t nupd;             // cells of the update box
+  int blocks, gx, xy0;       // blocks; those of ADJ_BZ planes; the plane cell the first one starts at
+  uint32_t nx_rcp;           // ceil(2^32 / nx)
 };
 
 // The adjoint sources: a bit per cell tells the thread that updates a cell whether receivers sit

@@ -632,7 +632,7 @@ int gradient_group(biot_batch *b, int s0, int s1, int nt, int every, const float
     for (int i = 0; i < S; ++i) {
       b->shots[s0 + i].h->adj_args(adj[i]);
       b->shots[s0 + i].h->inject_args(inj[i]);
-      bs[i + 1] = bs[i] + (int)((adj[i].nupd + 255) / 256);
+      bs[i + 1] = bs[i] + adj[i].blocks;
     }
     b->adj_blocks = bs[S];
     if (!b->d_adj) BHIP(b, hipMalloc((void **)&b->d_adj, S * sizeof(AdjArgs)));

@@ -329,7 +329,11 @@ void biot_handle::adj_args(AdjArgs &A) const
   A.nz = g.nz;
   A.sy = g.nx;
   A.sz = (int64_t)g.nx * g.ny;
-  A.nupd = (uint32_t)((int64_t)(g.nx - 2 * hh) * (g.ny - 2 * hh) * (g.nz - 2 * hh));
+  A.xy0 = (hh * g.nx) & ~63;
+  A.nx_rcp = (uint32_t)((((uint64_t)1 << 32) + (uint64_t)g.nx - 1) / (uint64_t)g.nx);
+  A.gx = (int)(((int64_t)(g.ny - hh) * g.nx - A.xy0 + ADJ_BX - 1) / ADJ_BX);
+  const bool empty = g.nx <= 2 * hh || g.ny <= 2 * hh || g.nz <= 2 * hh;
+  A.blocks = empty ? 0 : A.gx * ((g.nz - 2 * hh + ADJ_BZ - 1) / ADJ_BZ);
 }
 
 // The six gradient outputs go over the float partial sums (88 n bytes, flushed by now) or, on
