@@ -195,6 +195,28 @@ bool ReadBack::read(const std::vector<Piece> &pieces, int device, hipStream_t s)
   return ok;
 }
 
+int biot_handle::alloc_slots(int every)
+{
+  if (d_slots && slots_every == every) return BIOT_OK;
+  slots_seg = -1;
+  if (d_slots) {
+    (void)hipStreamSynchronize(stream);
+    (void)hipFree(d_slots);
+  }
+  slots_every = every;
+  if (hipMalloc(&d_slots, state_bytes() * (size_t)(every + 1)) != hipSuccess) {
+    d_slots = nullptr;
+    err = "adjoint buffers do not fit in device memory";
+    return BIOT_ERR_NOMEM;
+  }
+  const int rc = clear_borders((char *)d_slots, every + 1);
+  if (rc) {
+    (void)hipFree(d_slots);
+    d_slots = nullptr;
+  }
+  return rc;
+}
+
 int biot_handle::alloc_adjoint(int every)
 {
   const int64_t m = (int64_t)ncomp * nt_max * nrec;
@@ -202,13 +224,6 @@ int biot_handle::alloc_adjoint(int every)
   // 32-bit byte offsets from its base, as the forward kernels do their arrays
   const int64_t asz = prec == BIOT_FP64 ? 8 : 4, lim = (int64_t)1 << 32;
   bool fits = n * asz < lim;
-  if (every > 0 && d_slots && slots_every != every) {
-    (void)hipStreamSynchronize(stream);
-    (void)hipFree(d_slots);
-    d_slots = nullptr;
-  }
-  const bool new_slots = every > 0 && !d_slots;
-  if (new_slots) slots_every = every;
   for (int ax = 0; ax < 3; ++ax) fits = fits && NCARRY * slab[ax] * asz < lim;
   if (!fits) {
     err = "grid too large for the adjoint (an adjoint array would exceed 4 GiB)";
@@ -222,15 +237,15 @@ int biot_handle::alloc_adjoint(int every)
     }
     return true;
   };
-  if ((every > 0 && !get(&d_slots, state_bytes() * (size_t)(every + 1))) || !get(&d_lam, lam_bytes()) ||
+  if (every > 0)
+    if (int rc = alloc_slots(every)) return rc;
+  if (!get(&d_lam, lam_bytes()) ||
       !get((void **)&d_grad, (size_t)NKC * n * sizeof(double)) ||
       (prec != BIOT_FP64 && !get((void **)&d_gpart, (size_t)NKC * n * sizeof(float))) ||
       !get((void **)&d_adjsrc, (size_t)std::max<int64_t>(m, 1) * sizeof(float))) {
     err = "adjoint buffers do not fit in device memory";
     return BIOT_ERR_NOMEM;
   }
-  if (new_slots)
-    if (int rc = clear_borders((char *)d_slots, every + 1)) return rc;
   return build_inject();
 }
 
@@ -392,6 +407,7 @@ void biot_handle::free_adjoint()
     if (p) (void)hipFree(p);
   ckpt.clear();
   ckpt_every = ckpt_nt = room_every = room_nt = 0;
+  slots_seg = -1;
   if (prec == BIOT_FP16M && d_kpack) {  // the adjoint's coefficient copy of the last parameters
     (void)hipFree(d_kpack);
     d_kpack = nullptr;

@@ -132,6 +132,7 @@ struct biot_handle {
   // in place of segment recomputation
   void *d_slots = nullptr;                   // segment states (slots_every + 1), zero outside the update box
   int slots_every = 0;
+  int slots_seg = -1;                        // the checkpoint segment whose states d_slots holds, or -1
   void *d_lam = nullptr;                     // adjoint fields, carries, derivative adjoints
   double *d_grad = nullptr;                  // 22 FP64 coefficient gradients
   float *d_gpart = nullptr;                  // 22 float per-segment partial sums (not FP64 handles)
@@ -168,6 +169,7 @@ struct biot_handle {
   int clear_nonfinite();                     // enqueue a clear of d_flag on the stream
   int check_nonfinite();                     // synchronize; BIOT_ERR_NONFINITE if it was set
   size_t lam_bytes() const;                  // adjoint wavefields, carries, derivative adjoints
+  int alloc_slots(int every);                // d_slots
   int alloc_adjoint(int every);              // d_slots (every+1 states; none for 0), d_lam, d_grad, d_adjsrc, d_inj
   int build_inject();                        // d_inj from rec_cells
   void adj_args(biot::AdjArgs &A) const;     // after alloc_adjoint

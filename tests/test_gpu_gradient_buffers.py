@@ -3,11 +3,14 @@ batch whose buffers served other gradients (other data, steps, checkpoints, anot
 shot's own handle, a release in between) gives what a new batch gives: the same launches on the same
 values, so the gradients are equal bit for bit (J to 1e-12: its sum's order is free).  Gradients of
 sizes around the parts in which they are read back (2^18 doubles) equal the host's chain rule of the
-coefficient gradients of the same call, to 1e-12 as sums of up to 30 doubles in another order do."""
+coefficient gradients of the same call, to 1e-12 as sums of up to 30 doubles in another order do.  The
+last segment's states are the forward run's own or recomputed ones, equal bit for bit: a second sweep
+over the same checkpoints, which finds the first segment's states in their place, gives the same
+gradients, and the run that kept them the plain run's traces and fields."""
 import numpy as np
 import pytest
 
-from biot_amd import Solver, _lib, media, ricker
+from biot_amd import FIELDS, Solver, _lib, media, ricker
 from biot_amd._lib import PARAM_NAMES
 from biot_amd.batch import Batch
 from conftest import rel_l2
@@ -83,3 +86,32 @@ def test_gradients_read_back_whole(size):
     ref = _lib.params_chain(nx, ny, nz, 5.0, 4e-4, p, gk)
     for k, r in zip(PARAM_NAMES, ref):
         assert np.any(r.ravel()[-nx * ny * 4:]) and rel_l2(g[k].ravel(), r) <= 1e-12, k
+
+
+@pytest.mark.parametrize("precision,every", [("fp32", 7), ("fp64", 5), ("fp16t", 14), ("fp16m", 20), ("fp16", 13),
+                                             ("fp16c", 6)])
+def test_last_segment_of_the_forward_run_serves_the_sweep(precision, every):
+    nx, ny, nz, nt = 34, 25, 29, 14
+    print(f"last segment {precision} every {every}", flush=True)
+    rng = np.random.default_rng(3)
+    p = {k: v * rng.uniform(0.9, 1.1, (nz, ny, nx))
+         for k, v in media.params_from_medium(media.homogeneous((nz, ny, nx))).items()}
+    s = Solver(nx, ny, nz, 5.0, 4e-4, precision=precision, npml=4)
+    s.set_source(s.cell(nx // 2, ny // 2, nz // 2), ricker(60.0, 4e-4, nt) + 1.0, ("txx", "tyy", "tzz", "p"))
+    s.set_params(p)
+    s.set_receivers(rng.choice(nx * ny * nz, 40, replace=False), ("vx", "vz", "p"), nt)
+    s.reset()
+    s.run(nt)
+    plain = [s.traces()] + [s.field(f, f64=True) for f in FIELDS]
+    y = rng.standard_normal((3, nt, 40)).astype(np.float32)
+    first = None
+    for _ in range(2):  # the second run in the buffers of the first
+        s.forward_checkpointed(nt, every)
+        for a, b in zip(plain, [s.traces()] + [s.field(f, f64=True) for f in FIELDS]):
+            assert np.array_equal(a, b)
+        for _ in range(2):
+            g = s.adjoint(y)[0]
+            first = first or g
+            for k in PARAM_NAMES:
+                assert np.any(g[k]) and np.array_equal(g[k], first[k]), k
+    s.close()
