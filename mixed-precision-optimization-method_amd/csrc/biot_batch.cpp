@@ -63,8 +63,9 @@ struct biot_batch {
   int *d_blocks = nullptr;
   InjectArgs *d_inj = nullptr;
   CopyEntry *d_copy = nullptr;
-  StepArgs *d_step_s = nullptr;    // d_step and d_src over the segment states
+  StepArgs *d_step_s = nullptr;    // d_step, d_src and d_rec over the segment states
   SourceArgs *d_src_s = nullptr;
+  RecordArgs *d_rec_s = nullptr;
   int adj_blocks = 0;
   double *d_gout = nullptr;        // 6 model-grid arrays
   double *d_J = nullptr;
@@ -150,6 +151,7 @@ void biot_batch::free_gradient()
   dfree(d_copy);
   dfree(d_step_s);
   dfree(d_src_s);
+  dfree(d_rec_s);
   dfree(d_gout);
   dfree(d_J);
 }
@@ -644,23 +646,28 @@ int gradient_group(biot_batch *b, int s0, int s1, int nt, int every, const float
     // the half steps' and sources' arguments over the segment states
     std::vector<StepArgs> st(S);
     std::vector<SourceArgs> src(S);
+    std::vector<RecordArgs> rec(S);
     for (int i = 0; i < S; ++i) {
       biot_handle *h = b->shots[s0 + i].h;
       h->fill_args(st[i], (char *)h->d_slots);
       set_tiles(st[i], b->shape, order / 2);
       h->source_args(src[i], (char *)h->d_slots);
+      h->record_args(rec[i], (char *)h->d_slots);
     }
     if (!b->d_step_s) BHIP(b, hipMalloc((void **)&b->d_step_s, S * sizeof(StepArgs)));
     if (!b->d_src_s) BHIP(b, hipMalloc((void **)&b->d_src_s, S * sizeof(SourceArgs)));
     BHIP(b, hipMemcpy(b->d_step_s, st.data(), S * sizeof(StepArgs), hipMemcpyHostToDevice));
+    if (!b->d_rec_s) BHIP(b, hipMalloc((void **)&b->d_rec_s, S * sizeof(RecordArgs)));
     BHIP(b, hipMemcpy(b->d_src_s, src.data(), S * sizeof(SourceArgs), hipMemcpyHostToDevice));
+    BHIP(b, hipMemcpy(b->d_rec_s, rec.data(), S * sizeof(RecordArgs), hipMemcpyHostToDevice));
   }
   // copy tables: [save ckpt k] nseg entries of 5 pieces per shot (fields, the three carry blocks,
-  // the residuals: 0 bytes on the policies without), [ckpt k to the first segment state] nseg of one
+  // the residuals: 0 bytes on the policies without), [ckpt k to the first segment state] nseg of one,
+  // [the last segment's last state to the live arrays] 5 pieces per shot
   constexpr int NP = 5;
   const int per = NP * S;
   {
-    std::vector<CopyEntry> tab((size_t)nseg * (per + S));
+    std::vector<CopyEntry> tab((size_t)nseg * (per + S) + per);
     for (int i = 0; i < S; ++i) {
       biot_handle *h = b->shots[s0 + i].h;
       char *live[NP] = {(char *)h->d_fields, (char *)h->d_carry[0], (char *)h->d_carry[1], (char *)h->d_carry[2],
@@ -675,6 +682,10 @@ int gradient_group(biot_batch *b, int s0, int s1, int nt, int every, const float
               CopyEntry{live[p], ckpt + (p < 4 ? h->state_off(p) : h->state_lo_off()), bytes[p]};
         tab[(size_t)nseg * per + (size_t)k * S + i] = CopyEntry{ckpt, h->d_slots, h->state_bytes()};
       }
+      const char *end = (const char *)h->d_slots + (size_t)(nt - (nseg - 1) * every) * h->state_bytes();
+      for (int p = 0; p < NP; ++p)
+        tab[(size_t)nseg * (per + S) + NP * i + p] =
+            CopyEntry{end + (p < 4 ? h->state_off(p) : h->state_lo_off()), live[p], bytes[p]};
     }
     if (!b->d_copy) BHIP(b, hipMalloc((void **)&b->d_copy, tab.size() * sizeof(CopyEntry)));
     BHIP(b, hipMemcpy(b->d_copy, tab.data(), tab.size() * sizeof(CopyEntry), hipMemcpyHostToDevice));
@@ -688,10 +699,37 @@ int gradient_group(biot_batch *b, int s0, int s1, int nt, int every, const float
     if (r) return hfail(b, b->shots[i].h, r, "reset");
   }
 
-  // ---- forward with checkpoints
+  // the steps of a segment from state to state, the first one the checkpoint's; a shot's source that
+  // no stress launch can add has every shot's added by launches of their own
+  auto segment = [&](int k, int64_t record) -> int {
+    const int n0 = k * every, K = std::min(every, nt - n0);
+    BHIP(b, load_ckpt(k));
+    BHIP(b, launch_set_counter(b->d_it, n0, n0 + K, b->stream));
+    for (int q = 0; q < K; ++q) {
+      if (q == 0 || !b->fused) BHIP(b, launch_source_batch(prec, b->d_src_s, S, b->d_it, q, q, b->stream));
+      BatchArgs ba = batch_args(b);
+      ba.shots = b->d_step_s;
+      ba.src = b->fused ? b->d_src_s : nullptr;
+      ba.rec = b->d_rec_s;
+      ba.off = ba.q = q;
+      BHIP(b, launch_step_batch(prec, order, true, ba, b->shape, b->blocks, record, b->stream));
+      BHIP(b, launch_step_batch(prec, order, false, ba, b->shape, b->blocks, record, b->stream));
+    }
+    return BIOT_OK;
+  };
+  // ---- forward with checkpoints; the last segment through the segment states, where the sweep finds
+  // them (all shots' receivers have to ride on the half steps for that)
+  const bool hold = b->fused;
   for (int k = 0; k < nseg; ++k) {
     BHIP(b, save_ckpt(k));
-    if ((rc = run_steps(b, k * every, std::min(every, nt - k * every), 0, true))) return rc;
+    if (hold && k == nseg - 1) {
+      if ((rc = segment(k, b->max_nrec))) return rc;
+      BHIP(b, launch_copy_batch(b->d_copy + (size_t)nseg * (per + S), per, b->stream));
+      rc = end_steps(b, true, nt - k * every - 1);
+    } else {
+      rc = run_steps(b, k * every, std::min(every, nt - k * every), 0, true);
+    }
+    if (rc) return rc;
   }
   // the window parameters and the observed traces go up while the forward sweep runs
   if (!b->side) BHIP(b, hipStreamCreate(&b->side));
@@ -719,19 +757,8 @@ int gradient_group(biot_batch *b, int s0, int s1, int nt, int every, const float
   const AdjBatch ab{b->d_adj, b->d_blocks, S, b->adj_blocks, b->d_inj};
   for (int k = nseg - 1; k >= 0; --k) {
     const int n0 = k * every, K = std::min(every, nt - n0);
-    BHIP(b, load_ckpt(k));
-    // the segment's steps again, from state to state; a shot's source that no stress launch can
-    // add has every shot's added by launches of their own
-    BHIP(b, launch_set_counter(b->d_it, n0, n0 + K, b->stream));
-    for (int q = 0; q < K; ++q) {
-      if (q == 0 || !b->fused) BHIP(b, launch_source_batch(prec, b->d_src_s, S, b->d_it, q, q, b->stream));
-      BatchArgs ba = batch_args(b);
-      ba.shots = b->d_step_s;
-      ba.src = b->fused ? b->d_src_s : nullptr;
-      ba.off = ba.q = q;
-      BHIP(b, launch_step_batch(prec, order, true, ba, b->shape, b->blocks, 0, b->stream));
-      BHIP(b, launch_step_batch(prec, order, false, ba, b->shape, b->blocks, 0, b->stream));
-    }
+    if (!(hold && k == nseg - 1))
+      if ((rc = segment(k, 0))) return rc;
     for (int it = n0 + K - 1; it >= n0; --it) BHIP(b, launch_adjoint_step_batch(prec, order, ab, it - n0, it, b->stream));
     BHIP(b, launch_adjoint_flush_batch(prec, order, ab, b->stream));
   }
@@ -785,6 +812,7 @@ void free_group(biot_batch *b, int s0, int s1)
   dfree(b->d_copy);
   dfree(b->d_step_s);
   dfree(b->d_src_s);
+  dfree(b->d_rec_s);
 }
 
 }  // namespace

@@ -1117,17 +1117,18 @@ __device__ __forceinline__ void batch_tile(const BatchArgs &b, int t)
 // other block of the group touches them after its own last claim).  Two kernels, because one loop
 // for both kept the queue's state in scalar registers over the plane loop (6-35 of them spilled
 // at order 4; without the queue 0-5, and FP16's velocity kernel fits 5 waves a SIMD, not 4).
-// OOP (one block per tile, recording nothing): state b.q of each shot's run of states to the next.
+// OOP (one block per tile): state b.q of each shot's run of states to the next.
 template <class P, int ORDER, bool VEL, bool QUEUE, bool OOP>
 __global__ void __launch_bounds__(256) k_step_batch(const BatchArgs b)
 {
-  if (!OOP && (int)blockIdx.x >= b.tile_blocks) {
+  if ((int)blockIdx.x >= b.tile_blocks) {
     // velocity launch: the stresses and p of the step before; stress launch: the step's velocities
     const int rb = blockIdx.x - b.tile_blocks, s = rb / b.rec_blocks;
     const CRecordArgs &ra = ((CRecordArgs *)b.rec)[s];
     const int it = ((CInt *)b.it)[0] + b.off - (VEL ? 1 : 0);
     if (!ra.traces || it < ((CInt *)b.it)[2] || it >= ra.nt_max) return;
-    record_block<P>(ra, rb - s * b.rec_blocks, VEL ? ra.nvel : 0, VEL ? ra.ncomp : ra.nvel, it, 0);
+    const uint64_t off = OOP ? (uint64_t)(VEL ? b.q : b.q + 1) * ((CStepArgs *)b.shots)[s].sb : 0;
+    record_block<P>(ra, rb - s * b.rec_blocks, VEL ? ra.nvel : 0, VEL ? ra.ncomp : ra.nvel, it, off);
     return;
   }
   const int x = blockIdx.x & 7;

@@ -53,11 +53,13 @@ def test_batch_buffers_serve_the_next_gradient(precision):
         if m != model:
             b.set_model(params(m))
             model = m
-        if i == 1:
-            b.forward(14)
         if i == 5:
             b.release()
+        b.forward(nt, graph_steps=0)
+        plain = [b.traces(k) for k in range(len(SHOTS))]
         J, g = b.gradient(nt, data(obs), every=every)
+        for k, t in enumerate(plain):
+            assert np.any(t) and np.array_equal(b.traces(k), t), (i, k)
         fresh = new_batch(params(m), precision)
         J0, g0 = fresh.gradient(nt, data(obs), every=every)
         fresh.close()
