@@ -50,6 +50,7 @@ struct biot_batch {
   int *d_it = nullptr;
   int *d_queue = nullptr;          // 16 ints, the persistent grid's work-queue counters
   int total_tiles = 0;
+  int64_t cells = 0, state = 0;    // of the shots the tables cover: cells, bytes of a state
   int nactive = 0;                 // shots the current tables cover
   int64_t max_nrec = 0;
   bool fused = false;              // every shot's source and receivers can ride on the half steps
@@ -336,7 +337,7 @@ int build_tables(biot_batch *b, int s0 = 0, int s1 = -1)
   std::vector<int> tiles(S + 1, 0);
   std::vector<SourceArgs> src(S);
   std::vector<RecordArgs> rec(S);
-  b->max_nrec = 0;
+  b->max_nrec = b->cells = b->state = 0;
   b->fused = true;
   const int h2 = b->cfg.order / 2;
   for (int i = 0; i < S; ++i) {
@@ -345,6 +346,8 @@ int build_tables(biot_batch *b, int s0 = 0, int s1 = -1)
     h->fill_args(a);
     set_tiles(a, b->shape, h2);
     tiles[i + 1] = tiles[i] + a.ntiles;
+    b->cells += h->n;
+    b->state += (int64_t)h->state_bytes();
     h->source_args(src[i]);
     h->record_args(rec[i]);
     b->max_nrec = std::max(b->max_nrec, h->nrec);
@@ -376,6 +379,8 @@ BatchArgs batch_args(const biot_batch *b)
   a.tile_start = b->d_tiles;
   a.nshots = b->nactive;
   a.total_tiles = b->total_tiles;
+  a.cells = b->cells;
+  a.state = b->state;
   a.queue = q;
   a.src = b->fused ? b->d_src : nullptr;
   a.rec = b->d_rec;

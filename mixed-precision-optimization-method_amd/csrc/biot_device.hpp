@@ -281,6 +281,7 @@ struct BatchArgs {
   const RecordArgs *rec;
   const int *it;
   int off, tile_blocks, rec_blocks;
+  int64_t cells, state;     // of all the shots' windows: cells, bytes of a state
   int q;                    // >= 0: out of place, as launch_velocity's; one block per tile, no recording
 };
 // blocks: the persistent grid size (a multiple of 8); max_nrec: the most receivers a shot has

@@ -850,12 +850,12 @@ void biot_handle::drop_records()
 
 // Coefficients built from a medium or given by the caller; an inversion's (biot_set_params) differ
 // from cell to cell and are not looked through.  FP32 and FP64 kernels wait on memory whatever the
-// size, and gain at any (us a step, streamed arrays / records: 64^3 FP32 22.5 / 19.5, 160x144x129 152 /
-// 127, 256^3 851 / 689; FP64 64^3 42 / 33, 224^3 1254 / 1111).  The 16-bit kernels gain while the rest
-// of a step's arrays then about fit the 256 MB memory-side cache (160x144x129: FP16 92 / 79, FP16T 122 /
-// 87, FP16C 147 / 115; 192x192x160: FP16 161 / 142); past it they are bound by what they issue, and the
-// dependent load costs more than the bytes it saves (192x192x160: FP16T 212 / 221, FP16C 270 / 278;
-// 224^3: FP16 295 / 296, FP16C 499 / 514).  Without room for it the arrays are streamed as ever.
+// size, and gain at any (us a step, streamed arrays / records: 64^3 FP32 18.5 / 17, 160x144x129 145 /
+// 108, 256^3 851 / 689; FP64 64^3 36.5 / 32, 224^3 1214 / 1111).  The 16-bit kernels gain while the rest
+// of a step's arrays then about fit the 256 MB memory-side cache (160x144x129: FP16 77 / 69, FP16T 121 /
+// 87, FP16C 146 / 114; 192x192x160: FP16 160 / 117); past it they are bound by what they issue, and the
+// dependent load costs what the bytes save (192x192x160: FP16T 210 / 212, FP16C 266 / 268; 224^3: FP16
+// 295 / 296, FP16C 499 / 514).  Without room for it the arrays are streamed as ever.
 int biot_handle::find_records()
 {
   drop_records();

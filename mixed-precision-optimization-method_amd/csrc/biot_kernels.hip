@@ -27,9 +27,9 @@ namespace {
 using u32 = uint32_t;
 
 // cmask: the fields that carry a residual (packed: in FP16M's packed record); nt_v / nt_t:
-// the velocity / stress kernel's own-value loads and field stores are nontemporal (same-box
-// A/B: FP32 velocity kernel -3.5 % time, FP16 velocity kernel -1 % step time; the residual
-// policies 2-3 % slower with them, FP16's stress kernel neutral); medium: the coefficients
+// the velocity / stress kernel's own-value loads and field stores are nontemporal where the
+// state is past the caches (nt_level; the residual policies are 1-5 % slower with them at any
+// size, FP16's stress kernel neutral); medium: the coefficients
 // are formed from the stored moduli (FP16M) instead of read from the packed arrays; outer16:
 // the residual-carrying fields are read at the 4th-order outer taps as binary16
 struct P32 {
@@ -90,7 +90,7 @@ struct P64 {
   using A = double;
   static constexpr bool comp = false, scaled = false;
   static constexpr uint32_t cmask = 0u;
-  static constexpr bool nt_v = false, nt_t = false;
+  static constexpr bool nt_v = true, nt_t = true;
   static constexpr bool packed = false, medium = false;
   static constexpr bool outer16 = false;
 };
@@ -355,14 +355,14 @@ __device__ __forceinline__ typename P::A dbw(const V &v, u32 c, u32 s, typename 
 
 // The N coefficients of cell c from a packed block (biot_packed.hpp layout; nontemporal:
 // read once per half step), each times its array's scale for 16-bit storage.
-template <class P, int N, class AT>
+template <class P, int N, bool NT, class AT>
 __device__ __forceinline__ void coef_block(const AT &a, const void *base, u32 c, int k0,
                                            typename P::A (&out)[N])
 {
   using S = typename P::S;
   using A = typename P::A;
   uint32_t d[packed::block_dwords<S, N>()];
-  packed::load<S, N, true>(base, (uint64_t)a.nx * a.ny * a.nz, c, d);
+  packed::load<S, N, NT>(base, (uint64_t)a.nx * a.ny * a.nz, c, d);
 #pragma unroll
   for (int e = 0; e < N; ++e) {
     if constexpr (P::scaled) out[e] = (A)packed::value<S>(d, e) * a.ks[k0 + e];
@@ -554,10 +554,9 @@ __device__ __forceinline__ A prof(const void *p, int i)
 enum { FVX = 0, FVY, FVZ, FQX, FQY, FQZ, FTXX, FTYY, FTZZ, FTXY, FTXZ, FTYZ, FP };
 
 // one x-y tile of the update box, planes kb..ke-1 of z chunk tz
-// NT: the launch allows the policy's nontemporal accesses (the single-grid kernels; the
-// batched kernels, whose shot windows are reused from the caches, do not)
+// NT: what the launch leaves to the caches (nt_level)
 // DICT: the coefficients come from the medium's records (StepArgs::ids)
-template <class P, int ORDER, bool NT, bool OOP, bool DICT, class AT>
+template <class P, int ORDER, int NT, bool OOP, bool DICT, class AT>
 __device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int tz, uint64_t ioff, uint64_t ooff)
 {
   using A = typename P::A;
@@ -674,8 +673,8 @@ __device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int t
       s3 = dwin<ORDER>(wp);
     }
 
-    const A qx0 = LO<P, FQX, (P::nt_v && NT)>(vi, c), qy0 = LO<P, FQY, (P::nt_v && NT)>(vi, c), qz0 = LO<P, FQZ, (P::nt_v && NT)>(vi, c);
-    const A vx0 = LO<P, FVX, (P::nt_v && NT)>(vi, c), vy0 = LO<P, FVY, (P::nt_v && NT)>(vi, c), vz0 = LO<P, FVZ, (P::nt_v && NT)>(vi, c);
+    const A qx0 = LO<P, FQX, (P::nt_v && NT == 2)>(vi, c), qy0 = LO<P, FQY, (P::nt_v && NT == 2)>(vi, c), qz0 = LO<P, FQZ, (P::nt_v && NT == 2)>(vi, c);
+    const A vx0 = LO<P, FVX, (P::nt_v && NT == 2)>(vi, c), vy0 = LO<P, FVY, (P::nt_v && NT == 2)>(vi, c), vz0 = LO<P, FVZ, (P::nt_v && NT == 2)>(vi, c);
     A kv[14];  // K[0..13]: U1 xyz, U2 xyz, W1 xyz, W2 xyz, W3x, W3y
     dw2_t mn[3];
     if constexpr (P::medium) {
@@ -686,7 +685,7 @@ __device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int t
     } else if constexpr (DICT) {
       coef_record<P, 14, 16>(a, a.dv, id, 0, kv);
     } else {
-      coef_block<P, 14>(a, a.kv, c, 0, kv);
+      coef_block<P, 14, (NT > 0)>(a, a.kv, c, 0, kv);
     }
     const A w1x = kv[K_W1X], w2x = kv[K_W2X], w3x = kv[K_W3X];
     const A w1y = kv[K_W1Y], w2y = kv[K_W2Y], w3y = kv[K_W3Y];
@@ -744,16 +743,16 @@ __device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int t
     const A qx1 = w1x * qx0 - w2x * sx - w3x * s1;
     const A qy1 = w1y * qy0 - w2y * sy_ - w3y * s2;
     const A qz1 = w1z * qz0 - w2z * sz_ - w3y * s3;
-    ST<P, FQX, (P::nt_v && NT)>(vo, c, qx1);
-    ST<P, FQY, (P::nt_v && NT)>(vo, c, qy1);
-    ST<P, FQZ, (P::nt_v && NT)>(vo, c, qz1);
+    ST<P, FQX, (P::nt_v && NT == 2)>(vo, c, qx1);
+    ST<P, FQY, (P::nt_v && NT == 2)>(vo, c, qy1);
+    ST<P, FQZ, (P::nt_v && NT == 2)>(vo, c, qz1);
     // the solid update sees q as stored (rounded), as the reference re-reads it; q is
     // never a compensated field, so the stored value is the plain storage rounding
     using S = typename P::S;
     const A qx1s = (A)(S)qx1, qy1s = (A)(S)qy1, qz1s = (A)(S)qz1;
-    ST<P, FVX, (P::nt_v && NT)>(vo, c, vx0 + u1x * sx - u2x * (qx1s - qx0));
-    ST<P, FVY, (P::nt_v && NT)>(vo, c, vy0 + u1y * sy_ - u2y * (qy1s - qy0));
-    ST<P, FVZ, (P::nt_v && NT)>(vo, c, vz0 + u1z * sz_ - u2z * (qz1s - qz0));
+    ST<P, FVX, (P::nt_v && NT == 2)>(vo, c, vx0 + u1x * sx - u2x * (qx1s - qx0));
+    ST<P, FVY, (P::nt_v && NT == 2)>(vo, c, vy0 + u1y * sy_ - u2y * (qy1s - qy0));
+    ST<P, FVZ, (P::nt_v && NT == 2)>(vo, c, vz0 + u1z * sz_ - u2z * (qz1s - qz0));
 
 #pragma unroll
     for (int m = 0; m < W - 1; ++m) {
@@ -770,7 +769,7 @@ __device__ __forceinline__ void velocity_tile(const AT &a, int tx, int ty, int t
 
 // one x-y tile of the update box, planes kb..ke-1 of z chunk tz; true in the thread that updated
 // the source cell
-template <class P, int ORDER, bool NT, bool OOP, bool DICT, class AT>
+template <class P, int ORDER, int NT, bool OOP, bool DICT, class AT>
 __device__ __forceinline__ bool stress_tile(const AT &a, int tx, int ty, int tz, uint64_t ioff, uint64_t ooff)
 {
   using A = typename P::A;
@@ -852,13 +851,13 @@ __device__ __forceinline__ bool stress_tile(const AT &a, int tx, int ty, int tz,
     A uyz = dwin<ORDER>(wvy);
     A uzy = dfw<P, FVZ, ORDER>(vo, c, sy, vz_c);
 
-    const A p0 = LO<P, FP, (P::nt_t && NT)>(vi, c), txx0 = LO<P, FTXX, (P::nt_t && NT)>(vi, c), tyy0 = LO<P, FTYY, (P::nt_t && NT)>(vi, c);
-    const A tzz0 = LO<P, FTZZ, (P::nt_t && NT)>(vi, c), txy0 = LO<P, FTXY, (P::nt_t && NT)>(vi, c), tyz0 = LO<P, FTYZ, (P::nt_t && NT)>(vi, c);
-    const A txz0 = LO<P, FTXZ, (P::nt_t && NT)>(vi, c);
+    const A p0 = LO<P, FP, (P::nt_t && NT == 2)>(vi, c), txx0 = LO<P, FTXX, (P::nt_t && NT == 2)>(vi, c), tyy0 = LO<P, FTYY, (P::nt_t && NT == 2)>(vi, c);
+    const A tzz0 = LO<P, FTZZ, (P::nt_t && NT == 2)>(vi, c), txy0 = LO<P, FTXY, (P::nt_t && NT == 2)>(vi, c), tyz0 = LO<P, FTYZ, (P::nt_t && NT == 2)>(vi, c);
+    const A txz0 = LO<P, FTXZ, (P::nt_t && NT == 2)>(vi, c);
     A kt[8];  // K[14..21]: P1, P2, S1, S2, S3, Sxy, Sxz, Syz
     if constexpr (P::medium) medium_stress(a, c, sy, sz, rq, kt);
     else if constexpr (DICT) coef_record<P, 8, 8>(a, a.dt, id, K_P1, kt);
-    else coef_block<P, 8>(a, a.kt, c, K_P1, kt);
+    else coef_block<P, 8, (NT > 0)>(a, a.kt, c, K_P1, kt);
     const A s1 = kt[K_S1 - K_P1], s2 = kt[K_S2 - K_P1], s3 = kt[K_S3 - K_P1];
     const A kp1 = kt[0], kp2 = kt[K_P2 - K_P1];
     const A kxy = kt[K_SXY - K_P1], kyz = kt[K_SYZ - K_P1], kxz = kt[K_SXZ - K_P1];
@@ -933,13 +932,13 @@ __device__ __forceinline__ bool stress_tile(const AT &a, int tx, int ty, int tz,
       at<uint16_t>(vo.f(FP), c) = hb[pk_slot(FP)];
       at<u32>(vo.lo(PK_FIRST), c) = pk_record(rb);
     } else {
-      ST<P, FP, (P::nt_t && NT)>(vo, c, pn);
-      ST<P, FTXX, (P::nt_t && NT)>(vo, c, txxn);
-      ST<P, FTYY, (P::nt_t && NT)>(vo, c, tyyn);
-      ST<P, FTZZ, (P::nt_t && NT)>(vo, c, tzzn);
-      ST<P, FTXY, (P::nt_t && NT)>(vo, c, txyn);
-      ST<P, FTYZ, (P::nt_t && NT)>(vo, c, tyzn);
-      ST<P, FTXZ, (P::nt_t && NT)>(vo, c, txzn);
+      ST<P, FP, (P::nt_t && NT == 2)>(vo, c, pn);
+      ST<P, FTXX, (P::nt_t && NT == 2)>(vo, c, txxn);
+      ST<P, FTYY, (P::nt_t && NT == 2)>(vo, c, tyyn);
+      ST<P, FTZZ, (P::nt_t && NT == 2)>(vo, c, tzzn);
+      ST<P, FTXY, (P::nt_t && NT == 2)>(vo, c, txyn);
+      ST<P, FTYZ, (P::nt_t && NT == 2)>(vo, c, tyzn);
+      ST<P, FTXZ, (P::nt_t && NT == 2)>(vo, c, txzn);
     }
 
 #pragma unroll
@@ -1042,7 +1041,7 @@ __device__ __forceinline__ __attribute__((address_space(4))) const T *late_args(
 
 // OOP: the half step reads state u.q of a run of states at the arguments' pointers and writes state
 // u.q + 1
-template <class P, int ORDER, bool OOP, bool DICT>
+template <class P, int ORDER, int NT, bool OOP, bool DICT>
 __global__ void __launch_bounds__(256) k_velocity(const StepArgs a, const FuseArgs u)
 {
   const uint64_t ioff = OOP ? (uint64_t)u.q * a.sb : 0, ooff = OOP ? ioff + a.sb : 0;
@@ -1052,9 +1051,9 @@ __global__ void __launch_bounds__(256) k_velocity(const StepArgs a, const FuseAr
   }
   int tx, ty, tz;
   if (!tile_of(a, tx, ty, tz)) return;
-  velocity_tile<P, ORDER, true, OOP, DICT>(a, tx, ty, tz, ioff, ooff);
+  velocity_tile<P, ORDER, NT, OOP, DICT>(a, tx, ty, tz, ioff, ooff);
 }
-template <class P, int ORDER, bool OOP, bool DICT>
+template <class P, int ORDER, int NT, bool OOP, bool DICT>
 __global__ void __launch_bounds__(256) k_stress(const StepArgs a, const FuseArgs u)
 {
   const uint64_t ioff = OOP ? (uint64_t)u.q * a.sb : 0, ooff = OOP ? ioff + a.sb : 0;
@@ -1064,7 +1063,7 @@ __global__ void __launch_bounds__(256) k_stress(const StepArgs a, const FuseArgs
   }
   int tx, ty, tz;
   if (!tile_of(a, tx, ty, tz)) return;
-  if (!stress_tile<P, ORDER, true, OOP, DICT>(a, tx, ty, tz, ioff, ooff)) return;
+  if (!stress_tile<P, ORDER, NT, OOP, DICT>(a, tx, ty, tz, ioff, ooff)) return;
   // the arguments of what follows are read here, so that none of them is kept in scalar registers
   // over the plane loop (kept, they spilled 16 more of the FP16T kernel's)
   CStepArgs *a1 = late_args<StepArgs>();
@@ -1091,7 +1090,7 @@ __device__ __forceinline__ int shot_of(const BA &b, int t)
   return lo;
 }
 // tile t of the concatenated lists
-template <class P, int ORDER, bool VEL, bool OOP>
+template <class P, int ORDER, bool VEL, bool OOP, int NT>
 __device__ __forceinline__ void batch_tile(const BatchArgs &b, int t)
 {
   const int s = shot_of(b, t);
@@ -1100,8 +1099,8 @@ __device__ __forceinline__ void batch_tile(const BatchArgs &b, int t)
   const int tx = lt % a.gx, r = lt / a.gx, ty = r % a.gy, tz = r / a.gy;
   const uint64_t ioff = OOP ? (uint64_t)b.q * a.sb : 0, ooff = OOP ? ioff + a.sb : 0;
   if constexpr (VEL) {
-    velocity_tile<P, ORDER, false, OOP, false>(a, tx, ty, tz, ioff, ooff);
-  } else if (stress_tile<P, ORDER, false, OOP, false>(a, tx, ty, tz, ioff, ooff)) {
+    velocity_tile<P, ORDER, NT, OOP, false>(a, tx, ty, tz, ioff, ooff);
+  } else if (stress_tile<P, ORDER, NT, OOP, false>(a, tx, ty, tz, ioff, ooff)) {
     CBatchArgs &b1 = *late_args<BatchArgs>();
     const int s1 = shot_of(b1, t);
     CSourceArgs &sa = ((CSourceArgs *)b1.src)[s1];
@@ -1118,7 +1117,7 @@ __device__ __forceinline__ void batch_tile(const BatchArgs &b, int t)
 // for both kept the queue's state in scalar registers over the plane loop (6-35 of them spilled
 // at order 4; without the queue 0-5, and FP16's velocity kernel fits 5 waves a SIMD, not 4).
 // OOP (one block per tile): state b.q of each shot's run of states to the next.
-template <class P, int ORDER, bool VEL, bool QUEUE, bool OOP>
+template <class P, int ORDER, bool VEL, bool QUEUE, bool OOP, int NT>
 __global__ void __launch_bounds__(256) k_step_batch(const BatchArgs b)
 {
   if ((int)blockIdx.x >= b.tile_blocks) {
@@ -1134,7 +1133,7 @@ __global__ void __launch_bounds__(256) k_step_batch(const BatchArgs b)
   const int x = blockIdx.x & 7;
   if constexpr (!QUEUE) {
     const int t = xcd_tile(x, blockIdx.x >> 3, b.xg);
-    if (t < b.total_tiles) batch_tile<P, ORDER, VEL, OOP>(b, t);
+    if (t < b.total_tiles) batch_tile<P, ORDER, VEL, OOP, NT>(b, t);
   } else {
     // every thread of the block reaches each barrier: the claims are the block's
     __shared__ int s_next;
@@ -1147,7 +1146,7 @@ __global__ void __launch_bounds__(256) k_step_batch(const BatchArgs b)
     while (t < b.total_tiles) {
       __syncthreads();  // every thread has read s_next
       if (lead) s_next = atomicAdd(ctr, 1);
-      batch_tile<P, ORDER, VEL, OOP>(b, t);
+      batch_tile<P, ORDER, VEL, OOP, NT>(b, t);
       __syncthreads();  // the next claim is in s_next
       t = xcd_tile(x, s_next, b.xg);
     }
@@ -1294,6 +1293,44 @@ __global__ void k_rescale4(S *p, int64_t nrec, double f0, double f1, double f2, 
   }
 }
 
+// How much of a step's traffic is worth keeping in the caches between launches, against the 288 MiB
+// of the memory-side cache and the L2s: 0, everything, where the state and the streamed coefficients
+// fit together; 1, the state alone (coefficients, read once a half step, loaded nontemporal); 2, nothing
+// (the fields' own-value loads and stores nontemporal as well, for the policies that gain by it).  us a
+// step at 0 / 1 / 2, state + coefficients in MiB: 64^3 FP32 (21 + 22) 16.3 / 19.2 / 20.0, 120^3 FP32 (113
+// + 145) 82 / 86 / 90, 128^3 FP32 (135 + 176) 99.9 / 97.5 / 105.6, 160^3 FP32 (250 + 344) - / 180 / 194,
+// 176^3 FP32 (327) - / 254 / 245, 192^3 (413) - / 354 / 318; 128^3 FP64 (271) - / 205 / 220, 144^3 FP64
+// (376) - / 326 / 310; 128^3 FP16 (67 + 88) 52 / 66, 224^3 FP16 (326) - / 311 / 294; 144^3 FP16T (120 +
+// 125) 94 / 110, 157x131x173 FP16T (156 + 149) 144 / 142.
+template <class P>
+int nt_level(int64_t state, int64_t coefs)
+{
+  constexpr int64_t cache = (int64_t)288 << 20;
+  if ((P::nt_v || P::nt_t) && state > cache) return 2;
+  return !P::medium && state + coefs > cache ? 1 : 0;
+}
+template <class P>
+constexpr int64_t coef_bytes(int64_t cells)
+{
+  return P::medium ? 0 : cells * NKC * (int64_t)sizeof(typename P::S);
+}
+template <class P, int ORDER, bool VEL, int NT>
+hipError_t launch_half(const StepArgs &a, const FuseArgs &u, dim3 grid, dim3 block, hipStream_t s, int q)
+{
+  if constexpr (!P::medium) {
+    if (q < 0 && a.ids) {
+      if (VEL) hipLaunchKernelGGL((k_velocity<P, ORDER, NT, false, true>), grid, block, 0, s, a, u);
+      else hipLaunchKernelGGL((k_stress<P, ORDER, NT, false, true>), grid, block, 0, s, a, u);
+      return hipGetLastError();
+    }
+  }
+  if (VEL && q >= 0) hipLaunchKernelGGL((k_velocity<P, ORDER, NT, true, false>), grid, block, 0, s, a, u);
+  else if (VEL) hipLaunchKernelGGL((k_velocity<P, ORDER, NT, false, false>), grid, block, 0, s, a, u);
+  else if (q >= 0) hipLaunchKernelGGL((k_stress<P, ORDER, NT, true, false>), grid, block, 0, s, a, u);
+  else hipLaunchKernelGGL((k_stress<P, ORDER, NT, false, false>), grid, block, 0, s, a, u);
+  return hipGetLastError();
+}
+
 template <class P, int ORDER, bool VEL>
 hipError_t launch_step(const StepArgs &in, LaunchShape sh, hipStream_t s, const RecordArgs *rec,
                        const SourceArgs *src, int q)
@@ -1314,18 +1351,15 @@ hipError_t launch_step(const StepArgs &in, LaunchShape sh, hipStream_t s, const 
   if (u.source) u.src = *src;
   const int64_t rb = u.record ? (rec->nrec + sh.bx * sh.by - 1) / (sh.bx * sh.by) : 0;
   dim3 grid((unsigned)(u.tile_blocks + rb));
-  if constexpr (!P::medium) {
-    if (q < 0 && a.ids) {
-      if (VEL) hipLaunchKernelGGL((k_velocity<P, ORDER, false, true>), grid, block, 0, s, a, u);
-      else hipLaunchKernelGGL((k_stress<P, ORDER, false, true>), grid, block, 0, s, a, u);
-      return hipGetLastError();
-    }
+  const bool records = q < 0 && a.ids;
+  const int nt = nt_level<P>((int64_t)a.sb, records ? 0 : coef_bytes<P>((int64_t)a.nx * a.ny * a.nz));
+  if constexpr (P::nt_v || P::nt_t) {
+    if (nt == 2) return launch_half<P, ORDER, VEL, 2>(a, u, grid, block, s, q);
   }
-  if (VEL && q >= 0) hipLaunchKernelGGL((k_velocity<P, ORDER, true, false>), grid, block, 0, s, a, u);
-  else if (VEL) hipLaunchKernelGGL((k_velocity<P, ORDER, false, false>), grid, block, 0, s, a, u);
-  else if (q >= 0) hipLaunchKernelGGL((k_stress<P, ORDER, true, false>), grid, block, 0, s, a, u);
-  else hipLaunchKernelGGL((k_stress<P, ORDER, false, false>), grid, block, 0, s, a, u);
-  return hipGetLastError();
+  if constexpr (!P::medium) {
+    if (nt == 1) return launch_half<P, ORDER, VEL, 1>(a, u, grid, block, s, q);
+  }
+  return launch_half<P, ORDER, VEL, 0>(a, u, grid, block, s, q);
 }
 
 template <bool VEL, int ORDER>
@@ -1353,6 +1387,25 @@ hipError_t dispatch(int prec, int order, const StepArgs &a, LaunchShape sh, hipS
   return hipErrorInvalidValue;
 }
 
+template <class P, int ORDER, bool VEL, int NT>
+hipError_t batch_half(const BatchArgs &b, dim3 grid, dim3 block, hipStream_t s)
+{
+  if (b.q >= 0) hipLaunchKernelGGL((k_step_batch<P, ORDER, VEL, false, true, NT>), grid, block, 0, s, b);
+  else if (b.queue) hipLaunchKernelGGL((k_step_batch<P, ORDER, VEL, true, false, NT>), grid, block, 0, s, b);
+  else hipLaunchKernelGGL((k_step_batch<P, ORDER, VEL, false, false, NT>), grid, block, 0, s, b);
+  return hipGetLastError();
+}
+template <class P, int ORDER, bool VEL>
+hipError_t batch_launch(const BatchArgs &b, dim3 grid, dim3 block, hipStream_t s)
+{
+  // a batch's fields stay cacheable whatever its size: its windows follow one another
+  const int nt = nt_level<P>(b.state, coef_bytes<P>(b.cells));
+  if constexpr (!P::medium) {
+    if (nt >= 1) return batch_half<P, ORDER, VEL, 1>(b, grid, block, s);
+  }
+  return batch_half<P, ORDER, VEL, 0>(b, grid, block, s);
+}
+
 }  // namespace
 
 hipError_t launch_step_batch(int prec, int order, bool vel, const BatchArgs &in, LaunchShape sh,
@@ -1365,37 +1418,21 @@ hipError_t launch_step_batch(int prec, int order, bool vel, const BatchArgs &in,
   b.tile_blocks = b.queue ? blocks : (int)(8 * xcd_slots(b.total_tiles, b.xg));
   b.rec_blocks = (int)((max_nrec + sh.bx * sh.by - 1) / (sh.bx * sh.by));
   dim3 grid((unsigned)(b.tile_blocks + b.rec_blocks * b.nshots)), block(sh.bx, sh.by, 1);
-#define BIOT_BATCH_LAUNCH(PP, OO, VV)                                                            \
-  if (b.q >= 0) hipLaunchKernelGGL((k_step_batch<PP, OO, VV, false, true>), grid, block, 0, s, b);      \
-  else if (b.queue) hipLaunchKernelGGL((k_step_batch<PP, OO, VV, true, false>), grid, block, 0, s, b);  \
-  else hipLaunchKernelGGL((k_step_batch<PP, OO, VV, false, false>), grid, block, 0, s, b);
-#define BIOT_BATCH_CASE(PP, OO)                                                                 \
-  if (vel) { BIOT_BATCH_LAUNCH(PP, OO, true) } else { BIOT_BATCH_LAUNCH(PP, OO, false) }
   if (order != 2 && order != 4) return hipErrorInvalidValue;
+  auto go = [&](auto p) -> hipError_t {
+    using P = decltype(p);
+    if (order == 2) return vel ? batch_launch<P, 2, true>(b, grid, block, s) : batch_launch<P, 2, false>(b, grid, block, s);
+    return vel ? batch_launch<P, 4, true>(b, grid, block, s) : batch_launch<P, 4, false>(b, grid, block, s);
+  };
   switch (prec) {
-    case PREC_FP32:
-      if (order == 2) { BIOT_BATCH_CASE(P32, 2) } else { BIOT_BATCH_CASE(P32, 4) }
-      break;
-    case PREC_FP16:
-      if (order == 2) { BIOT_BATCH_CASE(P16, 2) } else { BIOT_BATCH_CASE(P16, 4) }
-      break;
-    case PREC_FP16C:
-      if (order == 2) { BIOT_BATCH_CASE(P16C, 2) } else { BIOT_BATCH_CASE(P16C, 4) }
-      break;
-    case PREC_FP16T:
-      if (order == 2) { BIOT_BATCH_CASE(P16T, 2) } else { BIOT_BATCH_CASE(P16T, 4) }
-      break;
-    case PREC_FP16M:
-      if (order == 2) { BIOT_BATCH_CASE(P16M, 2) } else { BIOT_BATCH_CASE(P16M, 4) }
-      break;
-    case PREC_FP64:
-      if (order == 2) { BIOT_BATCH_CASE(P64, 2) } else { BIOT_BATCH_CASE(P64, 4) }
-      break;
-    default: return hipErrorInvalidValue;
+    case PREC_FP32: return go(P32{});
+    case PREC_FP16: return go(P16{});
+    case PREC_FP16C: return go(P16C{});
+    case PREC_FP16T: return go(P16T{});
+    case PREC_FP16M: return go(P16M{});
+    case PREC_FP64: return go(P64{});
   }
-#undef BIOT_BATCH_CASE
-#undef BIOT_BATCH_LAUNCH
-  return hipGetLastError();
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_source_batch(int prec, const SourceArgs *tab, int nshots, const int *it, int off, int q,
