@@ -238,13 +238,13 @@ __global__ void __launch_bounds__(256) k_dict(DictArgs a)
     unsigned long long todo = __ballot(act);
     while (todo) {
       if (__builtin_amdgcn_readfirstlane(
-              __hip_atomic_load(a.state + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
+              __hip_atomic_load(a.state + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0u)
         return;
       const int lead = __ffsll(todo) - 1;
       const uint32_t h = (uint32_t)__shfl((int)hash, lead);
       for (uint32_t p = 0; (todo >> lead) & 1ull; ++p) {
         if (p == 64) {
-          if (lane == 0) __hip_atomic_store(a.state + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (lane == 0) __hip_atomic_store(a.state + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           return;
         }
         const uint32_t s = (h + p) & (DICT_SLOTS - 1);
@@ -253,8 +253,8 @@ __global__ void __launch_bounds__(256) k_dict(DictArgs a)
           r = atomicCAS(a.slots + s, DICT_EMPTY, (uint32_t)c);
           if (r == DICT_EMPTY) {
             r = (uint32_t)c;
-            if (atomicAdd(a.state, 1u) >= DICT_MAX)
-              __hip_atomic_store(a.state + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (atomicAdd(a.state, 1u) + 1u >= DICT_MAX)
+              __hip_atomic_store(a.state + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           }
         }
         r = (uint32_t)__shfl((int)r, lead);

@@ -324,7 +324,7 @@ struct DictArgs {
   uint16_t *ids;             // n
   void *dv, *dt;             // DICT_SLOTS records of 16 and 8 stored values
   uint32_t *slots;           // DICT_SLOTS: a cell with the record's values, or DICT_EMPTY
-  uint32_t *state;           // records found; 1 once there are too many (both cleared)
+  uint32_t *state;           // records found less one; 0 once there are too many (both DICT_EMPTY before)
 };
 hipError_t launch_dict(int prec, const DictArgs &a, hipStream_t s);
 hipError_t launch_pack_coef(int prec, const void *soa, void *kv, void *kt, int64_t n, hipStream_t s);

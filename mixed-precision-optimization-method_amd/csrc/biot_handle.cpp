@@ -841,11 +841,9 @@ int biot_handle::upload_from_ref(const float *d_ref)
 
 void biot_handle::drop_records()
 {
-  for (void **p : {(void **)&d_ids, &d_dict})
-    if (*p) {
-      (void)hipFree(*p);
-      *p = nullptr;
-    }
+  if (d_dict) (void)hipFree(d_dict);
+  d_dict = nullptr;
+  d_ids = nullptr;
 }
 
 // Coefficients built from a medium or given by the caller; an inversion's (biot_set_params) differ
@@ -862,12 +860,12 @@ int biot_handle::find_records()
   if (half() && n > (int64_t)1 << (prec == BIOT_FP16 ? 23 : 22)) return BIOT_OK;
   const size_t values = (size_t)DICT_SLOTS * 24 * esz;
   const size_t table = (size_t)DICT_SLOTS * sizeof(uint32_t);
-  if (hipMalloc((void **)&d_ids, (size_t)n * sizeof(uint16_t)) != hipSuccess ||
-      hipMalloc(&d_dict, values + table + 256) != hipSuccess) {
+  if (hipMalloc(&d_dict, values + table + 256 + (size_t)n * sizeof(uint16_t)) != hipSuccess) {
     (void)hipGetLastError();
-    drop_records();
+    d_dict = nullptr;
     return BIOT_OK;
   }
+  d_ids = (uint16_t *)((char *)d_dict + values + table + 256);
   DictArgs a{};
   a.coef = d_coef;
   a.n = n;
@@ -876,9 +874,8 @@ int biot_handle::find_records()
   a.dt = (char *)d_dict + (size_t)DICT_SLOTS * 16 * esz;
   a.slots = (uint32_t *)((char *)d_dict + values);
   a.state = (uint32_t *)((char *)d_dict + values + table);
-  uint32_t found[2] = {0, 0};
-  if (hipMemsetAsync(a.slots, 0xFF, table, stream) != hipSuccess ||
-      hipMemsetAsync(a.state, 0, sizeof found, stream) != hipSuccess ||
+  uint32_t found[2];
+  if (hipMemsetAsync(a.slots, 0xFF, table + sizeof found, stream) != hipSuccess ||
       launch_dict(prec, a, stream) != hipSuccess ||
       hipMemcpyAsync(found, a.state, sizeof found, hipMemcpyDeviceToHost, stream) != hipSuccess ||
       hipStreamSynchronize(stream) != hipSuccess) {
@@ -886,7 +883,7 @@ int biot_handle::find_records()
     err = "looking for the medium's distinct cells failed";
     return BIOT_ERR_HIP;
   }
-  if (found[1]) drop_records();
+  if (!found[1]) drop_records();
   return BIOT_OK;
 }
 

@@ -43,8 +43,10 @@ struct biot_handle {
   int8_t *d_lo = nullptr;  // FP16C / FP16T residuals, 13 * n (compensated fields used); FP16M residual records, 4 * n
   void *d_coef = nullptr;            // 22 * n (FP16M: the medium records, 18 bytes per cell)
   void *d_kpack = nullptr;           // the coefficients packed per cell (velocity, then stress block)
-  uint16_t *d_ids = nullptr;         // a medium of few distinct cells: their records (StepArgs), else null
-  void *d_dict = nullptr;            // those records' values, and the table they were found in
+  // a medium of few distinct cells, else null: the records' values, the table they were found in and,
+  // in the same block, the cells' records (StepArgs)
+  void *d_dict = nullptr;
+  uint16_t *d_ids = nullptr;
   void *d_carry[3] = {nullptr, nullptr, nullptr};
   float *h_slice = nullptr;          // pinned, nx * nz: the slice of biot_snapshot_xz (made on first use)
   int *d_flag = nullptr;             // first step with a non-finite receiver sample
