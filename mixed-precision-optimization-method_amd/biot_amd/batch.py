@@ -1,5 +1,5 @@
 """Batched shots over the C-ABI (biot_batch_*): many windows of one model grid advanced in
-one persistent, graph-captured launch per half step, and their summed misfit gradient."""
+one graph-captured launch per half step, and their summed misfit gradient."""
 import ctypes as C
 
 import numpy as np

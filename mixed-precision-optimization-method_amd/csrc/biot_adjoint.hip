@@ -23,9 +23,9 @@
 // which the stress half has 7 different ones and the velocity half 6, kept as full arrays; the
 // derivatives along an axis whose slab the cell lies in are four records of G, laid out as the
 // carries are.
-// The passes are bound by their bytes: 137 values a cell and step (FP32: 548 B) and 144 B a slab
+// The passes are bound by their bytes: 137 values a cell and step (FP32: 548 B) and 160 B a slab
 // membership, where four passes with twelve full arrays of G moved 175 and 96 B.  Per step, before and
-// now: 128^3 FP32 343 and 325 us (about 4.1 TB/s), 192^3 1198 and 1018 us, 128^3 FP64 721 and 665, 90^3
+// now: 128^3 FP32 343 and 320 us (about 4.1 TB/s), 192^3 1198 and 1000 us, 128^3 FP64 721 and 665, 90^3
 // FP16M 236 and 107, 128^3 FP16T 687 and 320.
 // With 16-bit storage everything runs in storage units (fields divided by their scales,
 // coefficients as the kernels apply them); the host converts dJ/dK with the per-array factor.

@@ -1,7 +1,7 @@
 // Batched shots: many windows of one model advanced together (include/biot.h, biot_batch_*).
 //
 // Every shot is a grid of its own (a biot_handle: its window of the model, its absorbing
-// boundary, source and receivers).  One persistent launch per half step walks the tiles of
+// boundary, source and receivers).  One launch per half step covers the tiles of
 // all shots (k_step_batch), the per-shot argument tables live in device memory, and the step
 // index comes from a device counter, so a run of steps is captured once into a HIP graph and
 // replayed.  The gradient runs the checkpointed forward, the FP64 misfit, the segment

@@ -282,7 +282,7 @@ struct BatchArgs {
   const int *it;
   int off, tile_blocks, rec_blocks;
   int64_t cells, state;     // of all the shots' windows: cells, bytes of a state
-  int q;                    // >= 0: out of place, as launch_velocity's; one block per tile, no recording
+  int q;                    // >= 0: out of place, as launch_velocity's; one block per tile
 };
 // blocks: the persistent grid size (a multiple of 8); max_nrec: the most receivers a shot has
 // (0: record nothing)
